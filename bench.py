@@ -362,10 +362,14 @@ def run(args):
     # the whole state (spins and int32 seeds) in one workgroup's 160 KiB of
     # LDS: one launch per call (the library's rule; proposal variants never)
     resident = (not args.no_resident and app not in VARIANTS and n * (sb + 4) <= 160 * 1024
-                and nlaunch < steps)
-    planes = (lattice == "sq/4n" and (app in ("ising", "ising/single") or q == 2)
-              and not args.no_bitplanes and not resident)
-    variant = app in VARIANTS and not planes
+                and nlaunch == 1)
+    two_state = lattice == "sq/4n" and (app in ("ising", "ising/single") or q == 2)
+    paired = two_state and 2050 <= shape[0] <= 4096 and shape[1] >= 64   # two sweeps a launch on planes
+    # lattices whose colour passes are short: boxes of the lattice in LDS,
+    # several passes a launch (the library's rule)
+    boxes = not resident and not paired and nlaunch < K * steps
+    planes = two_state and not args.no_bitplanes and not resident and not boxes
+    variant = app in VARIANTS and not planes and not boxes
     launches = None   # (two-sweep launches, per-colour launches) of a call on paired planes
     if variant:
         # one site per thread, neighbours gathered in the reference's order;
@@ -373,6 +377,12 @@ def run(args):
         kernel = "k_sweep_variant<%s, %s, %s>" % (lattice, tname, app)
         bytes_per_launch = B * n // K
         B_kernel = B
+    elif boxes:
+        # the state crosses HBM once each way per launch (halos come on top);
+        # the kernel is bound by the time of its passes in LDS
+        kernel = "k_sweep_tile<%s, %s> (boxes of the lattice in LDS)" % (lattice, tname)
+        bytes_per_launch = 2 * n * (sb + 4)
+        B_kernel = bytes_per_launch / (n * steps / nlaunch)
     elif resident:
         # all sweeps of the call in one single-workgroup launch: the state
         # crosses HBM once each way; the kernel is bound by the latency of
@@ -412,6 +422,7 @@ def run(args):
     # the default where it fits; the per-colour plane kernel and the byte
     # kernel have entries of their own
     traffic, traffic_detail = load_traffic(args.workload + (
+        "-boxes" if boxes else
         "-bytes" if lattice == "sq/4n" and not planes and not resident and q <= 2 else
         "-percolour" if planes and launches is None else ""))
     if resident:
@@ -450,6 +461,13 @@ def run(args):
         "pct_hbm_peak": round(100 * value * 1e9 * B_kernel / (HBM_PEAK_GBS * 1e9), 2),
         "spin_bytes": spin_bytes(app, q),
     }
+    if boxes:
+        out["roofline"] = {"bound": "latency", "kernel": kernel,
+                           "per_pass_us": round(dev_ms * 1e3 / (steps * K), 3),
+                           "passes_per_launch": round(steps * K / nlaunch, 2),
+                           "avg_launch_us": round(per_launch_s * 1e6, 3),
+                           "bytes_per_launch": bytes_per_launch, "traffic": traffic,
+                           "traffic_measurement": traffic_detail}
     # device-side set-up (`set site range` by jump-ahead, strict seeds by
     # tagreset) against the oracle's sequential restatement of the same
     if resident:

@@ -162,7 +162,10 @@ int spk_hip_sync(spk_hip_lattice *h);
 /* Launch configuration of the per-colour sweep kernel (results do not
    depend on it: colour/strict is decomposition independent).
    block = threads per workgroup (a power of two in 64..1024); a workgroup
-   covers a tile of sub-grid rows (x, y and z), rows in y and z. */
+   covers a tile of sub-grid rows (x, y and z), rows in y and z.  Without this
+   call, a lattice whose colour passes are short (up to a few million sites)
+   runs several of them per launch on boxes of the lattice held in LDS, where
+   that is expected to be faster; the call keeps it on the per-colour kernel. */
 int spk_hip_set_launch(spk_hip_lattice *h, int block);
 
 /* Two-state sq/4n lattices (Ising, ising/single, or Potts with Q = 2) sweep on bit planes
@@ -188,9 +191,10 @@ int spk_hip_set_bitplanes(spk_hip_lattice *h, int enable);
 /* Lattices whose spins and seeds fit one workgroup's LDS (up to about 30 k
    sites at one byte per spin on MI355X: the reference's CPU-sized cases)
    run every sweep of a spk_hip_sweeps call in one launch of a single
-   workgroup, the state read and written once.  On by default; enable = 0
-   sends them through the per-colour kernels.  Results are identical either
-   way.  No counterpart in the reference (a launch choice of this
+   workgroup, the state read and written once, except those that sweep
+   faster in boxes spread over the chip (set_launch), 128^2 sq/8n among them.
+   enable = 1 keeps every such lattice on the one workgroup; enable = 0 sends
+   none there.  Results are identical either way.  No counterpart in the reference (a launch choice of this
    implementation). */
 int spk_hip_set_resident(spk_hip_lattice *h, int enable);
 

@@ -88,14 +88,17 @@ def build_emulator():
     """Host-only emulator of the kernels' index math (tests/emul), built with
     AddressSanitizer for the CPU tests.  Test infrastructure."""
     emul = os.path.join(ROOT, "tests", "emul")
-    src = os.path.join(emul, "spk_emul.hip")
-    if not os.path.exists(src):
-        return None
-    out = os.path.join(emul, "spk_emul")
-    run([hipcc(), "-x", "hip", "--offload-host-only", "-O1", "-g", "-std=c++20", "-ffp-contract=off",
-         "-Xarch_host", "-fsanitize=address", "-I" + INCLUDE, "-I" + CSRC, "-o", out, src,
-         "-L" + LIBDIR, "-lspk_hip", "-Wl,-rpath," + LIBDIR])
-    return out
+    outs = []
+    for name in ("spk_emul", "spk_emul_tile"):
+        src = os.path.join(emul, name + ".hip")
+        if not os.path.exists(src):
+            continue
+        out = os.path.join(emul, name)
+        run([hipcc(), "-x", "hip", "--offload-host-only", "-O1", "-g", "-std=c++20", "-ffp-contract=off",
+             "-Xarch_host", "-fsanitize=address", "-I" + INCLUDE, "-I" + CSRC, "-o", out, src,
+             "-L" + LIBDIR, "-lspk_hip", "-Wl,-rpath," + LIBDIR])
+        outs.append(out)
+    return outs
 
 
 def build_abi_consumer():

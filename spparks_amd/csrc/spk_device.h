@@ -1038,10 +1038,12 @@ __host__ __device__ __forceinline__ PackWork<T, TWO, I> pack_count(const T *__re
   return w;
 }
 
+// Lanes outside [v0, v1) are decided and stored like the others but not
+// counted (sites of a box's halo); by default all are.
 template <int LAT, typename T, bool TWO, typename I>
 __host__ __device__ __forceinline__ Counts pack_decide(PackWork<T, TWO, I> &w, T *__restrict__ spin,
                                                       int32_t *__restrict__ seed, const Geom &g, const Rule &r,
-                                                      const int *thr, int c) {
+                                                      const int *thr, int c, int v0 = 0, int v1 = 4) {
   const I Mp = (I)g.Mp;
   T *const spin_c = elem<I>(spin, (I)c * Mp);
   int32_t *const seed_c = elem<I>(seed, (I)c * Mp);
@@ -1066,8 +1068,9 @@ __host__ __device__ __forceinline__ Counts pack_decide(PackWork<T, TWO, I> &w, T
     if (changed) nsp.set(v, (uint32_t)pr[v]);
     nsd.w[v] = (uint32_t)s[v];
     any |= changed;
-    out.nacc += changed;
-    out.de += changed ? ef - ei : 0;
+    const bool counted = changed && v >= v0 && v < v1;
+    out.nacc += counted;
+    out.de += counted ? ef - ei : 0;
   }
   *reinterpret_cast<Words<4> *>(elem<I>(seed_c, self)) = nsd;
   if (any) store_lanes<T, I>(spin_c, self, nsp);

@@ -18,6 +18,7 @@
 #include "spk_device.h"
 #include "spk_host.h"
 #include "spk_kernels.h"
+#include "spk_tile.h"
 
 using namespace spk;
 
@@ -260,6 +261,91 @@ __global__ __launch_bounds__(1024) void k_sweep_resident(T *__restrict__ spin, i
   for (uint32_t i = threadIdx.x; i < slots; i += blockDim.x) seed[i] = lk[i];
 }
 
+// Several colour passes in one launch (spk_tile.h): workgroup t loads box t
+// with its halo into LDS, runs the plan's passes on it with a barrier after
+// each, and writes the box it owns to the other state buffer.  The counts of
+// each sweep the passes touch go to consecutive rows at acc.
+// What bounds it: small boxes, one thread's chain per pass (LDS reads, draw,
+// compare, decide, barrier: 0.8-1 us for 32 passes of 128^2 sq/8n, VALU busy
+// 38%); large ones, the VALU (54% busy on 1500 x 1002 sq/8n, with 14% of the
+// events in the halo).  us a sweep, before and now:
+//   sq/4n Ising 256^2 10.2, 2.9; 1000^2 10.8, 4.8; 1500^2 11.5, 7.7
+//   sq/8n Potts 128^2 Q=100 9.2, 4.4 (one workgroup before)
+//   sq/8n Potts 1500 x 1002 Q=100 15.1, 9.5
+//   sc/26n Potts 32^3 Q=1000 33.6, 12.8; 64^3 Q=10^5 37.6, 15.5; 100^3 35.4, 26.3
+// One site a thread (VEC 1) against packs of 4: 16.2 against 24.1 on 64^3
+// sc/26n, 4.4 against 5.6 on 128^2 sq/8n, but 11.2 against 9.5 on 1500 x 1002,
+// where the VALU counts.
+template <int LAT, typename T, bool TWO, int VEC, int APP>
+__global__ __launch_bounds__(1024) void k_sweep_tile(const T *__restrict__ spin_in, const int32_t *__restrict__ seed_in,
+                                                     T *__restrict__ spin_out, int32_t *__restrict__ seed_out, Geom g,
+                                                     Rule r, TilePlan tp, unsigned long long *__restrict__ acc) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ int s_thr[32];
+  __shared__ int s_cnt[kTileMaxSweeps][2];
+  __shared__ TilePass s_pass[kTileMaxPass];
+  int nt = (int)blockDim.x;
+  asm("" : "+s"(nt));   // held, not read again from the dispatch in every pass
+  T *ls = reinterpret_cast<T *>(lds);
+  int32_t *lk = reinterpret_cast<int32_t *>(lds + tp.spin_bytes);
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  if (tile >= tp.cx * tp.cy * tp.cz) return;   // a padding workgroup: all its threads leave together
+  const TileBox bx = tile_box(tp, tile);
+  const uint32_t packs = (uint32_t)tp.gl.K * (uint32_t)(tp.gl.Mp / 4);
+  for (uint32_t i = threadIdx.x; i < packs; i += nt) tile_load<LAT, T>(spin_in, seed_in, g, tp, bx, i, ls, lk);
+  if (threadIdx.x < 28) s_thr[threadIdx.x] = r.thr[threadIdx.x];
+  if (threadIdx.x < 2 * kTileMaxSweeps) (&s_cnt[0][0])[threadIdx.x] = 0;
+  // the pass table to LDS: read from the kernel's arguments, each pass began
+  // with two scalar loads that missed, one after the other
+  constexpr int kPassWords = kTileMaxPass * (int)sizeof(TilePass) / 4;
+  for (int i = threadIdx.x; i < kPassWords; i += nt)
+    reinterpret_cast<uint32_t *>(s_pass)[i] = reinterpret_cast<const uint32_t *>(tp.pass)[i];
+  __syncthreads();
+  int c = tp.c0, row = 0, na = 0, de = 0;
+  for (int k = 0; k < tp.npass; k++) {
+    TilePass ps;
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(TilePass) / 4; i++)
+      reinterpret_cast<int *>(&ps)[i] = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int *>(&s_pass[k])[i]);
+    auto pass = [&]<int XD>() {
+      for (uint32_t i = threadIdx.x; i < ps.items; i += nt) {
+        Counts cnt;
+        if constexpr (VEC == 1) cnt = tile_event<LAT, T, TWO, APP>(ls, lk, g, r, s_thr, tp, bx, ps, c, i);
+        else cnt = tile_events<LAT, T, TWO, XD>(ls, lk, g, r, s_thr, tp, bx, ps, c, i);
+        na += cnt.nacc;
+        de += cnt.de;
+      }
+    };
+    // packs: the x-shift side is the colour's x parity on a Moore lattice
+    if constexpr (VEC > 1 && (LAT == SPK_HIP_SQ_8N || LAT == SPK_HIP_SC_26N)) {
+      if (c & 1) pass.template operator()<1>();
+      else pass.template operator()<0>();
+    } else {
+      pass.template operator()<-1>();
+    }
+    if (++c == tp.gl.K) c = 0;
+    if (c == 0 || k == tp.npass - 1) {   // the end of a sweep, or of the launch
+      na = wave_sum(na);
+      de = wave_sum(de);
+      if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&s_cnt[row][0], na);
+        atomicAdd(&s_cnt[row][1], de);
+      }
+      na = de = 0;
+      row++;
+    }
+    __syncthreads();   // the next pass reads this one's spins
+  }
+  const uint32_t own = tile_store_items<LAT>(tp);
+  for (uint32_t i = threadIdx.x; i < own; i += nt) tile_store<LAT, T>(spin_out, seed_out, g, tp, bx, i, ls, lk);
+  if (threadIdx.x < 2u * (unsigned)row) {
+    const int v = (&s_cnt[0][0])[threadIdx.x];
+    unsigned long long *a = acc + (size_t)(threadIdx.x >> 1) * kAccRow +
+                            (size_t)(blockIdx.x & (kAccSlots - 1)) * kSlotStride + (threadIdx.x & 1);
+    if (v) atomicAdd(a, (unsigned long long)(long long)v);
+  }
+}
+
 // One colour pass of a proposal variant (potts/neigh, potts/neighonly,
 // ising/single): one slot per thread (4 consecutive slots per pack, so a
 // wavefront's own-site accesses stay unit-stride), neighbours read in the
@@ -280,6 +366,18 @@ __global__ __launch_bounds__(1024) void k_sweep_variant(T *__restrict__ spin, in
 // ===================================================================== host
 
 constexpr int kBitSites = 32;   // default sites per thread on bit planes
+
+// Boxes of the tile kernel: extents of the owned box (lattice sites), sweeps
+// per launch, sites per thread, threads per workgroup.
+struct TileShape {
+  int w[3];
+  int sweeps;
+  int vec;
+  int block;
+};
+
+// How a sweeps call runs (route()).
+enum Route { kRouteColour, kRouteBits, kRouteTile };
 
 struct spk_hip_lattice {
   spk_hip_desc d;
@@ -310,6 +408,14 @@ struct spk_hip_lattice {
   int64_t sseed2_cap = 0;
   // lattices that fit one workgroup's LDS run every sweep in one launch
   int resident = 1;
+  bool resident_set = false;           // set_resident asked for it
+  // lattices whose colour passes are short run several per launch
+  // (spk_tile.h), from spin/seed to spin2/seed2 and back
+  TileShape tile{};                    // boxes of the tile kernel (sweeps 0: not used)
+  bool tile_known = false;             // tile is up to date with the settings
+  bool block_set = false;              // set_launch asked for the per-colour kernel
+  void *spin2 = nullptr;
+  int32_t *seed2 = nullptr;
   size_t max_lds = 0;                  // LDS bytes a workgroup may use
   int32_t *stage = nullptr;            // N int32, natural order (transfers)
   unsigned long long *acc = nullptr;   // [cap][kAccRow]: per-sweep slots
@@ -327,7 +433,7 @@ struct spk_hip_lattice {
   int chunk = 32;                      // sweeps per full graph (0: eager launches only)
   struct Piece {
     int sweeps;                        // sweeps the graph runs
-    bool bits;                         // captured on the bit planes
+    int route;                         // Route it was captured on
     hipGraphExec_t exec;
   };
   std::vector<Piece> graphs;
@@ -428,6 +534,165 @@ bool bits_eligible(const spk_hip_lattice *h) {
          (!variant_app(h->d.app) || h->d.app == SPK_HIP_ISING_SINGLE);
 }
 
+// LDS bytes of the resident kernel's copy of the state (spins, then seeds
+// at a 16-byte boundary), or 0 when the lattice does not fit one workgroup.
+size_t resident_bytes(const spk_hip_lattice *h) {
+  if (variant_app(h->d.app) || !h->resident) return 0;
+  const size_t slots = (size_t)h->g.K * h->g.Mp;
+  const size_t bytes = (slots * spin_bytes(h->stype) + 15) / 16 * 16 + slots * sizeof(int32_t);
+  return bytes <= h->max_lds ? bytes : 0;
+}
+
+// VALU instructions of a site event in the packed kernels, roughly: a part
+// per site (draws, proposal, decision) and one per neighbour.  From the
+// counters: 54 a site for two states on sq/4n, 71 for u8 on sq/8n, 131 for
+// u16 on sc/26n.
+double site_valu(const spk_hip_lattice *h) {
+  const int nn = maxneigh_of(h->g.lat);
+  if (h->rule.nspins == 2) return 40 + 3.5 * nn;
+  return h->stype == kU8 ? 45 + 3.3 * nn : h->stype == kU16 ? 66 + 2.5 * nn : 60 + 4.5 * nn;
+}
+
+// The same for the tile kernel's one-site events.
+double tile_site_valu(const spk_hip_lattice *h) {
+  const int nn = maxneigh_of(h->g.lat);
+  // the first-appearance rules compare every pair of neighbours, each
+  // compare's mask through the scalar unit (counted as their time, not only
+  // their instructions: 5.2 us a pass of sc/26n with one wavefront a SIMD)
+  if (variant_app(h->d.app) && h->d.app != SPK_HIP_ISING_SINGLE) return 75 + 8.0 * nn + 1.9 * nn * nn;
+  return h->rule.nspins == 2 ? 70 + 2.0 * nn : 75 + 5.0 * nn;
+}
+
+constexpr double kUsPerValu = 4.0 / 2400.0;   // a wavefront's instruction on its SIMD: 4 cycles at 2.4 GHz
+constexpr int kSimds = 4, kCus = 256;
+
+// Microseconds a sweep is expected to take through the kernels that pass
+// over the lattice one colour at a time (bit planes where they apply) or in
+// one workgroup.  Short passes are latency: 3 us and a thread's own chain
+// (measured 3.5 us on sc/6n at 40^3, 4.2 on sc/26n at 32^3 to 100^3, 5.1-6.2
+// on bit planes at 256^2 to 2000^2, 7.0 for potts/neigh on sc/26n at 32^3).
+double plain_sweep_us(const spk_hip_lattice *h) {
+  const double sites = (double)h->N;
+  if (resident_bytes(h)) {
+    const double waves = std::ceil((double)h->g.Mp / 4 / 64);
+    return h->g.K * (0.25 + std::max(1.0, waves / kSimds) * 4 * site_valu(h) * kUsPerValu * 1.2);
+  }
+  if (bits_eligible(h))
+    return pair_fits(h->g) ? std::max(8.0, sites / 850e3) : 2 * (4.7 + 0.38e-6 * sites);
+  if (variant_app(h->d.app)) {
+    const double us = tile_site_valu(h) * kUsPerValu, waves = (double)h->g.Mp / 64;
+    return h->g.K * std::max(3.0 + 1.6 * us, 2.6 + 0.8 * waves / (kCus * kSimds) * us);
+  }
+  const double us = 4 * site_valu(h) * kUsPerValu, waves = (double)h->g.Mp / 4 / 64;
+  return h->g.K * std::max(3.0 + 1.2 * us, 2.6 + 1.5 * waves / (kCus * kSimds) * us);
+}
+
+// a wavefront's time for one item (vec sites a thread) of a tile pass
+double tile_item_us(const spk_hip_lattice *h, int vec) {
+  return (vec == 1 ? tile_site_valu(h) : 4 * site_valu(h) + 40) * kUsPerValu;
+}
+
+// Microseconds a sweep is expected to take in boxes of w sites, S sweeps a
+// launch, vec sites a thread: the launch with its loads and stores, then each
+// pass bound by the wavefronts a SIMD has of it or by one wavefront's own time.
+double tile_sweep_us(const spk_hip_lattice *h, const int (&w)[3], int S, int vec, TileShape *shape) {
+  TilePlan tp;
+  const int size = (int)spin_bytes(h->stype);
+  if (S * h->g.K > kTileMaxPass || !tile_plan_make(h->g, w, 0, S * h->g.K, vec, size, &tp)) return 1e30;
+  const size_t lds = tile_lds(tp);
+  if (lds > h->max_lds) return 1e30;
+  uint32_t most = 0;
+  for (int k = 0; k < tp.npass; k++) most = std::max(most, tp.pass[k].items);
+  const uint32_t packs = (uint32_t)tp.gl.K * (uint32_t)(tp.gl.Mp / 4);   // loaded and stored by every thread
+  const int block = (int)std::min<uint32_t>(1024, (std::max(most, packs) + 63) / 64 * 64);
+  const int64_t tiles = (int64_t)tp.cx * tp.cy * tp.cz;
+  const int per_cu = (int)((tiles + kCus - 1) / kCus);
+  const int fit = std::max(1, std::min((int)((160 << 10) / (lds + 1024)), 16 * 64 / block));   // boxes a CU holds at once
+  const int together = std::min(per_cu, fit), rounds = (per_cu + together - 1) / together;
+  const double item_us = tile_item_us(h, vec);
+  double us = 0;
+  for (int k = 0; k < tp.npass; k++) {
+    const double waves = std::ceil(tp.pass[k].items / 64.0), turns = std::ceil(tp.pass[k].items / (double)block);
+    us += 0.3 + std::max(turns * (0.15 + 1.3 * item_us), 1.2 * together * waves / kSimds * item_us);
+  }
+  const double moved = (double)lds + (double)tp.wx * tp.wy * tp.wz * (4 + size);   // bytes a box moves
+  us += together * moved / 20e3;   // a CU's share of the memory rate, about 20 GB/s a us
+  if (shape) *shape = TileShape{{w[0], w[1], w[2]}, S, vec, block};
+  return (5.0 + rounds * us) / S;
+}
+
+// Whether boxes of w sites fit LDS for launches that start at any colour
+// (launch_tiles): a launch of fewer passes needs no more halo than S sweeps
+// that end at the same colour.
+bool tile_fits(const spk_hip_lattice *h, const int (&w)[3], int S, int vec) {
+  for (int c = 0; c < h->g.K; c++) {
+    TilePlan tp;
+    if (!tile_plan_make(h->g, w, c, S * h->g.K, vec, (int)spin_bytes(h->stype), &tp) || tile_lds(tp) > h->max_lds)
+      return false;
+  }
+  return true;
+}
+
+// The boxes for this lattice and its settings, or none (sweeps 0) where the
+// other kernels are expected to be as fast.
+void tile_choose(spk_hip_lattice *h) {
+  h->tile_known = true;
+  h->tile = TileShape{};
+  // settings that name another kernel keep it
+  if (h->block_set || (h->resident_set && resident_bytes(h))) return;
+  if (h->g.lat == SPK_HIP_SQ_4N && h->rule.nspins == 2 && h->stype == kU8 && h->bitplanes != 1) return;
+  if (h->N > (int64_t)8 << 20 || !offsets_fit_32(h->g)) return;
+  // the gain the model can be trusted with (within a fifth of the measured
+  // time from 64^2 to 2000^2 and 128^3)
+  double best = (resident_bytes(h) ? 0.75 : 0.9) * plain_sweep_us(h);
+  auto sizes = [](int n, int unit) {   // extents that cut n into near-equal boxes
+    std::vector<int> v;
+    for (int cuts : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64}) {
+      const int e = ((n + cuts - 1) / cuts + unit - 1) / unit * unit;
+      if (v.empty() || e < v.back()) v.push_back(cuts == 1 ? n : e);
+    }
+    return v;
+  };
+  const std::vector<int> vx = sizes(h->g.nx, 8), vy = sizes(h->g.ny, 2), vz = sizes(h->g.nz, 2);
+  for (int S : {1, 2, 3, 4, 6, 8}) {
+    if (S * h->g.K > kTileMaxPass) break;
+    for (int wx : vx)
+      for (int wy : vy)
+        for (int wz : vz) {
+          const int64_t own = (int64_t)wx * wy * wz;
+          const int64_t tiles = (h->N + own - 1) / own;
+          if (tiles > 1024 || tiles < 2 || own * (4 + (int)spin_bytes(h->stype)) > (int64_t)h->max_lds) continue;
+          const int w[3] = {wx, wy, wz};
+          for (int vec : {1, kVec}) {
+            if (vec > 1 && variant_app(h->d.app)) continue;
+            // no less than this whatever the halo: most shapes end here
+            const double item_us = tile_item_us(h, vec), items = (double)own / h->g.K / vec;
+            const int per_cu = (int)((tiles + kCus - 1) / kCus);
+            const double least = std::max(0.15 + 1.3 * item_us, 1.2 * per_cu * items / 64 / kSimds * item_us);
+            if ((5.0 + S * h->g.K * (0.3 + least)) / S >= best) continue;
+            TileShape t;
+            const double us = tile_sweep_us(h, w, S, vec, &t);
+            if (us < best && tile_fits(h, w, S, vec)) best = us, h->tile = t;
+          }
+        }
+  }
+}
+
+// Which kernels a sweeps call of a lattice beyond one workgroup's reach takes.
+Route route(spk_hip_lattice *h) {
+  if (!h->tile_known) tile_choose(h);
+  if (h->tile.sweeps > 0) return kRouteTile;
+  return bits_eligible(h) ? kRouteBits : kRouteColour;
+}
+
+// LDS bytes of the resident kernel where a call of n sweeps runs on it, else
+// 0.  A single sweep stays there also where more would take boxes: they need
+// two launches, so that the state ends where it began.
+size_t resident_call(spk_hip_lattice *h, int n) {
+  const size_t lds = resident_bytes(h);
+  return lds && (n == 1 || route(h) != kRouteTile) ? lds : 0;
+}
+
 // Packs the state into the planes (allocated on first use) and routes the
 // colour passes there until bits_leave.
 // (Re)allocates a shadow seed array to hold `slots` slots.
@@ -488,6 +753,35 @@ __global__ void k_zero_u64(unsigned long long *__restrict__ v, int64_t n) {
   if (t < n) v[t] = 0ull;
 }
 
+// The tile kernel's second state buffers; without room for them the
+// lattice keeps to the other kernels.
+bool ensure_tile_buffers(spk_hip_lattice *h) {
+  if (!h->spin2) {
+    const size_t sb = (size_t)h->slots * spin_bytes(h->stype), kb = (size_t)h->slots * sizeof(int32_t);
+    if (hipMalloc(&h->spin2, sb) != hipSuccess) h->spin2 = nullptr;
+    if (h->spin2 && hipMalloc(&h->seed2, kb) != hipSuccess) {
+      (void)hipFree(h->spin2);
+      h->spin2 = nullptr;
+      h->seed2 = nullptr;
+    }
+    if (!h->spin2) {
+      (void)hipGetLastError();   // not an error of the call
+      h->tile = TileShape{};
+    }
+  }
+  return h->spin2 != nullptr;
+}
+
+// Brings the state to the layout the next sweeps run on: the bit planes, or
+// the bytes.
+int enter_route(spk_hip_lattice *h, Route *out) {
+  Route rt = route(h);
+  if (rt == kRouteTile && !ensure_tile_buffers(h)) rt = route(h);
+  *out = rt;
+  if (rt == kRouteBits) return h->bits_active ? SPK_HIP_OK : bits_enter(h);
+  return bits_leave(h);
+}
+
 int ensure_pinned(spk_hip_lattice *h, int rows) {
   if (rows <= h->pinned_rows) return SPK_HIP_OK;
   int cap = std::max(rows, 2 * h->pinned_rows);
@@ -524,9 +818,66 @@ int launch_pair(spk_hip_lattice *h, int from, unsigned long long *acc) {
 }
 
 // Sweep-kernel launches that launch_sweeps makes for n sweeps.
-int64_t sweep_launches(const spk_hip_lattice *h, int n) {
+int tile_launches(const spk_hip_lattice *h, int n);
+int64_t sweep_launches(const spk_hip_lattice *h, int n, Route route) {
+  if (route == kRouteTile) return tile_launches(h, n);
   if (h->bits_active && h->pairs) return 2 * (n / 4) + (int64_t)h->g.K * (n % 4);
   return (int64_t)h->g.K * n;
+}
+
+// Launches of n sweeps through the tile kernel: an even number, so that the
+// state ends where it began; a single sweep is split between its colours.
+int tile_launches(const spk_hip_lattice *h, int n) {
+  const int m = (n + h->tile.sweeps - 1) / h->tile.sweeps;
+  return n == 1 ? 2 : (m + 1) / 2 * 2;
+}
+
+// One launch of the tile kernel: colour passes [q0, q1) of a run of sweeps,
+// from buffer `from` (0: spin/seed, 1: spin2/seed2) to the other; acc is the
+// row of sweep 0.
+int launch_tile(spk_hip_lattice *h, int from, int q0, int q1, unsigned long long *acc) {
+  TilePlan tp;
+  if (!tile_plan_make(h->g, h->tile.w, q0 % h->g.K, q1 - q0, h->tile.vec, (int)spin_bytes(h->stype), &tp))
+    return set_error(SPK_HIP_ESTATE, "no box plan for %d colour passes", q1 - q0);
+  const size_t lds = tile_lds(tp);
+  unsigned grid = (unsigned)(tp.cx * tp.cy * tp.cz);
+  grid = (grid + kNumXcd - 1) / kNumXcd * kNumXcd;   // xcd_tile needs a multiple of 8
+  const bool two = h->rule.nspins == 2;
+  with_lattice(h->g.lat, [&]<int LAT>() {
+    with_type(h->stype, [&]<typename T>() {
+      T *s0 = static_cast<T *>(h->spin), *s1 = static_cast<T *>(h->spin2);
+      auto go = [&](auto kern) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(h->tile.block), lds, h->stream, from ? s1 : s0,
+                           from ? h->seed2 : h->seed, from ? s0 : s1, from ? h->seed : h->seed2, h->g, h->rule, tp,
+                           acc + (size_t)(q0 / h->g.K) * kAccRow);
+      };
+      const int app = h->d.app;
+      if (app == SPK_HIP_POTTS_NEIGH) return go(k_sweep_tile<LAT, T, false, 1, SPK_HIP_POTTS_NEIGH>);
+      if (app == SPK_HIP_POTTS_NEIGHONLY) return go(k_sweep_tile<LAT, T, false, 1, SPK_HIP_POTTS_NEIGHONLY>);
+      const bool one = h->tile.vec == 1;
+      if constexpr (sizeof(T) == 1) {   // two states are always stored as u8
+        if (app == SPK_HIP_ISING_SINGLE) return go(k_sweep_tile<LAT, T, true, 1, SPK_HIP_ISING_SINGLE>);
+        if (two) return one ? go(k_sweep_tile<LAT, T, true, 1, SPK_HIP_POTTS>) : go(k_sweep_tile<LAT, T, true, kVec, SPK_HIP_POTTS>);
+      }
+      one ? go(k_sweep_tile<LAT, T, false, 1, SPK_HIP_POTTS>) : go(k_sweep_tile<LAT, T, false, kVec, SPK_HIP_POTTS>);
+    });
+  });
+  return check_hip(hipGetLastError(), "tile sweep launch");
+}
+
+// n sweeps through the tile kernel, split evenly over its launches: whole
+// sweeps each, or (one sweep, or one sweep a launch and an odd number of
+// them) at colours inside a sweep
+int launch_tiles(spk_hip_lattice *h, int n, unsigned long long *acc, int64_t *nlaunch) {
+  const int m = tile_launches(h, n);
+  auto cut = [&](int j) {
+    return m > n ? (int)((int64_t)n * h->g.K * j / m) : (int)((int64_t)n * j / m) * h->g.K;
+  };
+  for (int j = 0; j < m; j++, (*nlaunch)++)
+    if (const int rc = launch_tile(h, j & 1, cut(j), cut(j + 1), acc)) return rc;
+  return SPK_HIP_OK;
 }
 
 // launches of sweeps whose accumulator rows start at acc; returns launches.
@@ -552,15 +903,6 @@ int launch_fold(spk_hip_lattice *h, const unsigned long long *acc, int rows, uns
   hipLaunchKernelGGL(k_fold_rows, dim3(rows), dim3(64), 0, h->stream, acc, kAccSlots, kAccRow,
                      out);
   return check_hip(hipGetLastError(), "fold launch");
-}
-
-// LDS bytes of the resident kernel's copy of the state (spins, then seeds
-// at a 16-byte boundary), or 0 when the lattice does not fit one workgroup.
-size_t resident_bytes(const spk_hip_lattice *h) {
-  if (variant_app(h->d.app) || !h->resident) return 0;
-  const size_t slots = (size_t)h->g.K * h->g.Mp;
-  const size_t bytes = (slots * spin_bytes(h->stype) + 15) / 16 * 16 + slots * sizeof(int32_t);
-  return bytes <= h->max_lds ? bytes : 0;
 }
 
 // nsweeps sweeps through the resident kernel, in pieces of at most acc_cap
@@ -641,9 +983,9 @@ int finish_sweeps(spk_hip_lattice *h, int nsweeps, int64_t nlaunch, int64_t e0, 
 // a kernel zeroes accumulator rows [0, n) (no memset node), then the n
 // sweeps' launches, then the fold of those rows into accc[0, n).  Cached
 // per (n, layout) until a settings change drops the cache.
-int piece_graph(spk_hip_lattice *h, int n, hipGraphExec_t *out) {
+int piece_graph(spk_hip_lattice *h, int n, Route rt, hipGraphExec_t *out) {
   for (auto &p : h->graphs)
-    if (p.sweeps == n && p.bits == h->bits_active) {
+    if (p.sweeps == n && p.route == rt) {
       *out = p.exec;
       return SPK_HIP_OK;
     }
@@ -655,7 +997,7 @@ int piece_graph(spk_hip_lattice *h, int n, hipGraphExec_t *out) {
   hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->acc, words);
   int64_t nl = 0;
   rc = check_hip(hipGetLastError(), "zero launch");
-  if (!rc) rc = launch_sweeps(h, n, h->acc, &nl);
+  if (!rc) rc = rt == kRouteTile ? launch_tiles(h, n, h->acc, &nl) : launch_sweeps(h, n, h->acc, &nl);
   if (!rc) rc = launch_fold(h, h->acc, n, h->accc);
   const hipError_t e = hipStreamEndCapture(h->stream, &graph);
   if (!rc) rc = check_hip(e, "end capture");
@@ -667,7 +1009,7 @@ int piece_graph(spk_hip_lattice *h, int n, hipGraphExec_t *out) {
   rc = check_hip(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "graph instantiate");
   (void)hipGraphDestroy(graph);
   if (rc) return rc;
-  h->graphs.push_back({n, h->bits_active, exec});
+  h->graphs.push_back({n, rt, exec});
   *out = exec;
   return SPK_HIP_OK;
 }
@@ -825,12 +1167,13 @@ int spk_hip_create(const spk_hip_desc *d, spk_hip_lattice **out) {
     return rc;
   }
   {
-    // LDS a workgroup may take, less room for the resident kernel's static arrays
+    // LDS a workgroup may take, less room for the static arrays of the resident
+    // and the tile kernel
     int lds = 0, optin = 0;
     (void)hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, h->device);
     (void)hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, h->device);
     const int most = std::max(lds, optin);
-    h->max_lds = most > 1024 ? (size_t)most - 1024 : 0;
+    h->max_lds = most > 2048 ? (size_t)most - 2048 : 0;
   }
   if (hipMalloc(&h->spin, (size_t)h->slots * spin_bytes(h->stype)) != hipSuccess ||
       hipMalloc(&h->seed, (size_t)h->slots * sizeof(int32_t)) != hipSuccess ||
@@ -867,6 +1210,8 @@ void spk_hip_destroy(spk_hip_lattice *h) {
   if (h->sseed) (void)hipFree(h->sseed);
   if (h->bits2) (void)hipFree(h->bits2);
   if (h->sseed2) (void)hipFree(h->sseed2);
+  if (h->spin2) (void)hipFree(h->spin2);
+  if (h->seed2) (void)hipFree(h->seed2);
   if (h->acc) (void)hipFree(h->acc);
   if (h->accc) (void)hipFree(h->accc);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
@@ -1003,15 +1348,15 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
   }
   const size_t row = 2 * sizeof(unsigned long long);   // a folded row
   int64_t nlaunch = 0;
-  if (const size_t lds = resident_bytes(h)) {
+  if (const size_t lds = resident_call(h, nsweeps)) {
     if ((rc = bits_leave(h)) || (rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows))) ||
         (rc = ensure_pinned(h, nsweeps)) || (rc = run_resident(h, nsweeps, lds, &nlaunch)))
       return rc;
     return finish_sweeps(h, nsweeps, nlaunch, e0, naccept_total, naccept_per_sweep, energy_per_sweep);
   }
-  // two-state sq/4n: the state moves to the bit planes and stays there
-  if (bits_eligible(h) && !h->bits_active && (rc = bits_enter(h))) return rc;
-  if ((rc = ensure_pinned(h, nsweeps))) return rc;
+  // (on the bit planes the state stays there)
+  Route rt;
+  if ((rc = enter_route(h, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
   if (h->chunk > 0) {
     // graph replays (graph_pieces); each piece's rows are folded into
     // accc[0, n) and copied to the pinned rows [done, done + n) in stream order
@@ -1019,7 +1364,7 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
     if ((rc = ensure_acc(h, pieces[0]))) return rc;
     std::vector<hipGraphExec_t> execs(pieces.size());
     for (size_t k = 0; k < pieces.size(); k++)
-      if ((rc = piece_graph(h, pieces[k], &execs[k]))) return rc;
+      if ((rc = piece_graph(h, pieces[k], rt, &execs[k]))) return rc;
     if ((rc = check_hip(hipEventRecord(h->ev0, h->stream), "event"))) return rc;
     int done = 0;
     for (size_t k = 0; k < pieces.size(); k++) {
@@ -1030,14 +1375,16 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
         return rc;
       done += pieces[k];
     }
-    for (int n : pieces) nlaunch += sweep_launches(h, n);
+    for (int n : pieces) nlaunch += sweep_launches(h, n, rt);
   } else {
     // every launch from the host: rows [0, nsweeps)
     if ((rc = ensure_acc(h, nsweeps))) return rc;
     const int64_t words = (int64_t)nsweeps * kAccRow;
     if ((rc = check_hip(hipEventRecord(h->ev0, h->stream), "event"))) return rc;
     hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->acc, words);
-    if ((rc = check_hip(hipGetLastError(), "zero launch")) || (rc = launch_sweeps(h, nsweeps, h->acc, &nlaunch)) ||
+    if ((rc = check_hip(hipGetLastError(), "zero launch")) ||
+        (rc = rt == kRouteTile ? launch_tiles(h, nsweeps, h->acc, &nlaunch)
+                               : launch_sweeps(h, nsweeps, h->acc, &nlaunch)) ||
         (rc = launch_fold(h, h->acc, nsweeps, h->accc)) ||
         (rc = check_hip(hipMemcpyAsync(h->pinned, h->accc, row * nsweeps, hipMemcpyDeviceToHost, h->stream),
                         "accumulator readback")))
@@ -1072,16 +1419,16 @@ int spk_hip_sweeps_noalloc(spk_hip_lattice *h, int nsweeps, unsigned long long *
 int spk_hip_prepare(spk_hip_lattice *h, int nsweeps) {
   if (!h) return set_error(SPK_HIP_EINVAL, "null handle");
   if (nsweeps < 0) return set_error(SPK_HIP_EINVAL, "nsweeps < 0");
-  if (nsweeps == 0 || resident_bytes(h)) return SPK_HIP_OK;
+  if (nsweeps == 0 || resident_call(h, nsweeps)) return SPK_HIP_OK;
   int rc;
-  if (bits_eligible(h) && !h->bits_active && (rc = bits_enter(h))) return rc;
-  if ((rc = ensure_pinned(h, nsweeps))) return rc;
+  Route rt;
+  if ((rc = enter_route(h, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
   if (h->chunk > 0) {
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
     if ((rc = ensure_acc(h, pieces[0]))) return rc;
     for (int n : pieces) {
       hipGraphExec_t exec;
-      if ((rc = piece_graph(h, n, &exec))) return rc;
+      if ((rc = piece_graph(h, n, rt, &exec))) return rc;
     }
   } else if ((rc = ensure_acc(h, nsweeps))) {
     return rc;
@@ -1126,6 +1473,8 @@ int spk_hip_set_launch(spk_hip_lattice *h, int block) {
   if (block < 64 || block > 1024 || (block & (block - 1)))
     return set_error(SPK_HIP_EINVAL, "block must be a power of two in [64, 1024]");
   h->block = block;
+  h->block_set = true;   // the per-colour kernel, with this workgroup
+  h->tile_known = false;
   drop_graphs(h);
   return SPK_HIP_OK;
 }
@@ -1133,6 +1482,9 @@ int spk_hip_set_launch(spk_hip_lattice *h, int block) {
 int spk_hip_set_resident(spk_hip_lattice *h, int enable) {
   if (!h) return set_error(SPK_HIP_EINVAL, "null handle");
   h->resident = enable ? 1 : 0;
+  h->resident_set = enable != 0;
+  h->tile_known = false;
+  drop_graphs(h);
   return SPK_HIP_OK;
 }
 
@@ -1143,6 +1495,7 @@ int spk_hip_set_bitplanes(spk_hip_lattice *h, int enable) {
   const int rc = bits_leave(h);   // the plane layout depends on the sites per thread
   if (rc) return rc;
   h->bitplanes = enable;
+  h->tile_known = false;
   drop_graphs(h);   // captured launches name one kernel or the other
   return SPK_HIP_OK;
 }
