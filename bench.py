@@ -368,6 +368,9 @@ def run(args):
     # lattices whose colour passes are short: boxes of the lattice in LDS,
     # several passes a launch (the library's rule)
     boxes = not resident and not paired and nlaunch < K * steps
+    # large sc/26n lattices: bit planes of the spins, two colours a launch
+    sliced = lattice == "sc/26n" and app not in VARIANTS and 2 * nlaunch == K * steps
+    boxes = boxes and not sliced
     planes = two_state and not args.no_bitplanes and not resident and not boxes
     variant = app in VARIANTS and not planes and not boxes
     launches = None   # (two-sweep launches, per-colour launches) of a call on paired planes
@@ -377,6 +380,13 @@ def run(args):
         kernel = "k_sweep_variant<%s, %s, %s>" % (lattice, tname, app)
         bytes_per_launch = B * n // K
         B_kernel = B
+    elif sliced:
+        # a launch reads and writes the seeds of two colours, reads the planes
+        # of the whole lattice (held in groups of four) and writes two colours'
+        groups = -(-max(1, (q - 1).bit_length()) // 4)
+        kernel = "k_sweep_slice<%d plane groups> (bit planes, two colours per launch)" % groups
+        bytes_per_launch = int(n * (2 * 8 / K + 0.5 * groups * (1 + 2 / K)))
+        B_kernel = bytes_per_launch / (n * 2 / K)
     elif boxes:
         # the state crosses HBM once each way per launch (halos come on top);
         # the kernel is bound by the time of its passes in LDS
@@ -422,7 +432,7 @@ def run(args):
     # the default where it fits; the per-colour plane kernel and the byte
     # kernel have entries of their own
     traffic, traffic_detail = load_traffic(args.workload + (
-        "-boxes" if boxes else
+        "-boxes" if boxes else "-sliced" if sliced else
         "-bytes" if lattice == "sq/4n" and not planes and not resident and q <= 2 else
         "-percolour" if planes and launches is None else ""))
     if resident:

@@ -18,6 +18,7 @@
 #include "spk_device.h"
 #include "spk_host.h"
 #include "spk_kernels.h"
+#include "spk_slice.h"
 #include "spk_tile.h"
 
 using namespace spk;
@@ -261,6 +262,52 @@ __global__ __launch_bounds__(1024) void k_sweep_resident(T *__restrict__ spin, i
   for (uint32_t i = threadIdx.x; i < slots; i += blockDim.x) seed[i] = lk[i];
 }
 
+// The two colours of row pair m on bit planes of the spins (spk_slice.h): a
+// wavefront works on s.rw whole rows, four lanes on a word of each colour.
+// What bounds it at 256^3 (Q = 10^4, 14 planes, 4096 wavefronts, all resident
+// at once): VALU 55% busy (1400 instructions a wavefront, 88 a site against 131
+// of the packed kernel), 70 MB a launch at 4.2 TB/s, the seeds of all
+// wavefronts asked for at once at the start and written at the end.  us a
+// sweep, the packed per-colour kernel and this one:
+//   Q = 3000: 64^3 34.0, 25.1; 128^3 35.5, 25.4; 160^3 45.2, 36.4; 224^3 79.1, 55.0;
+//   256^3 96.6, 59.0; 320^3 162, 121; Q = 5 at 256^3 80.4, 41.4; Q = 10^6 137, 78.4
+constexpr int kSliceThreads = 256;
+
+template <bool FULL, int PG>
+__global__ __launch_bounds__(kSliceThreads) void k_sweep_slice(uint32_t *__restrict__ planes,
+                                                               int32_t *__restrict__ sseed, Geom g, SliceGeom s, Rule r,
+                                                               int m, unsigned long long *__restrict__ acc) {
+  __shared__ SliceLds L[kSliceThreads / 64];
+  const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t v = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * (kSliceThreads / 64) + wid;
+  Counts cnt{0, 0};
+  if (v < (uint32_t)s.waves)
+    cnt = slice_counts(slice_wave<FULL, PG>(planes, sseed, g, s, r, L[wid], m, v, threadIdx.x & 63));
+  block_accumulate(cnt.nacc, cnt.de, acc, blockIdx.x & (kAccSlots - 1));
+}
+
+template <typename T>
+__global__ void k_slice_pack(const T *__restrict__ spin, Geom g, SliceGeom s, uint32_t *__restrict__ planes) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < (int64_t)g.K * s.nw) slice_pack_word<T>(spin, g, s, (int)(q / s.nw), (uint32_t)(q % s.nw), planes);
+}
+
+template <typename T>
+__global__ void k_slice_unpack(const uint32_t *__restrict__ planes, Geom g, SliceGeom s, T *__restrict__ spin) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < (int64_t)g.K * s.nw) slice_unpack_word<T>(planes, g, s, (int)(q / s.nw), (uint32_t)(q % s.nw), spin);
+}
+
+__global__ void k_slice_seeds_in(const int32_t *__restrict__ seed, Geom g, SliceGeom s, int32_t *__restrict__ sseed) {
+  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x < g.K * s.seedc / 4) slice_seeds_in(seed, g, s, x, sseed);
+}
+
+__global__ void k_slice_seeds_out(const int32_t *__restrict__ sseed, Geom g, SliceGeom s, int32_t *__restrict__ seed) {
+  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x < g.K * s.seedc / 4) slice_seeds_out(sseed, g, s, x, seed);
+}
+
 // Several colour passes in one launch (spk_tile.h): workgroup t loads box t
 // with its halo into LDS, runs the plan's passes on it with a barrier after
 // each, and writes the box it owns to the other state buffer.  The counts of
@@ -377,7 +424,7 @@ struct TileShape {
 };
 
 // How a sweeps call runs (route()).
-enum Route { kRouteColour, kRouteBits, kRouteTile };
+enum Route { kRouteColour, kRouteBits, kRouteTile, kRouteSlice };
 
 struct spk_hip_lattice {
   spk_hip_desc d;
@@ -399,6 +446,11 @@ struct spk_hip_lattice {
   int bitplanes = 1;
   bool bits_active = false;
   bool pairs = false;                  // planes in the spt-8 layout, sweeps two per launch
+  // the same for bit-sliced lattices (spk_slice.h), which use bits and sseed
+  // for their planes and seeds
+  bool slice_active = false;
+  bool slice_ok = true;                // false once the planes did not fit the device's memory
+  SliceGeom sg{};
   BitGeom bg{};
   uint32_t *bits = nullptr;
   int32_t *sseed = nullptr;
@@ -566,6 +618,12 @@ double tile_site_valu(const spk_hip_lattice *h) {
 constexpr double kUsPerValu = 4.0 / 2400.0;   // a wavefront's instruction on its SIMD: 4 cycles at 2.4 GHz
 constexpr int kSimds = 4, kCus = 256;
 
+// Lattices that sweep on bit planes of the spins (spk_slice.h).
+bool slice_eligible(const spk_hip_lattice *h) {
+  return h->slice_ok && !variant_app(h->d.app) && !h->block_set && slice_fits(h->g, h->rule.nspins) &&
+         h->rule.half == (1 << 30);
+}
+
 // Microseconds a sweep is expected to take through the kernels that pass
 // over the lattice one colour at a time (bit planes where they apply) or in
 // one workgroup.  Short passes are latency: 3 us and a thread's own chain
@@ -579,6 +637,13 @@ double plain_sweep_us(const spk_hip_lattice *h) {
   }
   if (bits_eligible(h))
     return pair_fits(h->g) ? std::max(8.0, sites / 850e3) : 2 * (4.7 + 0.38e-6 * sites);
+  if (slice_eligible(h)) {
+    // a wavefront's own time, and what a launch adds as its wavefronts fill
+    // the SIMDs (22 to 31 us a sweep for 1 to 5 plane groups up to 128^3, 41
+    // to 78 at 256^3)
+    const SliceGeom sg = slice_geom(h->g, h->rule.nspins);
+    return h->g.K / 2 * (4.6 + 0.55 * sg.PG + sg.waves / 4096.0 * (3.4 + 1.75 * sg.PG));
+  }
   if (variant_app(h->d.app)) {
     const double us = tile_site_valu(h) * kUsPerValu, waves = (double)h->g.Mp / 64;
     return h->g.K * std::max(3.0 + 1.6 * us, 2.6 + 0.8 * waves / (kCus * kSimds) * us);
@@ -644,7 +709,7 @@ void tile_choose(spk_hip_lattice *h) {
   if (h->N > (int64_t)8 << 20 || !offsets_fit_32(h->g)) return;
   // the gain the model can be trusted with (within a fifth of the measured
   // time from 64^2 to 2000^2 and 128^3)
-  double best = (resident_bytes(h) ? 0.75 : 0.9) * plain_sweep_us(h);
+  double best = (resident_bytes(h) ? 0.75 : slice_eligible(h) ? 0.85 : 0.9) * plain_sweep_us(h);
   auto sizes = [](int n, int unit) {   // extents that cut n into near-equal boxes
     std::vector<int> v;
     for (int cuts : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64}) {
@@ -682,7 +747,8 @@ void tile_choose(spk_hip_lattice *h) {
 Route route(spk_hip_lattice *h) {
   if (!h->tile_known) tile_choose(h);
   if (h->tile.sweeps > 0) return kRouteTile;
-  return bits_eligible(h) ? kRouteBits : kRouteColour;
+  if (bits_eligible(h)) return kRouteBits;
+  return slice_eligible(h) ? kRouteSlice : kRouteColour;
 }
 
 // LDS bytes of the resident kernel where a call of n sweeps runs on it, else
@@ -737,7 +803,57 @@ int bits_enter(spk_hip_lattice *h) {
   return rc;
 }
 
+// The same for a bit-sliced lattice.
+int slice_enter(spk_hip_lattice *h) {
+  h->sg = slice_geom(h->g, h->rule.nspins);
+  const int64_t words = (int64_t)h->g.K * h->sg.nw;
+  int rc;
+  if (!h->bits && hipMalloc(&h->bits, (size_t)words * h->sg.PG * sizeof(Words<4>)) != hipSuccess) {
+    h->bits = nullptr;
+    return set_error(SPK_HIP_ENOMEM, "bit planes not available");
+  }
+  if ((rc = ensure_shadow(h, h->sseed, h->sseed_cap, h->g.K * h->sg.seedc))) return rc;
+  with_type(h->stype, [&]<typename T>() {
+    hipLaunchKernelGGL((k_slice_pack<T>), dim3(grid_for(words, 256)), dim3(256), 0, h->stream,
+                       static_cast<const T *>(h->spin), h->g, h->sg, h->bits);
+  });
+  hipLaunchKernelGGL(k_slice_seeds_in, dim3(grid_for(h->g.K * h->sg.seedc / 4, 256)), dim3(256), 0, h->stream, h->seed,
+                     h->g, h->sg, h->sseed);
+  rc = check_hip(hipGetLastError(), "bit-plane pack");
+  if (!rc) h->slice_active = true;
+  return rc;
+}
+
+int slice_leave(spk_hip_lattice *h) {
+  h->slice_active = false;
+  const int64_t words = (int64_t)h->g.K * h->sg.nw;
+  with_type(h->stype, [&]<typename T>() {
+    hipLaunchKernelGGL((k_slice_unpack<T>), dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->bits, h->g, h->sg,
+                       static_cast<T *>(h->spin));
+  });
+  hipLaunchKernelGGL(k_slice_seeds_out, dim3(grid_for(h->g.K * h->sg.seedc / 4, 256)), dim3(256), 0, h->stream,
+                     h->sseed, h->g, h->sg, h->seed);
+  return check_hip(hipGetLastError(), "bit-plane unpack");
+}
+
+// One launch of the sliced pass: colours 2m and 2m+1.
+int launch_slice(spk_hip_lattice *h, int m, unsigned long long *acc) {
+  const SliceGeom &s = h->sg;
+  const int per = kSliceThreads / 64;
+  unsigned grid = (unsigned)((s.waves + per - 1) / per);
+  grid = (grid + kNumXcd - 1) / kNumXcd * kNumXcd;   // xcd_tile needs a multiple of 8
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kSliceThreads), 0, h->stream, h->bits, h->sseed, h->g, s, h->rule, m,
+                       acc);
+  };
+  with_plane_groups(s.PG, [&]<int PG>() {
+    s.W == 32 && s.last == 32 ? go(k_sweep_slice<true, PG>) : go(k_sweep_slice<false, PG>);
+  });
+  return check_hip(hipGetLastError(), "sliced sweep launch");
+}
+
 int bits_leave(spk_hip_lattice *h) {
+  if (h->slice_active) return slice_leave(h);
   if (!h->bits_active) return SPK_HIP_OK;
   h->bits_active = false;
   const int64_t words = 2 * (int64_t)h->g.hy * h->bg.pw;
@@ -779,6 +895,14 @@ int enter_route(spk_hip_lattice *h, Route *out) {
   if (rt == kRouteTile && !ensure_tile_buffers(h)) rt = route(h);
   *out = rt;
   if (rt == kRouteBits) return h->bits_active ? SPK_HIP_OK : bits_enter(h);
+  if (rt == kRouteSlice) {
+    const int rc = h->slice_active ? SPK_HIP_OK : slice_enter(h);
+    if (rc != SPK_HIP_ENOMEM) return rc;
+    (void)hipGetLastError();   // no room for the planes: the per-colour kernels
+    h->slice_ok = false;
+    *out = kRouteColour;
+    return SPK_HIP_OK;
+  }
   return bits_leave(h);
 }
 
@@ -821,6 +945,7 @@ int launch_pair(spk_hip_lattice *h, int from, unsigned long long *acc) {
 int tile_launches(const spk_hip_lattice *h, int n);
 int64_t sweep_launches(const spk_hip_lattice *h, int n, Route route) {
   if (route == kRouteTile) return tile_launches(h, n);
+  if (route == kRouteSlice) return (int64_t)h->g.K / 2 * n;
   if (h->bits_active && h->pairs) return 2 * (n / 4) + (int64_t)h->g.K * (n % 4);
   return (int64_t)h->g.K * n;
 }
@@ -892,6 +1017,10 @@ int launch_sweeps(spk_hip_lattice *h, int n, unsigned long long *acc, int64_t *n
       if ((rc = launch_pair(h, 0, acc + (size_t)s * kAccRow)) ||
           (rc = launch_pair(h, 1, acc + (size_t)(s + 2) * kAccRow)))
         return rc;
+  if (h->slice_active)
+    for (; s < n; s++)
+      for (int m = 0; m < h->g.K / 2; m++, (*nlaunch)++)
+        if ((rc = launch_slice(h, m, acc + (size_t)s * kAccRow))) return rc;
   for (; s < n; s++)
     for (int c = 0; c < h->g.K; c++, (*nlaunch)++)
       if ((rc = launch_sweep(h, c, acc + (size_t)s * kAccRow))) return rc;
@@ -1473,6 +1602,8 @@ int spk_hip_set_launch(spk_hip_lattice *h, int block) {
   if (block < 64 || block > 1024 || (block & (block - 1)))
     return set_error(SPK_HIP_EINVAL, "block must be a power of two in [64, 1024]");
   h->block = block;
+  const int rc = bits_leave(h);
+  if (rc) return rc;
   h->block_set = true;   // the per-colour kernel, with this workgroup
   h->tile_known = false;
   drop_graphs(h);
