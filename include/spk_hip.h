@@ -175,9 +175,10 @@ int spk_hip_set_launch(spk_hip_lattice *h, int block);
    sweeps calls, and a call that needs the byte layout (upload, download,
    energy, checksum, set_range, set_value, init_seeds, set_bitplanes, the
    one-workgroup kernel) unpacks them first.  By default (enable = 1) a
-   lattice whose sub-grid rows hold 33..64 plane words (nx 2050..4096) and
-   at least 64 rows runs two whole sweeps per launch: a workgroup owns a
-   band of 16 rows, keeps its planes with 4 halo rows either side in LDS
+   lattice whose sub-grid rows hold at most 64 plane words (nx up to 4096)
+   and that has at least 64 rows runs two whole sweeps per launch where that
+   is expected to be faster: a workgroup owns a band of 4, 8, 12 or 16 rows,
+   keeps its planes with 4 halo rows either side in LDS
    and its threads' seeds in registers through the four colour passes, so
    each seed is read and written once per two sweeps; the last n % 4 sweeps
    of a call take the per-colour kernel with 8 sites per thread (the same

@@ -10,6 +10,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -17,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 INCLUDE = os.path.join(ROOT, "include")
 
-HIP_SOURCES = ["spk_common.hip", "spk_plain.hip", "spk_batch.hip", "spk_serve.hip"]
+HIP_SOURCES = ["spk_common.hip", "spk_plain.hip", "spk_pair.hip", "spk_batch.hip", "spk_serve.hip"]
 FRONT_SOURCES = ["front/spk_front.cpp", "front/spk_dump_writer.cpp"]
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-pthread", "-Wall", "-Wextra", "-ffp-contract=off"]
 
@@ -47,11 +48,10 @@ def build_hip():
     os.makedirs(LIBDIR, exist_ok=True)
     out = os.path.join(LIBDIR, "libspk_hip.so")
     tmp = out + ".tmp"
-    objs = []
-    for src in HIP_SOURCES:
-        obj = os.path.join(LIBDIR, os.path.splitext(src)[0] + ".o")
-        run([hipcc(), *HIPCC_FLAGS, "-I" + INCLUDE, "-I" + CSRC, "-c", os.path.join(CSRC, src), "-o", obj])
-        objs.append(obj)
+    objs = [os.path.join(LIBDIR, os.path.splitext(src)[0] + ".o") for src in HIP_SOURCES]
+    with ThreadPoolExecutor(4) as pool:
+        list(pool.map(lambda src, obj: run([hipcc(), *HIPCC_FLAGS, "-I" + INCLUDE, "-I" + CSRC, "-c",
+                                            os.path.join(CSRC, src), "-o", obj]), HIP_SOURCES, objs))
     run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs])
     os.replace(tmp, out)
     for o in objs:
@@ -89,7 +89,7 @@ def build_emulator():
     AddressSanitizer for the CPU tests.  Test infrastructure."""
     emul = os.path.join(ROOT, "tests", "emul")
     outs = []
-    for name in ("spk_emul", "spk_emul_tile", "spk_emul_slice"):
+    for name in ("spk_emul", "spk_emul_tile", "spk_emul_slice", "spk_emul_pair"):
         src = os.path.join(emul, name + ".hip")
         if not os.path.exists(src):
             continue

@@ -445,17 +445,18 @@ __host__ __device__ __forceinline__ Counts bits_thread(uint32_t *__restrict__ bi
 }
 
 // ------------------------------------------------- two sweeps per launch
-// A lattice whose sub-grid rows hold 33..64 plane words (sq/4n, nx 2050 ..
+// A lattice whose sub-grid rows hold up to 64 plane words (sq/4n, nx up to
 // 4096) can run two whole sweeps (colour passes 0, 1, 0, 1) in one launch,
 // reading each seed once and writing it once per two sweeps instead of per
-// sweep.  A workgroup owns a band of kPairBand rows starting at y0 and holds
-// the planes of the band and kPairHalo rows either side in LDS.  Pass p
-// (colour p & 1) updates the rows y0-3+p <= rho < y0+kPairBand+3-p: each
+// sweep.  A workgroup owns a band of BAND rows (4, 8, 12 or 16) starting at y0 and
+// holds the planes of the band and kPairHalo rows either side in LDS.  Pass p
+// (colour p & 1) updates the rows y0-3+p <= rho < y0+BAND+3-p: each
 // pass shrinks the span that is still exact by one row at each end, and the
 // band's own rows are exact after all four.  Rows are taken periodically,
-// so rho may lie outside 0..hy-1.  The workgroup's threads form kPairGroups
-// groups of kPairStage (8 sites each: the spt-8 layout); group g takes the
-// rows y0-3+c+g+kPairGroups*j (slot j) of colour c in every pass, so each
+// so rho may lie outside 0..hy-1.  The workgroup's threads form groups of STAGE
+// (64, 128 or 256: 8 sites each, the spt-8 layout, so a row of up to STAGE/4
+// words); group g takes the rows y0-3+c+g+G*j (slot j, G groups) of colour c
+// in every pass, so each
 // thread keeps the seeds of its rows in registers from their one load (two
 // slots ahead of first use) to the one store of the band's own rows after
 // the colour's last pass; outside the ising/single rule one colour-0 slot
@@ -463,29 +464,48 @@ __host__ __device__ __forceinline__ Counts bits_thread(uint32_t *__restrict__ bi
 // colour's rows and writes only its own).  Planes and seeds go from one
 // pair of buffers to another, so no workgroup reads what another writes
 // during a launch.
-constexpr int kPairBand = 16;                            // rows a workgroup owns
 constexpr int kPairHalo = 4;                             // rows of input either side
-constexpr int kPairRows = kPairBand + 2 * kPairHalo;     // plane rows in LDS
 constexpr int kPairMaxPw = 64;                           // words per row, at most
-constexpr int kPairMinPw = 33;                           // and at least
-constexpr int kPairStage = 4 * kPairMaxPw;               // threads per group (8 sites each)
-constexpr int kPairGroups = 4;
-constexpr int kPairThreads = kPairGroups * kPairStage;   // the workgroup
-constexpr int kPairSlots0 = (kPairBand + 6 + kPairGroups - 1) / kPairGroups;   // colour-0 rows per thread
-constexpr int kPairSlots1 = (kPairBand + 4 + kPairGroups - 1) / kPairGroups;   // colour-1 rows per thread
+constexpr int kPairThreads = 1024;                       // the workgroup
 constexpr int kPairMinRows = 64;                         // rows (hy) a lattice needs for pairs
 
-struct PairLds {
-  uint32_t planes[2][kPairRows][kPairMaxPw];             // colour, row - (y0 - kPairHalo), word
-  Words<4> parked[2][kPairThreads];                      // one slot of seeds per thread, through pass 1
+template <int BAND, int STAGE>
+struct PairShape {
+  static constexpr int band = BAND;                      // rows a workgroup owns
+  static constexpr int rows = BAND + 2 * kPairHalo;      // plane rows in LDS
+  static constexpr int stage = STAGE;                    // threads per group
+  static constexpr int groups = kPairThreads / STAGE;
+  static constexpr int slots0 = (BAND + 6 + groups - 1) / groups;   // colour-0 rows per thread
+  static constexpr int slots1 = (BAND + 4 + groups - 1) / groups;   // colour-1 rows per thread
+  // colour 0's last slot lies past pass 2 in every group: its seeds are not
+  // kept beyond pass 0
+  static constexpr bool last0 = -3 + groups * (slots0 - 1) >= BAND + 1;
+  static constexpr int slots2 = last0 ? slots0 - 1 : slots0;        // of pass 2
 };
 
-// sq/4n with 33..64 plane words per row, at least kPairMinRows rows, and
+// the widest shape, for lattices of 64-word rows and 4096 of them
+constexpr int kPairBand = 16;
+constexpr int kPairStage = 4 * kPairMaxPw;
+using PairWide = PairShape<kPairBand, kPairStage>;
+constexpr int kPairRows = PairWide::rows;
+constexpr int kPairGroups = PairWide::groups;
+constexpr int kPairSlots0 = PairWide::slots0;
+constexpr int kPairSlots1 = PairWide::slots1;
+
+template <int BAND>
+struct PairLdsOf {
+  static constexpr int rows = BAND + 2 * kPairHalo;
+  uint32_t planes[2][rows][kPairMaxPw];                  // colour, row - (y0 - kPairHalo), word
+  Words<4> parked[2][kPairThreads];                      // one slot of seeds per thread, through pass 1
+};
+using PairLds = PairLdsOf<kPairBand>;
+
+// sq/4n with up to 64 plane words per row, at least kPairMinRows rows, and
 // shadow seeds (2 colours x hy*4*pw threads x 8 sites, 4 bytes each) below
 // 2^31 bytes, so a seed's byte offset fits 31 bits
 __host__ __device__ inline bool pair_fits(const Geom &g) {
   const int pw = (g.hx + 31) / 32;
-  return g.lat == SPK_HIP_SQ_4N && pw >= kPairMinPw && pw <= kPairMaxPw && g.hy >= kPairMinRows &&
+  return g.lat == SPK_HIP_SQ_4N && pw <= kPairMaxPw && g.hy >= kPairMinRows &&
          (int64_t)g.hy * pw * 4 * 8 * 2 * 4 < (int64_t(1) << 31);
 }
 
@@ -495,11 +515,13 @@ __host__ __device__ __forceinline__ int pair_row(int rho, int hy) {
 }
 
 // Row of slot j of group g for colour c, and whether pass p works on it.
+template <class Shape = PairWide>
 __host__ __device__ __forceinline__ int pair_slot_row(int y0, int c, int g, int j) {
-  return y0 - 3 + c + g + kPairGroups * j;
+  return y0 - 3 + c + g + Shape::groups * j;
 }
+template <class Shape = PairWide>
 __host__ __device__ __forceinline__ bool pair_pass_row(int y0, int p, int rho) {
-  return rho >= y0 - 3 + p && rho < y0 + kPairBand + 3 - p;
+  return rho >= y0 - 3 + p && rho < y0 + Shape::band + 3 - p;
 }
 
 // Global offset of local sites 4j..4j+3 of group thread tau on physical row
@@ -530,11 +552,12 @@ __host__ __device__ __forceinline__ auto pair_seeds(S *base, const BitGeom &bg, 
   }
 }
 
-// Plane word i (0 .. 2*kPairRows*pw - 1) of the band: its global offset, and
-// its place in LDS.
+// Plane word i (0 .. 2*rows*pw - 1) of the band: its global offset, and its
+// place in LDS.
+template <class Shape = PairWide>
 __host__ __device__ __forceinline__ int64_t pair_plane_src(const Geom &g, const BitGeom &bg, int y0, int i, int &c,
                                                            int &lr, int &w) {
-  const int per = kPairRows * bg.pw;
+  const int per = Shape::rows * bg.pw;
   c = i >= per;
   const int r = i - (c ? per : 0);
   lr = r / bg.pw;
@@ -542,10 +565,11 @@ __host__ __device__ __forceinline__ int64_t pair_plane_src(const Geom &g, const 
   return ((int64_t)c * g.hy + pair_row(y0 - kPairHalo + lr, g.hy)) * bg.pw + w;
 }
 
-// Plane word i (0 .. 2*kPairBand*pw - 1) of the band's own rows out of LDS.
-__host__ __device__ __forceinline__ void pair_store_plane(const PairLds &L, uint32_t *__restrict__ bits_out,
+// Plane word i (0 .. 2*BAND*pw - 1) of the band's own rows out of LDS.
+template <int BAND>
+__host__ __device__ __forceinline__ void pair_store_plane(const PairLdsOf<BAND> &L, uint32_t *__restrict__ bits_out,
                                                           const Geom &g, const BitGeom &bg, int y0, int i) {
-  const int per = kPairBand * bg.pw;
+  const int per = BAND * bg.pw;
   const int c = i >= per;
   const int r = i - (c ? per : 0);
   const int rr = r / bg.pw, w = r - rr * bg.pw;
@@ -553,9 +577,9 @@ __host__ __device__ __forceinline__ void pair_store_plane(const PairLds &L, uint
 }
 
 // Row rho's x-neighbour side for colour c: 1 when a site's x-neighbours
-// sit at a and a+1, 0 for a-1 and a.  FULL rows (the form needs hy even):
-// rho's row has rho's parity and y0 is even, so for group grp's rows
-// (y0-3+c+grp+4j) the side is (1 + grp) & 1 in every pass.
+// sit at a and a+1, 0 for a-1 and a.  FULL takes it from the group (hy, the
+// lattice's ny, is even): rho's row has rho's parity and y0 is even, so for group grp's rows
+// (y0-3+c+grp+G*j, G even) the side is (1 + grp) & 1 in every pass.
 template <bool FULL>
 __host__ __device__ __forceinline__ int pair_side(const Geom &g, int rho, int c, int grp) {
   if constexpr (FULL) return (1 + grp) & 1;
@@ -566,8 +590,9 @@ __host__ __device__ __forceinline__ int pair_side(const Geom &g, int rho, int c,
 // grp: its word w (own, above, below, beside), the x-neighbour word, and
 // its byte of its own word (w*4 + q = tau), all from the start of plane row
 // grp, so that what remains of a row's offset (its LDS row less grp: 1 + c
-// + 4j for slot j) is the same on every lane.  FULL: the same for every row
-// of the group (pair_side), so computed once.
+// + G*j for slot j) is the same on every lane.  They are the same for every
+// row of the group (pair_side), so the kernel computes them once.  FULL: rows
+// of kPairMaxPw words.
 struct PairLane {
   uint32_t w4, wn4, b;
 };
@@ -584,21 +609,24 @@ __host__ __device__ __forceinline__ PairLane pair_lane(const Geom &g, const BitG
 }
 
 // Byte `at` of the plane rows of colour c from LDS row lr0.
-__host__ __device__ __forceinline__ uint8_t *pair_lds(PairLds &L, int c, int lr0, uint32_t at) {
+template <int BAND>
+__host__ __device__ __forceinline__ uint8_t *pair_lds(PairLdsOf<BAND> &L, int c, int lr0, uint32_t at) {
   return reinterpret_cast<uint8_t *>(&L.planes[c][lr0][0]) + at;
 }
-__host__ __device__ __forceinline__ uint32_t pair_lds_word(const PairLds &L, int c, int lr0, uint32_t at) {
+template <int BAND>
+__host__ __device__ __forceinline__ uint32_t pair_lds_word(const PairLdsOf<BAND> &L, int c, int lr0, uint32_t at) {
   return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(&L.planes[c][lr0][0]) + at);
 }
 
 // The five plane words pass p's thread reads at row rho of group grp: its
 // own colour's word, and the other colour's words above, below, beside and
-// next along (bits_events).  rho's LDS row must lie in 1..kPairRows-2.
+// next along (bits_events).  rho's LDS row must lie in 1..rows-2.
 struct PairWords {
   uint32_t own, up, down, x, xe;
 };
 
-__host__ __device__ __forceinline__ PairWords pair_words(const PairLds &L, int y0, int p, int rho, int grp,
+template <int BAND>
+__host__ __device__ __forceinline__ PairWords pair_words(const PairLdsOf<BAND> &L, int y0, int p, int rho, int grp,
                                                          const PairLane &ln) {
   const int c = p & 1, o = c ^ 1;
   const int lr0 = rho - (y0 - kPairHalo) - grp;
@@ -626,8 +654,8 @@ __host__ __device__ __forceinline__ Counts pair_counts(const PairCounts &a) {
 // the colour's last pass (p >= 2), for the band's own rows, to seed_out.
 // The changes of the band's own rows go into acc.  FULL: pw = kPairMaxPw,
 // with 32 sites in the last word as in every other, and hy even.
-template <bool SINGLE, bool FULL>
-__host__ __device__ __forceinline__ void pair_thread(PairLds &L, const Geom &g, const BitGeom &bg, const Rule &r,
+template <bool SINGLE, bool FULL, int BAND>
+__host__ __device__ __forceinline__ void pair_thread(PairLdsOf<BAND> &L, const Geom &g, const BitGeom &bg, const Rule &r,
                                                      int y0, int p, int rho, int grp, uint32_t tau, const PairLane &ln,
                                                      const PairWords &pwd, Words<4> (&sq)[2],
                                                      int32_t *__restrict__ seed_out, PairCounts &acc) {
@@ -635,8 +663,8 @@ __host__ __device__ __forceinline__ void pair_thread(PairLds &L, const Geom &g, 
   const int lr0 = rho - (y0 - kPairHalo) - grp;
   const int prow = pair_row(rho, g.hy);
   const int w = (int)(tau >> 2), q = (int)(tau & 3);
-  const int px = pair_side<FULL>(g, rho, c, grp);
-  const bool owned = rho >= y0 && rho < y0 + kPairBand && rho < g.hy;
+  const int px = pair_side<true>(g, rho, c, grp);
+  const bool owned = rho >= y0 && rho < y0 + BAND && rho < g.hy;
   const BitsEi ei = bits_ei(pwd.own, pwd.up, pwd.down, pwd.x, bits_xshift<FULL>(pwd.x, pwd.xe, w, px, bg));
   const int i0 = 8 * q;
   const uint32_t own_q = pwd.own >> i0, upw_q = ei.upw >> i0, s0_q = ei.s0 >> i0, s1_q = ei.s1 >> i0;

@@ -18,6 +18,7 @@
 #include "spk_device.h"
 #include "spk_host.h"
 #include "spk_kernels.h"
+#include "spk_pair.h"
 #include "spk_slice.h"
 #include "spk_tile.h"
 
@@ -35,129 +36,6 @@ __global__ __launch_bounds__(1024) void k_sweep_bits(uint32_t *__restrict__ bits
   Counts cnt{0, 0};
   if ((int64_t)t < bg.threads) cnt = bits_thread<SPT, SINGLE>(bits, sseed, g, bg, r, color, t);
   block_accumulate_pack(cnt.nacc, cnt.de, acc, blockIdx.x & (kAccSlots - 1));
-}
-
-// Two sweeps of a lattice that pair_fits, one band of kPairBand rows per
-// workgroup (spk_bits.h): planes and seeds from (bits_in, seed_in) to
-// (bits_out, seed_out); sweep 1's counts to the row at acc, sweep 2's to
-// the next row.  The grid is the bands rounded up to a multiple of 8.
-// Every thread issues the loads of its band's planes first, then the loads
-// of its seed slots in the order it uses them, two slots ahead of their use:
-// each is waited for just before that use while the later ones are in
-// flight.  The seed loads are unconditional (a slot outside every pass, or
-// an idle lane, loads a row that exists and is not used) so that the count
-// of loads in flight is the same on every path and those waits stay exact.  FULL: rows of kPairMaxPw
-// whole words (sub-grid rows of 2048 sites: nx = 4096) and an even number
-// of them, so every lane works and the row arithmetic is simpler
-// (pair_side, pair_thread).
-template <bool SINGLE, bool FULL>
-__global__ __launch_bounds__(kPairThreads) void k_sweep_bits_pair(const uint32_t *__restrict__ bits_in,
-                                                                 const int32_t *__restrict__ seed_in,
-                                                                 uint32_t *__restrict__ bits_out,
-                                                                 int32_t *__restrict__ seed_out, Geom g, BitGeom bg,
-                                                                 Rule r, unsigned long long *__restrict__ acc) {
-  __shared__ PairLds L;
-  const int y0 = xcd_tile(blockIdx.x, gridDim.x) * kPairBand;
-  if (y0 >= g.hy) return;   // a padding workgroup: all its threads leave together
-  // the group is the same on all lanes of a wavefront (kPairStage is a
-  // multiple of 64); saying so keeps it and the rows in scalar registers
-  const int grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kPairStage));
-  const uint32_t tau = threadIdx.x % kPairStage;
-  const bool lane_on = FULL || tau < 4u * (uint32_t)bg.pw;
-  const uint32_t ta = lane_on ? tau : 0u;
-  // the planes: at most 3 words per thread (2 * kPairRows * 64 <= 3 * 1024)
-  constexpr int kPlaneLoads = (2 * kPairRows * kPairMaxPw + kPairThreads - 1) / kPairThreads;
-  const int nplane = 2 * kPairRows * bg.pw;
-  uint32_t pv[kPlaneLoads];
-#pragma unroll
-  for (int k = 0; k < kPlaneLoads; k++) {
-    int c, lr, w;
-    pv[k] = bits_in[pair_plane_src(g, bg, y0, min((int)threadIdx.x + k * kPairThreads, nplane - 1), c, lr, w)];
-  }
-  // (a thread past the last word writes that word again, with its value:
-  // no condition, so the compiler keeps the loads where they were issued)
-#pragma unroll
-  for (int k = 0; k < kPlaneLoads; k++) {
-    int c, lr, w;
-    (void)pair_plane_src(g, bg, y0, min((int)threadIdx.x + k * kPairThreads, nplane - 1), c, lr, w);
-    L.planes[c][lr][w] = pv[k];
-  }
-  // The seeds of the thread's rows, colour 0 (passes 0, 2) and colour 1
-  // (passes 1, 3), go out a few at a time, two slots ahead of their use:
-  // colour 0's first two slots now, the others during pass 0 (below).
-  // Issuing all of them at the start had every workgroup's plane loads wait
-  // behind every other's seed loads (7 us of a 48 us launch).
-  Words<4> s0[kPairSlots0][2], s1[kPairSlots1][2];
-  auto load = [&](int c, int j, Words<4>(&dst)[2]) {
-    const int rho = min(pair_slot_row(y0, c, grp, j), y0 + kPairBand + 2 - c);   // within pass c's rows
-    const int prow = pair_row(rho, g.hy);
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-      dst[h] = *pair_seeds<FULL>(seed_in, bg, c, prow, ta, h);
-  };
-  constexpr int kAhead = 2;
-#pragma unroll
-  for (int j = 0; j < kAhead; j++) load(0, j, s0[j]);
-  __syncthreads();
-  PairCounts a1, a2;   // sweep 1 (passes 0, 1) and sweep 2
-  // full rows: the thread's LDS offsets are the same on every row; opaque,
-  // so the compiler keeps them rather than recomputing them a row at a time
-  PairLane lane_full{};
-  if constexpr (FULL) {
-    lane_full = pair_lane<true>(g, bg, 0, 0, grp, tau);
-    asm volatile("" : "+v"(lane_full.w4), "+v"(lane_full.wn4), "+v"(lane_full.b));
-  }
-  // a pass over the thread's slots; before(j) runs before slot j
-  auto pass = [&](int p, auto &seeds, int slots, auto &&before) {
-#pragma unroll
-    for (int j = 0; j < slots; j++) {
-      before(j);
-      const int rho = pair_slot_row(y0, p & 1, grp, j);
-      if (lane_on && pair_pass_row(y0, p, rho)) {
-        const PairLane ln = FULL ? lane_full : pair_lane<false>(g, bg, rho, p & 1, grp, tau);
-        const PairWords pwd = pair_words(L, y0, p, rho, grp, ln);
-        pair_thread<SINGLE, FULL>(L, g, bg, r, y0, p, rho, grp, tau, ln, pwd, seeds[j], seed_out, p < 2 ? a1 : a2);
-      }
-    }
-    __syncthreads();
-  };
-  // colour 1's first kAhead slots go out during pass 0's last slots and the
-  // rest during pass 1, two slots ahead of use, so that each pass reads
-  // about one colour's seeds rather than pass 0 reading both
-  static_assert(kPairSlots0 - kAhead >= kAhead, "colour 1's first slots go out after colour 0's");
-  auto loads_ahead0 = [&](int j) {
-    if (j + kAhead < kPairSlots0) load(0, j + kAhead, s0[j + kAhead]);
-    if (j >= kPairSlots0 - kAhead) load(1, j - (kPairSlots0 - kAhead), s1[j - (kPairSlots0 - kAhead)]);
-  };
-  auto loads_ahead1 = [&](int j) {
-    if (j + kAhead < kPairSlots1) load(1, j + kAhead, s1[j + kAhead]);
-  };
-  auto nothing = [](int) {};
-  pass(0, s0, kPairSlots0, loads_ahead0);
-  // colour 0's last slot that pass 2 uses waits in LDS through pass 1, when
-  // both colours' seeds are held (its registers go to pass 1's work), and
-  // comes back one slot before pass 2 needs it; the single-flip events need
-  // fewer registers and keep it
-  constexpr int kParked = kPairSlots0 - 2;
-  if constexpr (!SINGLE) {
-#pragma unroll
-    for (int h = 0; h < 2; h++) L.parked[h][threadIdx.x] = s0[kParked][h];
-  }
-  pass(1, s1, kPairSlots1, loads_ahead1);
-  // the last colour-0 slot's rows (y0+13+g+4 >= y0+kPairBand+1) lie past
-  // pass 2's span: its seeds are not kept beyond pass 0
-  static_assert(-3 + kPairGroups * (kPairSlots0 - 1) >= kPairBand + 1, "last colour-0 slot outside pass 2");
-  auto unpark = [&](int j) {
-    if (!SINGLE && j == kParked - 1) {
-#pragma unroll
-      for (int h = 0; h < 2; h++) s0[kParked][h] = L.parked[h][threadIdx.x];
-    }
-  };
-  pass(2, s0, kPairSlots0 - 1, unpark);
-  pass(3, s1, kPairSlots1, nothing);
-  for (int i = threadIdx.x; i < 2 * kPairBand * bg.pw; i += kPairThreads) pair_store_plane(L, bits_out, g, bg, y0, i);
-  const Counts c1 = pair_counts(a1), c2 = pair_counts(a2);
-  block_accumulate2(c1.nacc, c1.de, c2.nacc, c2.de, acc, acc + kAccRow, blockIdx.x & (kAccSlots - 1));
 }
 
 // u8 state -> planes, one thread per plane word of both colours
@@ -441,7 +319,7 @@ struct spk_hip_lattice {
   // call has packed them they hold the state (bits_active) until a call
   // that needs the byte layout unpacks them (bits_leave).
   // bitplanes: 0 planes off; 1 the default (two sweeps per launch where
-  // pair_fits, else kBitSites sites per thread); 8, 16, 32 sites per thread
+  // that pays, else kBitSites sites per thread); 8, 16, 32 sites per thread
   // of the per-colour kernel
   int bitplanes = 1;
   bool bits_active = false;
@@ -624,6 +502,17 @@ bool slice_eligible(const spk_hip_lattice *h) {
          h->rule.half == (1 << 30);
 }
 
+// Microseconds a sweep is expected to take on bit planes, one colour a launch
+// and two sweeps a launch.
+double colour_bits_us(const spk_hip_lattice *h) { return 2 * std::max(4.7 + 0.38e-6 * h->N, 2.5 + h->N / 1520e3); }
+double pair_sweep_us(const spk_hip_lattice *h) {
+  const int band = pair_band(h->g), rounds = ((h->g.hy + band - 1) / band + kCus - 1) / kCus;
+  // band rows of the four passes, wavefronts a row, their time a row
+  const double rows = 4 * band + 12, waves = pair_stage((h->g.hx + 31) / 32) / 64;
+  const double us = h->d.app == SPK_HIP_ISING_SINGLE ? 0.085 : 0.105;
+  return (5.0 + rounds * rows * waves * us) / 2;
+}
+
 // Microseconds a sweep is expected to take through the kernels that pass
 // over the lattice one colour at a time (bit planes where they apply) or in
 // one workgroup.  Short passes are latency: 3 us and a thread's own chain
@@ -636,7 +525,7 @@ double plain_sweep_us(const spk_hip_lattice *h) {
     return h->g.K * (0.25 + std::max(1.0, waves / kSimds) * 4 * site_valu(h) * kUsPerValu * 1.2);
   }
   if (bits_eligible(h))
-    return pair_fits(h->g) ? std::max(8.0, sites / 850e3) : 2 * (4.7 + 0.38e-6 * sites);
+    return h->bitplanes == 1 && pair_fits(h->g) ? std::min(pair_sweep_us(h), colour_bits_us(h)) : colour_bits_us(h);
   if (slice_eligible(h)) {
     // a wavefront's own time, and what a launch adds as its wavefronts fill
     // the SIMDs (22 to 31 us a sweep for 1 to 5 plane groups up to 128^3, 41
@@ -785,7 +674,7 @@ int ensure_planes(uint32_t *&p, const spk_hip_lattice *h) {
 }
 
 int bits_enter(spk_hip_lattice *h) {
-  h->pairs = h->bitplanes == 1 && pair_fits(h->g);
+  h->pairs = h->bitplanes == 1 && pair_fits(h->g) && pair_sweep_us(h) < colour_bits_us(h);
   h->bg = bit_geom(h->g, h->pairs ? 8 : h->bitplanes == 1 ? kBitSites : h->bitplanes);
   int rc;
   if ((rc = ensure_planes(h->bits, h)) || (rc = ensure_shadow(h, h->sseed, h->sseed_cap, 2 * h->bg.seedc)))
@@ -925,19 +814,8 @@ int ensure_pinned(spk_hip_lattice *h, int rows) {
 // Two sweeps in one launch (k_sweep_bits_pair), from the planes and seeds
 // at `from` (0: bits/sseed, 1: bits2/sseed2) to the others.
 int launch_pair(spk_hip_lattice *h, int from, unsigned long long *acc) {
-  const int bands = (h->g.hy + kPairBand - 1) / kPairBand;
-  const unsigned grid = (unsigned)((bands + kNumXcd - 1) / kNumXcd * kNumXcd);   // xcd_tile: a multiple of 8
-  const uint32_t *bi = from ? h->bits2 : h->bits;
-  const int32_t *si = from ? h->sseed2 : h->sseed;
-  uint32_t *bo = from ? h->bits : h->bits2;
-  int32_t *so = from ? h->sseed : h->sseed2;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kPairThreads), 0, h->stream, bi, si, bo, so, h->g, h->bg, h->rule, acc);
-  };
-  // 64 words, the last one whole, and an even number of rows
-  const bool full = h->bg.pw == kPairMaxPw && h->bg.r == 31 && h->g.hy % 2 == 0;
-  if (h->d.app == SPK_HIP_ISING_SINGLE) full ? go(k_sweep_bits_pair<true, true>) : go(k_sweep_bits_pair<true, false>);
-  else full ? go(k_sweep_bits_pair<false, true>) : go(k_sweep_bits_pair<false, false>);
+  launch_pair_kernel(h->stream, from ? h->bits2 : h->bits, from ? h->sseed2 : h->sseed, from ? h->bits : h->bits2,
+                     from ? h->sseed : h->sseed2, h->g, h->bg, h->rule, h->d.app == SPK_HIP_ISING_SINGLE, acc);
   return check_hip(hipGetLastError(), "two-sweep launch");
 }
 

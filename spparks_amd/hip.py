@@ -246,8 +246,8 @@ class Lattice:
         _check(self.L.spk_hip_set_resident(self.h, int(bool(enable))))
 
     def set_bitplanes(self, enable):
-        """0/False: off; 1/True: on (two sweeps per launch where the rows
-        hold 33..64 plane words); 8, 16 or 32: the per-colour kernel with
+        """0/False: off; 1/True: on (two sweeps per launch where rows of up
+        to 64 plane words make that pay); 8, 16 or 32: the per-colour kernel with
         that many sites per thread."""
         _check(self.L.spk_hip_set_bitplanes(self.h, int(enable)))
 
