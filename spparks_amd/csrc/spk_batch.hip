@@ -234,8 +234,7 @@ struct spk_hip_batch {
   StepDesc *d_steps = nullptr;
   int *d_act = nullptr, *d_pre = nullptr;
   unsigned long long *d_acc = nullptr;    // [rows][kBatchRow] slots
-  unsigned long long *d_accc = nullptr;   // [rows][2] folded (Naccept, dE)
-  int cap_reps = 0, cap_steps = 0, cap_act = 0, cap_pre = 0, cap_acc = 0, cap_accc = 0;
+  int cap_reps = 0, cap_steps = 0, cap_act = 0, cap_pre = 0, cap_acc = 0;
   std::vector<BatchRep> h_reps;
   std::vector<StepDesc> h_steps;
   std::vector<int> h_act, h_pre;
@@ -317,12 +316,8 @@ int replica_energy_async(spk_hip_batch *b, int id, Replica &R) {
                          reinterpret_cast<const T *>(b->pool + R.spin_off), R.g, row);
     });
   });
-  hipLaunchKernelGGL(k_fold_rows, dim3(1), dim3(64), 0, b->stream, row, kAccSlots, kAccRow, b->d_slot + 4 * (size_t)id);
-  int rc = check_hip(hipGetLastError(), "energy launch");
-  if (!rc)
-    rc = check_hip(hipMemcpyAsync(b->h_slot + 4 * (size_t)id, b->d_slot + 4 * (size_t)id, sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, b->stream),
-                   "energy readback");
+  hipLaunchKernelGGL(k_fold_rows, dim3(1), dim3(64), 0, b->stream, row, kAccSlots, kAccRow, b->h_slot + 4 * (size_t)id);
+  const int rc = check_hip(hipGetLastError(), "energy launch");
   if (!rc) R.energy_pending = true;
   return rc;
 }
@@ -436,8 +431,7 @@ int upload_schedule(spk_hip_batch *b, int rows, bool clear_acc) {
       (rc = grow(&b->d_steps, &b->cap_steps, std::max<int>(1, b->h_steps.size()), "step table", &moved)) ||
       (rc = grow(&b->d_act, &b->cap_act, std::max<int>(1, b->h_act.size()), "step lists", &moved)) ||
       (rc = grow(&b->d_pre, &b->cap_pre, std::max<int>(1, b->h_pre.size()), "step lists", &moved)) ||
-      (rc = grow(&b->d_acc, &b->cap_acc, std::max(1, rows) * kBatchRow, "accumulators", &moved)) ||
-      (rc = grow(&b->d_accc, &b->cap_accc, std::max(2, 2 * rows), "accumulators", &moved))) {
+      (rc = grow(&b->d_acc, &b->cap_acc, std::max(1, rows) * kBatchRow, "accumulators", &moved))) {
     if (moved) drop_graphs(b);   // an earlier table moved before a later one failed
     return rc;
   }
@@ -577,7 +571,6 @@ void spk_hip_batch_destroy(spk_hip_batch *b) {
   if (b->d_act) (void)hipFree(b->d_act);
   if (b->d_pre) (void)hipFree(b->d_pre);
   if (b->d_acc) (void)hipFree(b->d_acc);
-  if (b->d_accc) (void)hipFree(b->d_accc);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b->alloc;
   delete b;
@@ -727,11 +720,12 @@ int spk_hip_batch_download(spk_hip_batch *b, int id, int32_t *spin, int32_t *see
                          reinterpret_cast<const int32_t *>(b->pool + R.seed_off), b->stage, R.g);
     }
     if ((rc = check_hip(hipGetLastError(), "layout kernel"))) return rc;
+    // (the second kernel writes the staging array after the first copy has
+    // read it: stream order)
     if ((rc = check_hip(hipMemcpyAsync(dst, b->stage, n * 4, hipMemcpyDeviceToHost, b->stream), "download")))
       return rc;
-    if ((rc = check_hip(hipStreamSynchronize(b->stream), "download sync"))) return rc;
   }
-  return SPK_HIP_OK;
+  return check_hip(hipStreamSynchronize(b->stream), "download sync");
 }
 
 int spk_hip_batch_set_launch(spk_hip_batch *b, int block, int grid) {
@@ -753,7 +747,7 @@ namespace spk {
 
 bool batch_inflight(const spk_hip_batch *b) { return b && b->inflight; }
 
-// Folds the block's accumulator rows and queues their copy to pinned memory.
+// Folds the block's accumulator rows into pinned memory.
 static int queue_rows(spk_hip_batch *b, int rows) {
   if (rows > b->cap_h_rows) {   // only between blocks: nothing reads h_rows now
     unsigned long long *p = nullptr;
@@ -764,13 +758,8 @@ static int queue_rows(spk_hip_batch *b, int rows) {
     b->h_rows = p;
     b->cap_h_rows = cap;
   }
-  hipLaunchKernelGGL(k_fold_rows, dim3(rows), dim3(64), 0, b->stream, b->d_acc, kBatchSlots, kBatchRow, b->d_accc);
-  int rc = check_hip(hipGetLastError(), "fold launch");
-  if (!rc)
-    rc = check_hip(hipMemcpyAsync(b->h_rows, b->d_accc, 2 * (size_t)rows * sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, b->stream),
-                   "accumulator readback");
-  return rc;
+  hipLaunchKernelGGL(k_fold_rows, dim3(rows), dim3(64), 0, b->stream, b->d_acc, kBatchSlots, kBatchRow, b->h_rows);
+  return check_hip(hipGetLastError(), "fold launch");
 }
 
 // After the stream has passed the block: each replica's per-sweep Naccept

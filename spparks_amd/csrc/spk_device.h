@@ -1129,6 +1129,30 @@ __device__ __forceinline__ void block_accumulate(int x, int y, unsigned long lon
   }
 }
 
+// block_accumulate for a workgroup that is the whole launch: its totals are
+// the row (out[0], out[1]), stored and not added.
+__device__ __forceinline__ void block_store(int x, int y, unsigned long long *out) {
+  __shared__ int red[2][16];
+  x = wave_sum(x);
+  y = wave_sum(y);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 0) {
+    red[0][wid] = x;
+    red[1][wid] = y;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int sx = 0, sy = 0;
+    const int nw = blockDim.x >> 6;
+    for (int w = 0; w < nw; w++) {
+      sx += red[0][w];
+      sy += red[1][w];
+    }
+    out[0] = (unsigned long long)(long long)sx;
+    out[1] = (unsigned long long)(long long)sy;
+  }
+}
+
 // block_accumulate for small per-thread counts: 0 <= x, 64 * x < 2^16 and
 // 64 * |y| < 2^15 (one pack of 4 sites: x <= 4, |y| <= 4 * 26).  A wave's
 // two sums then fit one 32-bit word, x in the low half and y in the high

@@ -56,6 +56,21 @@ __global__ void k_to_natural(const T *__restrict__ blk, int32_t *__restrict__ na
   nat[t] = (int32_t)blk[blocked_index(g, i, j, k)];
 }
 
+// Spins and seeds (either may be null: skipped) of a whole lattice in natural
+// order, for the small ones whose state a kernel writes straight to host
+// memory.
+template <typename T>
+__global__ void k_state_natural(const T *__restrict__ spin, const int32_t *__restrict__ seed, int32_t *__restrict__ out,
+                                Geom g) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, n = (int64_t)g.M * g.K;
+  if (t >= n) return;
+  int i, j, k;
+  natural_ijk(g, t, i, j, k);
+  const int64_t p = blocked_index(g, i, j, k);
+  if (spin) out[t] = (int32_t)spin[p];
+  if (seed) out[n + t] = seed[p];
+}
+
 // Compacts accumulator rows: out[2r], out[2r+1] = the sums of row r's
 // `slots` slots (row r at acc + r*row_words, slot k at +k*kSlotStride).
 __global__ __launch_bounds__(64) void k_fold_rows(const unsigned long long *__restrict__ acc, int slots,

@@ -104,10 +104,11 @@ __global__ __launch_bounds__(1024) void k_sweep_color(T *__restrict__ spin, int3
 // (the reference's CPU-sized cases): spins and seeds are read once, all
 // colour passes run on the LDS copy with a barrier between passes, and the
 // state is written back once.  The same per-pack events as k_sweep_color,
-// on LDS addresses; sweep s's (Naccept, dE) go to slot 0 of acc row s.
+// on LDS addresses; sweep s's (Naccept, dE) go to rows[2s], rows[2s+1] (host
+// memory).
 template <int LAT, typename T, bool TWO>
 __global__ __launch_bounds__(1024) void k_sweep_resident(T *__restrict__ spin, int32_t *__restrict__ seed, Geom g,
-                                                         Rule r, int nsweeps, unsigned long long *__restrict__ acc) {
+                                                         Rule r, int nsweeps, unsigned long long *__restrict__ rows) {
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ int s_thr[32];
   const uint32_t slots = (uint32_t)g.K * (uint32_t)g.Mp;
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(1024) void k_sweep_resident(T *__restrict__ spin, i
       }
       __syncthreads();   // the next colour reads this colour's new spins
     }
-    block_accumulate(na, de, acc + (size_t)sw * kAccRow, 0);
+    block_store(na, de, rows + 2 * (size_t)sw);
     __syncthreads();
   }
   for (uint32_t i = threadIdx.x; i < spin_words; i += blockDim.x)
@@ -349,7 +350,6 @@ struct spk_hip_lattice {
   size_t max_lds = 0;                  // LDS bytes a workgroup may use
   int32_t *stage = nullptr;            // N int32, natural order (transfers)
   unsigned long long *acc = nullptr;   // [cap][kAccRow]: per-sweep slots
-  unsigned long long *accc = nullptr;  // [cap][2]: rows folded to (Naccept, dE)
   int acc_cap = 0;
   int block = 256;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -357,7 +357,6 @@ struct spk_hip_lattice {
   int64_t last_nlaunch = 0;
   bool energy_valid = false;
   int64_t energy = 0;                  // total energy, exact integer
-  std::vector<unsigned long long> hacc;
   // graph replay: a call of n sweeps replays n / chunk graphs of `chunk`
   // sweeps, then one graph of the remainder
   int chunk = 32;                      // sweeps per full graph (0: eager launches only)
@@ -367,15 +366,27 @@ struct spk_hip_lattice {
     hipGraphExec_t exec;
   };
   std::vector<Piece> graphs;
-  unsigned long long *pinned = nullptr;   // per-sweep rows of a call, host pinned
+  // per-sweep rows of a call, (Naccept, dE), in pinned host memory: the fold
+  // (or the one-workgroup kernel) writes them there itself, so a call takes no
+  // copy back
+  unsigned long long *pinned = nullptr;
   int pinned_rows = 0;
+  int32_t *pinned_state = nullptr;     // spins and seeds of a small lattice, natural order (download)
 };
 
 namespace {
 
 constexpr int kInitialAccRows = 1024;
+constexpr int64_t kHostStateSites = 1 << 16;   // lattices whose downloads go through pinned_state
 constexpr int kMaxChunk = 1024;   // sweeps per captured graph
 constexpr int kVec = 4;   // sites per thread in the sweep kernel
+
+// Lets a kernel take `lds` bytes of dynamic LDS (64 KiB need no leave).
+template <typename K>
+void allow_lds(K kern, size_t lds) {
+  if (lds > (64u << 10))
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+}
 
 unsigned grid_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -519,7 +530,6 @@ double pair_sweep_us(const spk_hip_lattice *h) {
 // (measured 3.5 us on sc/6n at 40^3, 4.2 on sc/26n at 32^3 to 100^3, 5.1-6.2
 // on bit planes at 256^2 to 2000^2, 7.0 for potts/neigh on sc/26n at 32^3).
 double plain_sweep_us(const spk_hip_lattice *h) {
-  const double sites = (double)h->N;
   if (resident_bytes(h)) {
     const double waves = std::ceil((double)h->g.Mp / 4 / 64);
     return h->g.K * (0.25 + std::max(1.0, waves / kSimds) * 4 * site_valu(h) * kUsPerValu * 1.2);
@@ -850,8 +860,7 @@ int launch_tile(spk_hip_lattice *h, int from, int q0, int q1, unsigned long long
     with_type(h->stype, [&]<typename T>() {
       T *s0 = static_cast<T *>(h->spin), *s1 = static_cast<T *>(h->spin2);
       auto go = [&](auto kern) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)lds);
+        allow_lds(kern, lds);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(h->tile.block), lds, h->stream, from ? s1 : s0,
                            from ? h->seed2 : h->seed, from ? s0 : s1, from ? h->seed : h->seed2, h->g, h->rule, tp,
                            acc + (size_t)(q0 / h->g.K) * kAccRow);
@@ -912,24 +921,20 @@ int launch_fold(spk_hip_lattice *h, const unsigned long long *acc, int rows, uns
   return check_hip(hipGetLastError(), "fold launch");
 }
 
-// nsweeps sweeps through the resident kernel, in pieces of at most acc_cap
-// sweeps; each piece's rows are folded and copied to pinned rows [done, ..).
+// nsweeps sweeps through the resident kernel, in pieces of at most
+// kInitialAccRows sweeps, each writing pinned rows [done, ..).
 int run_resident(spk_hip_lattice *h, int nsweeps, size_t lds, int64_t *nlaunch) {
-  const size_t row = 2 * sizeof(unsigned long long);
   int rc;
   if ((rc = check_hip(hipEventRecord(h->ev0, h->stream), "event"))) return rc;
   for (int done = 0; done < nsweeps;) {
-    const int n = std::min(nsweeps - done, h->acc_cap);
-    hipLaunchKernelGGL(k_zero_u64, dim3(grid_for((int64_t)n * kAccRow, 256)), dim3(256), 0, h->stream, h->acc,
-                       (int64_t)n * kAccRow);
+    const int n = std::min(nsweeps - done, kInitialAccRows);
     const bool two = h->rule.nspins == 2;
     with_lattice(h->g.lat, [&]<int LAT>() {
       with_type(h->stype, [&]<typename T>() {
         auto go = [&](auto kern) {
-          (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+          allow_lds(kern, lds);
           hipLaunchKernelGGL(kern, dim3(1), dim3(1024), lds, h->stream, static_cast<T *>(h->spin), h->seed, h->g,
-                             h->rule, n, h->acc);
+                             h->rule, n, h->pinned + (size_t)done * 2);
         };
         if constexpr (sizeof(T) == 1) {
           if (two) {
@@ -942,11 +947,6 @@ int run_resident(spk_hip_lattice *h, int nsweeps, size_t lds, int64_t *nlaunch) 
     });
     if ((rc = check_hip(hipGetLastError(), "resident sweep launch"))) return rc;
     (*nlaunch)++;
-    if ((rc = launch_fold(h, h->acc, n, h->accc)) ||
-        (rc = check_hip(hipMemcpyAsync(h->pinned + (size_t)done * 2, h->accc, row * n, hipMemcpyDeviceToHost,
-                                       h->stream),
-                        "accumulator readback")))
-      return rc;
     done += n;
   }
   return check_hip(hipEventRecord(h->ev1, h->stream), "event");
@@ -958,16 +958,12 @@ void row_sum(const spk_hip_lattice *h, int row, int64_t *x, int64_t *y);
 // the folded rows in pinned memory into cumulative Naccept and energies.
 int finish_sweeps(spk_hip_lattice *h, int nsweeps, int64_t nlaunch, int64_t e0, int64_t *naccept_total,
                   int64_t *naccept_per_sweep, double *energy_per_sweep) {
-  const size_t row = 2 * sizeof(unsigned long long);
   int rc;
   if ((rc = check_hip(hipStreamSynchronize(h->stream), "sweeps sync"))) return rc;
   float ms = 0.f;
   if ((rc = check_hip(hipEventElapsedTime(&ms, h->ev0, h->ev1), "event time"))) return rc;
   h->last_ms = ms;
   h->last_nlaunch = nlaunch;
-  if (h->hacc.size() < (size_t)nsweeps * 2) h->hacc.resize((size_t)nsweeps * 2);
-  std::memcpy(h->hacc.data(), h->pinned, row * nsweeps);
-
   int64_t nacc = 0, eng = e0;
   const bool track = h->energy_valid || energy_per_sweep;
   if (track && !energy_per_sweep) eng = h->energy;
@@ -988,7 +984,7 @@ int finish_sweeps(spk_hip_lattice *h, int nsweeps, int64_t nlaunch, int64_t e0, 
 
 // The graph of `n` sweeps on the current layout (bit planes or bytes):
 // a kernel zeroes accumulator rows [0, n) (no memset node), then the n
-// sweeps' launches, then the fold of those rows into accc[0, n).  Cached
+// sweeps' launches; the fold of those rows follows each replay.  Cached
 // per (n, layout) until a settings change drops the cache.
 int piece_graph(spk_hip_lattice *h, int n, Route rt, hipGraphExec_t *out) {
   for (auto &p : h->graphs)
@@ -1005,7 +1001,6 @@ int piece_graph(spk_hip_lattice *h, int n, Route rt, hipGraphExec_t *out) {
   int64_t nl = 0;
   rc = check_hip(hipGetLastError(), "zero launch");
   if (!rc) rc = rt == kRouteTile ? launch_tiles(h, n, h->acc, &nl) : launch_sweeps(h, n, h->acc, &nl);
-  if (!rc) rc = launch_fold(h, h->acc, n, h->accc);
   const hipError_t e = hipStreamEndCapture(h->stream, &graph);
   if (!rc) rc = check_hip(e, "end capture");
   if (rc) {
@@ -1052,30 +1047,23 @@ int ensure_acc(spk_hip_lattice *h, int nsweeps) {
   if (nsweeps <= h->acc_cap) return SPK_HIP_OK;
   int cap = h->acc_cap ? h->acc_cap : kInitialAccRows;
   while (cap < nsweeps) cap *= 2;
-  unsigned long long *p = nullptr, *q = nullptr;
+  unsigned long long *p = nullptr;
   if (hipMalloc(&p, (size_t)cap * kAccRow * sizeof(unsigned long long)) != hipSuccess)
     return set_error(SPK_HIP_ENOMEM, "device allocation of %d accumulator rows failed", cap);
-  if (hipMalloc(&q, (size_t)cap * 2 * sizeof(unsigned long long)) != hipSuccess) {
-    (void)hipFree(p);
-    return set_error(SPK_HIP_ENOMEM, "device allocation of %d accumulator rows failed", cap);
-  }
   if (h->acc) {
     (void)hipStreamSynchronize(h->stream);
     (void)hipFree(h->acc);
-    (void)hipFree(h->accc);
   }
   drop_graphs(h);   // the accumulator addresses are baked into captured launches
   h->acc = p;
-  h->accc = q;
   h->acc_cap = cap;
-  h->hacc.resize((size_t)cap * 2);
   return SPK_HIP_OK;
 }
 
-// (Naccept, dE) of accumulator row `row`, already folded and copied to h->hacc
+// (Naccept, dE) of accumulator row `row`, already folded into h->pinned
 void row_sum(const spk_hip_lattice *h, int row, int64_t *x, int64_t *y) {
-  *x = (int64_t)h->hacc[2 * (size_t)row];
-  *y = (int64_t)h->hacc[2 * (size_t)row + 1];
+  *x = (int64_t)h->pinned[2 * (size_t)row];
+  *y = (int64_t)h->pinned[2 * (size_t)row + 1];
 }
 
 int compute_energy(spk_hip_lattice *h, int64_t *e) {
@@ -1083,11 +1071,7 @@ int compute_energy(spk_hip_lattice *h, int64_t *e) {
   if ((rc = bits_leave(h)) || (rc = ensure_acc(h, 1))) return rc;
   if ((rc = check_hip(hipMemsetAsync(h->acc, 0, kAccRow * sizeof(unsigned long long), h->stream), "memset")))
     return rc;
-  if ((rc = launch_energy(h, h->acc)) || (rc = launch_fold(h, h->acc, 1, h->accc))) return rc;
-  if ((rc = check_hip(hipMemcpyAsync(h->hacc.data(), h->accc, 2 * sizeof(unsigned long long),
-                                     hipMemcpyDeviceToHost, h->stream),
-                      "energy readback")))
-    return rc;
+  if ((rc = launch_energy(h, h->acc)) || (rc = launch_fold(h, h->acc, 1, h->pinned))) return rc;
   if ((rc = check_hip(hipStreamSynchronize(h->stream), "energy sync"))) return rc;
   int64_t y;
   row_sum(h, 0, e, &y);
@@ -1129,11 +1113,11 @@ int validate_on_device(spk_hip_lattice *h, const int32_t *buf, int lo, int hi, i
   hipLaunchKernelGGL(k_count_outside, dim3(grid_for(h->N, 256)), dim3(256), 0, h->stream, buf, h->N, lo,
                      hi, h->acc);
   if ((rc = check_hip(hipGetLastError(), "validate launch"))) return rc;
-  unsigned long long v = 0;
-  if ((rc = check_hip(hipMemcpyAsync(&v, h->acc, sizeof(v), hipMemcpyDeviceToHost, h->stream), "readback")))
+  if ((rc = check_hip(hipMemcpyAsync(h->pinned, h->acc, sizeof(*h->pinned), hipMemcpyDeviceToHost, h->stream),
+                      "readback")) ||
+      (rc = check_hip(hipStreamSynchronize(h->stream), "validate sync")))
     return rc;
-  if ((rc = check_hip(hipStreamSynchronize(h->stream), "validate sync"))) return rc;
-  *nbad = (int64_t)v;
+  *nbad = (int64_t)h->pinned[0];
   return SPK_HIP_OK;
 }
 
@@ -1220,7 +1204,7 @@ void spk_hip_destroy(spk_hip_lattice *h) {
   if (h->spin2) (void)hipFree(h->spin2);
   if (h->seed2) (void)hipFree(h->seed2);
   if (h->acc) (void)hipFree(h->acc);
-  if (h->accc) (void)hipFree(h->accc);
+  if (h->pinned_state) (void)hipHostFree(h->pinned_state);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1275,25 +1259,45 @@ int spk_hip_download(spk_hip_lattice *h, int32_t *spin, int32_t *seed) {
   const size_t bytes = (size_t)h->N * sizeof(int32_t);
   int rc;
   if ((rc = bits_leave(h))) return rc;
+  if (!spin && !seed) return SPK_HIP_OK;
+  // small lattices: one kernel writes the arrays to host memory, and one wait
+  // ends it.  As two kernels, two copies and two waits, and so: 64^2 30.8 and
+  // 13.9 us, 128^2 45.5 and 17.4, 40^3 52.5 and 32.0; from 50^3 on the copy out
+  // of that memory takes what is saved.
+  if (h->N <= kHostStateSites &&
+      (h->pinned_state ||
+       hipHostMalloc(&h->pinned_state, 2 * bytes, hipHostMallocDefault) == hipSuccess)) {
+    with_type(h->stype, [&]<typename T>() {
+      hipLaunchKernelGGL((k_state_natural<T>), dim3(grid_for(h->N, 256)), dim3(256), 0, h->stream,
+                         spin ? static_cast<const T *>(h->spin) : nullptr, seed ? h->seed : nullptr, h->pinned_state,
+                         h->g);
+    });
+    if ((rc = check_hip(hipGetLastError(), "layout kernel")) ||
+        (rc = check_hip(hipStreamSynchronize(h->stream), "download sync")))
+      return rc;
+    if (spin) std::memcpy(spin, h->pinned_state, bytes);
+    if (seed) std::memcpy(seed, h->pinned_state + h->N, bytes);
+    return SPK_HIP_OK;
+  }
+  // the second kernel writes the staging array after the first copy has read
+  // it (stream order)
   if (spin) {
     with_type(h->stype, [&]<typename T>() {
       hipLaunchKernelGGL((k_to_natural<T>), dim3(grid_for(h->N, 256)), dim3(256), 0, h->stream,
                          static_cast<const T *>(h->spin), h->stage, h->g);
     });
-    if ((rc = check_hip(hipGetLastError(), "layout kernel"))) return rc;
-    if ((rc = check_hip(hipMemcpyAsync(spin, h->stage, bytes, hipMemcpyDeviceToHost, h->stream), "download")))
+    if ((rc = check_hip(hipGetLastError(), "layout kernel")) ||
+        (rc = check_hip(hipMemcpyAsync(spin, h->stage, bytes, hipMemcpyDeviceToHost, h->stream), "download")))
       return rc;
-    if ((rc = check_hip(hipStreamSynchronize(h->stream), "download sync"))) return rc;
   }
   if (seed) {
     hipLaunchKernelGGL(k_to_natural<int32_t>, dim3(grid_for(h->N, 256)), dim3(256), 0, h->stream, h->seed,
                        h->stage, h->g);
-    if ((rc = check_hip(hipGetLastError(), "layout kernel"))) return rc;
-    if ((rc = check_hip(hipMemcpyAsync(seed, h->stage, bytes, hipMemcpyDeviceToHost, h->stream), "download")))
+    if ((rc = check_hip(hipGetLastError(), "layout kernel")) ||
+        (rc = check_hip(hipMemcpyAsync(seed, h->stage, bytes, hipMemcpyDeviceToHost, h->stream), "download")))
       return rc;
-    if ((rc = check_hip(hipStreamSynchronize(h->stream), "download sync"))) return rc;
   }
-  return SPK_HIP_OK;
+  return check_hip(hipStreamSynchronize(h->stream), "download sync");
 }
 
 int spk_hip_set_range(spk_hip_lattice *h, int seed0, int lo, int hi) {
@@ -1353,11 +1357,9 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
     if (h->energy_valid) e0 = h->energy;
     else if ((rc = compute_energy(h, &e0))) return rc;
   }
-  const size_t row = 2 * sizeof(unsigned long long);   // a folded row
   int64_t nlaunch = 0;
   if (const size_t lds = resident_call(h, nsweeps)) {
-    if ((rc = bits_leave(h)) || (rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows))) ||
-        (rc = ensure_pinned(h, nsweeps)) || (rc = run_resident(h, nsweeps, lds, &nlaunch)))
+    if ((rc = bits_leave(h)) || (rc = ensure_pinned(h, nsweeps)) || (rc = run_resident(h, nsweeps, lds, &nlaunch)))
       return rc;
     return finish_sweeps(h, nsweeps, nlaunch, e0, naccept_total, naccept_per_sweep, energy_per_sweep);
   }
@@ -1365,8 +1367,8 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
   Route rt;
   if ((rc = enter_route(h, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
   if (h->chunk > 0) {
-    // graph replays (graph_pieces); each piece's rows are folded into
-    // accc[0, n) and copied to the pinned rows [done, done + n) in stream order
+    // graph replays (graph_pieces); each piece's rows are folded into the
+    // pinned rows [done, done + n) before the next piece clears them
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
     if ((rc = ensure_acc(h, pieces[0]))) return rc;
     std::vector<hipGraphExec_t> execs(pieces.size());
@@ -1376,9 +1378,7 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
     int done = 0;
     for (size_t k = 0; k < pieces.size(); k++) {
       if ((rc = check_hip(hipGraphLaunch(execs[k], h->stream), "graph launch")) ||
-          (rc = check_hip(hipMemcpyAsync(h->pinned + (size_t)done * 2, h->accc, row * pieces[k],
-                                         hipMemcpyDeviceToHost, h->stream),
-                          "accumulator readback")))
+          (rc = launch_fold(h, h->acc, pieces[k], h->pinned + (size_t)done * 2)))
         return rc;
       done += pieces[k];
     }
@@ -1392,9 +1392,7 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
     if ((rc = check_hip(hipGetLastError(), "zero launch")) ||
         (rc = rt == kRouteTile ? launch_tiles(h, nsweeps, h->acc, &nlaunch)
                                : launch_sweeps(h, nsweeps, h->acc, &nlaunch)) ||
-        (rc = launch_fold(h, h->acc, nsweeps, h->accc)) ||
-        (rc = check_hip(hipMemcpyAsync(h->pinned, h->accc, row * nsweeps, hipMemcpyDeviceToHost, h->stream),
-                        "accumulator readback")))
+        (rc = launch_fold(h, h->acc, nsweeps, h->pinned)))
       return rc;
   }
   if ((rc = check_hip(hipEventRecord(h->ev1, h->stream), "event"))) return rc;
@@ -1462,11 +1460,11 @@ int spk_hip_checksum(spk_hip_lattice *h, uint64_t *sum) {
                        static_cast<const T *>(h->spin), h->seed, h->g, h->acc);
   });
   if ((rc = check_hip(hipGetLastError(), "checksum launch"))) return rc;
-  unsigned long long v = 0;
-  if ((rc = check_hip(hipMemcpyAsync(&v, h->acc, sizeof v, hipMemcpyDeviceToHost, h->stream), "readback")) ||
+  if ((rc = check_hip(hipMemcpyAsync(h->pinned, h->acc, sizeof(*h->pinned), hipMemcpyDeviceToHost, h->stream),
+                      "readback")) ||
       (rc = check_hip(hipStreamSynchronize(h->stream), "sync")))
     return rc;
-  *sum = v;
+  *sum = h->pinned[0];
   return SPK_HIP_OK;
 }
 
