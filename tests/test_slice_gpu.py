@@ -52,7 +52,7 @@ def test_sliced_sweeps_equal_oracle(orc, case):
 
 def test_state_carries_from_planes_to_sweeps_without_allocation(orc):
     import spparks_amd as S
-    import torch
+    from test_zz_no_alloc import DeviceRows
     d = orc.make_desc("potts", "sc/26n", 128, 128, 128, 500, 0.6)
     spin, seeds = orc.script_init(d, 9, 1, 500)
     orc.sweeps(d, spin, seeds, 3)
@@ -61,9 +61,10 @@ def test_state_carries_from_planes_to_sweeps_without_allocation(orc):
         L.set_range(s0, 1, 500)
         L.init_seeds(rseed)
         L.sweeps(1)
-        rows = torch.zeros(2, dtype=torch.int64, device="cuda")
-        L.sweeps_noalloc(1, rows.data_ptr())
+        rows = DeviceRows(2)
+        L.sweeps_noalloc(1, rows.ptr.value)
         L.sync()
+        rows.free()
         L.sweeps(1)
         s, k = L.download()
     assert np.array_equal(s, spin) and np.array_equal(k, seeds)
