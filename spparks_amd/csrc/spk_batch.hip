@@ -7,14 +7,15 @@
 #include <algorithm>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <new>
-#include <tuple>
 #include <vector>
 
 #include "spk_batch_async.h"
 #include "spk_device.h"
 #include "spk_host.h"
 #include "spk_kernels.h"
+#include "spk_slice.h"
 
 using namespace spk;
 
@@ -30,6 +31,11 @@ struct BatchRep {
   int tiles;       // tiles per pass
   int64_t spin_off;  // byte offsets into the pool
   int64_t seed_off;
+  // replicas of k_batch_slice only (P counts colour pairs, a tile is a
+  // wavefront's rows)
+  SliceGeom s;
+  uint32_t *planes;
+  int32_t *sseed;
 };
 
 // Active replicas of one step: table indices act[first .. first+count) with
@@ -138,7 +144,62 @@ __global__ __launch_bounds__(1024) void k_batch_step(char *__restrict__ pool, co
   }
 }
 
-constexpr int kNumVariants = 12;   // 4 lattice styles x 3 spin storage types
+// One step of the replicas that sweep on bit planes of the spins
+// (spk_slice.h): both colours of a row pair, a wavefront a tile.  A tile is
+// some 1000 site events in one chain of about 10 us, so every tile of the step
+// has a wavefront of its own (those past the last leave) and the hardware
+// spreads them; the replicas' plane counts differ, hence the switch, which is
+// the same on a whole wavefront.
+// Batches of 100 sweeps, ms a sweep of the device, packed spins and planes:
+// 32 replicas of edge 34..126 (13.6M sites) beside 32 two-state ones 0.151,
+// 0.098; 24 solves of edge 32..190 (18.2e9 updates in all) 128, 94 ms.  What
+// bounds it is k_sweep_slice's (VALU and a wavefront's own chain), on words a
+// quarter empty on the average, and the last wavefronts of a step.  Replicas
+// with most planes first in the list: 0.099 and 97, taken back.
+constexpr int kSliceBlock = 256;
+
+__global__ __launch_bounds__(kSliceBlock, 4) void k_batch_slice(const BatchRep *__restrict__ reps,
+                                                             const StepDesc *__restrict__ steps,
+                                                             const int *__restrict__ act, const int *__restrict__ pre,
+                                                             int j, int L, unsigned long long *__restrict__ acc) {
+  __shared__ SliceLds lds[kSliceBlock / 64];
+  const StepDesc sd = steps[j];
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int t = xcd_tile(blockIdx.x, gridDim.x) * (kSliceBlock / 64) + wid;
+  if (t >= sd.total) return;   // no wavefront waits for another
+  const int *pp = pre + sd.pre_first;
+  int lo = 0, hi = sd.count - 1;   // the replica holding tile t: last i with pp[i] <= t
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (pp[mid] <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  const BatchRep &rep = reps[act[sd.first + lo]];
+  const Geom g = rep.g;
+  const SliceGeom s = rep.s;
+  const int p = (int)(((int64_t)j * rep.P) / L);
+  SliceCounts n;
+  with_plane_groups(s.PG, [&]<int PG>() {
+    slice_wave<false, PG>(rep.planes, rep.sseed, g, s, rep.rule, lds[wid], p % (g.K / 2), (uint32_t)(t - pp[lo]),
+                          threadIdx.x & 63, n);
+  });
+  const Counts cnt = slice_counts(n);
+  wave_accumulate(cnt.nacc, cnt.de, acc + (int64_t)(rep.acc_row + p / (g.K / 2)) * kBatchRow, t & (kBatchSlots - 1));
+}
+
+// natural order of a sliced replica's spins (sseed null) or seeds (planes null)
+__global__ void k_slice_natural(const uint32_t *__restrict__ planes, const int32_t *__restrict__ sseed, Geom g,
+                                SliceGeom s, int32_t *__restrict__ nat) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (int64_t)g.M * g.K) return;
+  int i, j, k;
+  natural_ijk(g, t, i, j, k);
+  const SliceSite x = slice_site(g, s, i, j, k);
+  nat[t] = planes ? slice_spin_at(planes, s, x) : sseed[slice_seed_slot(s, x)];
+}
+
+constexpr int kSliceVariant = 12;
+constexpr int kNumVariants = 13;   // 4 lattice styles x 3 spin storage types, and k_batch_slice
 
 __global__ void k_fill_u64(unsigned long long *__restrict__ v, int64_t n) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -165,7 +226,14 @@ struct Replica {
   int block_sweeps = 0;             // sweeps in the current block
   int acc_row = 0;
   bool energy_pending = false;      // initial energy on its way to pinned memory
-  int variant = 0;                  // lat*3 + stype: which step kernel runs it
+  int variant = 0;                  // lat*3 + stype, or kSliceVariant: which step kernel runs it
+  // on planes these hold the state, and the pool's extent an older one while
+  // `stale`
+  SliceGeom s{};
+  uint32_t *planes = nullptr;
+  int32_t *sseed = nullptr;
+  int64_t side_bytes = 0;
+  bool stale = false;
 };
 
 // first-fit extent allocator with coalescing
@@ -216,6 +284,62 @@ struct Shape {
   int block, grid;
 };
 
+// Device memory for the planes of sliced replicas, beside the pool (whose
+// extents and admission are as for any replica): chunks taken as replicas need
+// them and given back with the batch.  A chunk is taken only while a quarter of
+// the device's memory stays free; a replica without one runs on its packed spins.
+class SideMemory {
+ public:
+  ~SideMemory() {
+    for (auto &c : chunks_) (void)hipFree(c->base);
+  }
+  char *take(int64_t n) {
+    int64_t off;
+    for (auto &c : chunks_)
+      if (c->alloc.alloc(n, &off)) return c->base + off;
+    const int64_t size = std::max<int64_t>(n, (int64_t)64 << 20);
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || (int64_t)free_bytes - size < (int64_t)(total / 4)) return nullptr;
+    char *p = nullptr;
+    if (hipMalloc(&p, (size_t)size) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    chunks_.push_back(std::make_unique<Chunk>(p, size));
+    chunks_.back()->alloc.alloc(n, &off);
+    return p + off;
+  }
+  void give(char *p, int64_t n) {
+    for (auto &c : chunks_)
+      if (p >= c->base && p < c->base + c->size) c->alloc.release(p - c->base, n);
+  }
+
+ private:
+  struct Chunk {
+    char *base;
+    int64_t size;
+    PoolAlloc alloc;
+    Chunk(char *b, int64_t n) : base(b), size(n), alloc(n) {}
+  };
+  std::vector<std::unique_ptr<Chunk>> chunks_;
+};
+
+// Replicas that sweep on bit planes: those that leave at least half of a
+// step's bits to real sites.  G updates/s, packed and on planes, Q = 100 and
+// 10^4: 128 replicas of 36^3 (0.56 full) 81.1, 119.7 and 78.2, 96.8; 32 of 66^3
+// (0.52) 97.0, 136.6 and 87.0, 106.4; 2000 of 24^3 (0.375) 145.3, 137.2 and
+// 135.9, 110.6.  (Few replicas of 24^3 gain as well, a step's time being a
+// wavefront's own and the steps half as many: 256 of them 60.1, 71.3; the line
+// is where it holds for any number.)
+constexpr double kSliceFill = 0.5;
+
+bool slice_batched(const Geom &g, const Rule &r) {
+  if (!slice_fits(g, r.nspins) || r.half != (1 << 30)) return false;
+  const SliceGeom s = slice_geom(g, r.nspins);
+  const double fill = (double)g.hx / (32 * s.pw) * (s.rw * s.pw / 16.0) * s.rows / ((double)s.waves * s.rw);
+  return fill >= kSliceFill;
+}
+
 }  // namespace
 
 struct spk_hip_batch {
@@ -225,6 +349,7 @@ struct spk_hip_batch {
   char *pool = nullptr;
   int64_t pool_bytes = 0;
   PoolAlloc *alloc = nullptr;
+  SideMemory side;
   std::vector<Replica> reps;        // slot table
   // staging for transfers and per-replica set-up
   int32_t *stage = nullptr;
@@ -240,12 +365,19 @@ struct spk_hip_batch {
   std::vector<int> h_act, h_pre;
   std::vector<unsigned long long> h_acc;
   // variants present in the current block, one stream each (fork/join)
-  std::vector<int> variants;
+  struct Variant {
+    int v;        // which step kernel
+    int L;        // its steps
+    int first;    // of them in h_steps
+    int grid;     // workgroups of the largest step (k_batch_slice)
+  };
+  std::vector<Variant> variants;
   hipStream_t vstream[kNumVariants] = {};
   hipEvent_t fork_ev = nullptr, join_ev[kNumVariants] = {};
   // launch shape
   int block = 0, grid = 0;          // 0 = autotune on the next run
-  std::map<std::tuple<int, int, int, int>, hipGraphExec_t> graphs;   // (L, block, grid, variant mask)
+  // by (block, grid, then v and L of each variant), then by k_batch_slice's grid
+  std::map<std::vector<int>, std::map<int, hipGraphExec_t>> graphs;
   std::vector<hipEvent_t> events;
   double last_ms = 0.0;
   int64_t last_updates = 0, last_nlaunch = 0;
@@ -336,7 +468,12 @@ void resolve_energies(spk_hip_batch *b) {
 // Queues the checksum of replica slot `id` (after everything already on the
 // batch stream) into its device slot and pinned copy.
 int replica_checksum_async(spk_hip_batch *b, int id) {
-  const Replica &R = b->reps[id];
+  Replica &R = b->reps[id];
+  if (R.stale) {
+    slice_out(b->stream, R.planes, R.sseed, R.g, R.s, b->pool + R.spin_off, R.stype,
+              reinterpret_cast<int32_t *>(b->pool + R.seed_off));
+    R.stale = false;
+  }
   unsigned long long *out = b->d_slot + 4 * (size_t)id + 2;
   hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, b->stream, out, (int64_t)1);
   const int64_t n = (int64_t)R.g.M * R.g.K;
@@ -355,15 +492,15 @@ int replica_checksum_async(spk_hip_batch *b, int id) {
 
 // Builds the block's replica table and, per variant present, the step
 // schedule.  Replica r with P_r passes is due at step j when
-// floor((j+1)P_r/L) > floor(j P_r/L); its pass index is then floor(j P_r/L),
-// so its passes run once each, in order.  Steps of variant k live at
-// h_steps[k*L + j].
+// floor((j+1)P_r/L) > floor(j P_r/L), L being its variant's steps; its pass
+// index is then floor(j P_r/L), so its passes run once each, in order.  L_out
+// is the largest of the variants' L, which launch_steps counts in.
 int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, int64_t *updates_out) {
   b->h_reps.clear();
   std::vector<int> vrep;   // variant of each table entry
   int L = 0, rows = 0;
   int64_t updates = 0;
-  bool present[kNumVariants] = {};
+  int steps[kNumVariants] = {};
   for (int id = 0; id < (int)b->reps.size(); id++) {
     Replica &R = b->reps[id];
     R.block_sweeps = 0;
@@ -377,42 +514,50 @@ int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, 
     br.g = R.g;
     br.rule = R.rule;
     br.stype = R.stype;
-    br.P = R.g.K * R.block_sweeps;
+    const bool sliced = R.variant == kSliceVariant;
+    br.P = (sliced ? R.g.K / 2 : R.g.K) * R.block_sweeps;
     br.acc_row = R.acc_row;
-    br.tiles = (int)((R.g.Mp / kVec + kTile - 1) / kTile);
+    br.tiles = sliced ? R.s.waves : (int)((R.g.Mp / kVec + kTile - 1) / kTile);
     br.spin_off = R.spin_off;
     br.seed_off = R.seed_off;
+    br.s = R.s;
+    br.planes = R.planes;
+    br.sseed = R.sseed;
+    R.stale = sliced;
     b->h_reps.push_back(br);
     vrep.push_back(R.variant);
-    present[R.variant] = true;
+    steps[R.variant] = std::max(steps[R.variant], br.P);
     L = std::max(L, br.P);
     updates += (int64_t)R.g.M * R.g.K * R.block_sweeps;
   }
   b->variants.clear();
-  for (int v = 0; v < kNumVariants; v++)
-    if (present[v]) b->variants.push_back(v);
-  b->h_steps.assign((size_t)L * b->variants.size(), StepDesc{0, 0, 0, 0});
+  b->h_steps.clear();
   b->h_act.clear();
   b->h_pre.clear();
-  for (size_t k = 0; k < b->variants.size(); k++)
-    for (int j = 0; j < L; j++) {
-      StepDesc &sd = b->h_steps[k * L + j];
-      sd.first = (int)b->h_act.size();
-      sd.pre_first = (int)b->h_pre.size();
-      int tot = 0;
+  for (int v = 0; v < kNumVariants; v++) {
+    if (!steps[v]) continue;
+    spk_hip_batch::Variant var{v, steps[v], (int)b->h_steps.size(), 0};
+    for (int j = 0; j < var.L; j++) {
+      StepDesc sd{(int)b->h_act.size(), 0, (int)b->h_pre.size(), 0};
       b->h_pre.push_back(0);
       for (int r = 0; r < (int)b->h_reps.size(); r++) {
-        if (vrep[r] != b->variants[k]) continue;
+        if (vrep[r] != v) continue;
         const int64_t P = b->h_reps[r].P;
-        if (((int64_t)(j + 1) * P) / L > ((int64_t)j * P) / L) {
+        if (((int64_t)(j + 1) * P) / var.L > ((int64_t)j * P) / var.L) {
           b->h_act.push_back(r);
-          tot += b->h_reps[r].tiles;
-          b->h_pre.push_back(tot);
+          sd.total += b->h_reps[r].tiles;
+          b->h_pre.push_back(sd.total);
         }
       }
       sd.count = (int)b->h_act.size() - sd.first;
-      sd.total = tot;
+      b->h_steps.push_back(sd);
+      if (v == kSliceVariant) {
+        const int wg = (sd.total + kSliceBlock / 64 - 1) / (kSliceBlock / 64);
+        var.grid = std::max(var.grid, (wg + kNumXcd - 1) / kNumXcd * kNumXcd);
+      }
     }
+    b->variants.push_back(var);
+  }
   *L_out = L;
   *rows_out = rows;
   *updates_out = updates;
@@ -420,7 +565,8 @@ int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, 
 }
 
 void drop_graphs(spk_hip_batch *b) {
-  for (auto &kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
+  for (auto &kv : b->graphs)
+    for (auto &gv : kv.second) (void)hipGraphExecDestroy(gv.second);
   b->graphs.clear();
 }
 
@@ -455,7 +601,8 @@ int ensure_streams(spk_hip_batch *b) {
   int rc;
   if (!b->fork_ev && (rc = check_hip(hipEventCreateWithFlags(&b->fork_ev, hipEventDisableTiming), "event")))
     return rc;
-  for (int v : b->variants) {
+  for (const auto &var : b->variants) {
+    const int v = var.v;
     if (!b->vstream[v] && (rc = check_hip(hipStreamCreate(&b->vstream[v]), "hipStreamCreate"))) return rc;
     if (!b->join_ev[v] && (rc = check_hip(hipEventCreateWithFlags(&b->join_ev[v], hipEventDisableTiming), "event")))
       return rc;
@@ -463,31 +610,43 @@ int ensure_streams(spk_hip_batch *b) {
   return SPK_HIP_OK;
 }
 
-// Steps j0..j1-1 of the block: each variant's chain on its own stream,
-// forked from and joined back into the batch stream (so a graph captured on
-// the batch stream holds one independent branch per variant).
+// Steps j0..j1-1 of the block's L (a variant with fewer takes its own in step
+// with them): each variant's chain on its own stream, forked from and joined
+// back into the batch stream (so a graph captured on the batch stream holds
+// one independent branch per variant).
 int launch_steps(spk_hip_batch *b, int j0, int j1, int L, int block, int grid) {
   int rc;
   if ((rc = check_hip(hipEventRecord(b->fork_ev, b->stream), "fork"))) return rc;
-  for (int v : b->variants)
-    if ((rc = check_hip(hipStreamWaitEvent(b->vstream[v], b->fork_ev, 0), "fork wait"))) return rc;
+  for (const auto &var : b->variants)
+    if ((rc = check_hip(hipStreamWaitEvent(b->vstream[var.v], b->fork_ev, 0), "fork wait"))) return rc;
   for (int j = j0; j < j1; j++)
-    for (size_t k = 0; k < b->variants.size(); k++) {
-      const int v = b->variants[k];
-      const StepDesc *steps = b->d_steps + k * L;
-      with_lattice(v / 3, [&]<int LAT>() {
-        with_type(v % 3, [&]<typename T>() {
-          hipLaunchKernelGGL((k_batch_step<LAT, T>), dim3(grid), dim3(block), 0, b->vstream[v], b->pool, b->d_reps,
-                             steps, b->d_act, b->d_pre, j, L, b->d_acc);
+    for (const auto &var : b->variants) {
+      const int v = var.v, at = (int)(((int64_t)j * var.L) / L);
+      if (at == (int)(((int64_t)(j + 1) * var.L) / L)) continue;
+      const StepDesc *steps = b->d_steps + var.first;
+      if (v == kSliceVariant)
+        hipLaunchKernelGGL(k_batch_slice, dim3(var.grid), dim3(kSliceBlock), 0, b->vstream[v], b->d_reps, steps,
+                           b->d_act, b->d_pre, at, var.L, b->d_acc);
+      else
+        with_lattice(v / 3, [&]<int LAT>() {
+          with_type(v % 3, [&]<typename T>() {
+            hipLaunchKernelGGL((k_batch_step<LAT, T>), dim3(grid), dim3(block), 0, b->vstream[v], b->pool, b->d_reps,
+                               steps, b->d_act, b->d_pre, at, var.L, b->d_acc);
+          });
         });
-      });
       if ((rc = check_hip(hipGetLastError(), "step kernel launch"))) return rc;
     }
-  for (int v : b->variants) {
-    if ((rc = check_hip(hipEventRecord(b->join_ev[v], b->vstream[v]), "join"))) return rc;
-    if ((rc = check_hip(hipStreamWaitEvent(b->stream, b->join_ev[v], 0), "join wait"))) return rc;
+  for (const auto &var : b->variants) {
+    if ((rc = check_hip(hipEventRecord(b->join_ev[var.v], b->vstream[var.v]), "join"))) return rc;
+    if ((rc = check_hip(hipStreamWaitEvent(b->stream, b->join_ev[var.v], 0), "join wait"))) return rc;
   }
   return SPK_HIP_OK;
+}
+
+int64_t block_launches(const spk_hip_batch *b) {
+  int64_t n = 0;
+  for (const auto &var : b->variants) n += var.L;
+  return n;
 }
 
 int ensure_events(spk_hip_batch *b, size_t n) {
@@ -637,9 +796,21 @@ int spk::batch_add_async(spk_hip_batch *b, const spk_hip_replica_desc *r, int *i
   });
   hipLaunchKernelGGL(k_init_seeds, dim3(gs), dim3(256), 0, b->stream, seed, R.g, draws[4] * (double)kIM,
                      park_warmup100());
+  if (slice_batched(R.g, R.rule)) {
+    R.s = slice_geom(R.g, R.rule.nspins);
+    const int64_t pbytes = round_up((int64_t)R.g.K * R.s.PG * R.s.nw * (int64_t)sizeof(Words<4>), 256);
+    R.side_bytes = pbytes + round_up(R.g.K * R.s.seedc * 4, 256);
+    if (char *p = b->side.take(R.side_bytes)) {
+      R.variant = kSliceVariant;
+      R.planes = reinterpret_cast<uint32_t *>(p);
+      R.sseed = reinterpret_cast<int32_t *>(p + pbytes);
+      slice_in(b->stream, b->pool + R.spin_off, R.stype, seed, R.g, R.s, R.planes, R.sseed);
+    }
+  }
   if ((rc = check_hip(hipGetLastError(), "replica set-up launch")) ||
       (rc = replica_energy_async(b, slot, R))) {
     b->alloc->release(R.off, R.bytes);
+    if (R.planes) b->side.give(reinterpret_cast<char *>(R.planes), R.side_bytes);
     return rc;
   }
   R.live = true;
@@ -664,6 +835,7 @@ int spk_hip_batch_remove(spk_hip_batch *b, int id) {
   if (rc || (rc = batch_complete(b))) return rc;
   Replica &R = b->reps[id];
   b->alloc->release(R.off, R.bytes);
+  if (R.planes) b->side.give(reinterpret_cast<char *>(R.planes), R.side_bytes);
   R = Replica();
   return SPK_HIP_OK;
 }
@@ -693,6 +865,9 @@ int spk_hip_batch_upload(spk_hip_batch *b, int id, const int32_t *spin, const in
       hipLaunchKernelGGL(k_to_blocked<int32_t>, dim3(grid_for(n, 256)), dim3(256), 0, b->stream, b->stage,
                          reinterpret_cast<int32_t *>(b->pool + R.seed_off), R.g);
     }
+    if (R.planes)
+      slice_in(b->stream, w == 0 ? b->pool + R.spin_off : nullptr, R.stype,
+               w == 0 ? nullptr : reinterpret_cast<const int32_t *>(b->pool + R.seed_off), R.g, R.s, R.planes, R.sseed);
     if ((rc = check_hip(hipGetLastError(), "layout kernel"))) return rc;
   }
   if (spin && (rc = replica_energy_async(b, id, R))) return rc;
@@ -710,7 +885,10 @@ int spk_hip_batch_download(spk_hip_batch *b, int id, int32_t *spin, int32_t *see
   for (int w = 0; w < 2; w++) {
     int32_t *dst = w == 0 ? spin : seed;
     if (!dst) continue;
-    if (w == 0) {
+    if (R.planes) {
+      hipLaunchKernelGGL(k_slice_natural, dim3(grid_for(n, 256)), dim3(256), 0, b->stream, w == 0 ? R.planes : nullptr,
+                         R.sseed, R.g, R.s, b->stage);
+    } else if (w == 0) {
       with_type(R.stype, [&]<typename T>() {
         hipLaunchKernelGGL((k_to_natural<T>), dim3(grid_for(n, 256)), dim3(256), 0, b->stream,
                            reinterpret_cast<const T *>(b->pool + R.spin_off), b->stage, R.g);
@@ -791,19 +969,27 @@ int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph) {
   int64_t updates = 0;
   if ((rc = build_schedule(b, max_sweeps, &L, &rows, &updates))) return rc;
   b->last_updates = updates;
-  b->last_nlaunch = (int64_t)L * (int64_t)std::max<size_t>(1, b->variants.size());
+  b->last_nlaunch = block_launches(b);
   b->last_ms = 0.0;
   if (L == 0) return SPK_HIP_OK;
   if ((rc = ensure_events(b, 2 * (size_t)L + 2)) || (rc = ensure_streams(b)) ||
       (rc = upload_schedule(b, rows, true)))
     return rc;
   const Shape sh{b->block, b->grid};
-  int mask = 0;
-  for (int v : b->variants) mask |= 1 << v;
   if (use_graph) {
-    auto key = std::make_tuple(L, sh.block, sh.grid, mask);
-    auto it = b->graphs.find(key);
-    if (it == b->graphs.end()) {
+    std::vector<int> key{sh.block, sh.grid};
+    int need = 0;   // workgroups of k_batch_slice
+    for (const auto &var : b->variants) {
+      key.push_back(var.v);
+      key.push_back(var.L);
+      if (var.v == kSliceVariant) need = var.grid;
+    }
+    // a graph recorded for more workgroups serves, up to half as many again
+    // (the surplus ones leave at once): a queue of solves changes its tiles
+    // with every one that comes or goes
+    auto &shapes = b->graphs[key];
+    auto it = shapes.lower_bound(need);
+    if (it == shapes.end() || it->first > need + need / 2) {
       hipGraph_t graph = nullptr;
       if ((rc = check_hip(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "begin capture")))
         return rc;
@@ -818,7 +1004,7 @@ int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph) {
       rc = check_hip(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "graph instantiate");
       (void)hipGraphDestroy(graph);
       if (rc) return rc;
-      it = b->graphs.emplace(key, exec).first;
+      it = shapes.emplace(need, exec).first;
     }
     if ((rc = check_hip(hipEventRecord(b->events[0], b->stream), "event")) ||
         (rc = check_hip(hipGraphLaunch(it->second, b->stream), "graph launch")) ||
@@ -881,7 +1067,7 @@ int spk_hip_batch_run(spk_hip_batch *b, int max_sweeps, int use_graph) {
   int64_t updates = 0;
   if ((rc = build_schedule(b, max_sweeps, &L, &rows, &updates))) return rc;
   b->last_updates = updates;
-  b->last_nlaunch = (int64_t)L * (int64_t)std::max<size_t>(1, b->variants.size());
+  b->last_nlaunch = block_launches(b);
   if (L == 0) {
     b->last_ms = 0.0;
     return SPK_HIP_OK;
@@ -894,16 +1080,20 @@ int spk_hip_batch_run(spk_hip_batch *b, int max_sweeps, int use_graph) {
     // the block's own steps, as a replay runs them (no wait between steps);
     // results do not depend on the shape.  The tile list is the same for
     // every shape (a tile is one wavefront's work).
+    // (k_batch_slice has its own grid: a block of nothing else has nothing to try)
     std::vector<Shape> cand;
-    for (int bs : {64, 128, 256})
-      for (int wpc : {8, 16, 32}) {
+    const bool only_sliced = b->variants.size() == 1 && b->variants[0].v == kSliceVariant;
+    for (int bs : only_sliced ? std::vector<int>{256} : std::vector<int>{64, 128, 256})
+      for (int wpc : only_sliced ? std::vector<int>{16} : std::vector<int>{8, 16, 32}) {
         const int grid = std::max(kNumXcd, b->ncu * wpc * 64 / bs / kNumXcd * kNumXcd);
         cand.push_back(Shape{bs, grid});
       }
     auto step_work = [&](int j) {   // sites updated in step j
       double w = 0.0;
-      for (size_t k = 0; k < b->variants.size(); k++) {
-        const StepDesc &sd = b->h_steps[k * L + j];
+      for (const auto &var : b->variants) {
+        const int at = (int)(((int64_t)j * var.L) / L);
+        if (at == (int)(((int64_t)(j + 1) * var.L) / L)) continue;
+        const StepDesc &sd = b->h_steps[var.first + at];
         for (int a = 0; a < sd.count; a++) w += (double)b->h_reps[b->h_act[sd.first + a]].g.M;
       }
       return w;

@@ -5,6 +5,7 @@
 
 #include "spk_device.h"
 #include "spk_host.h"
+#include "spk_slice.h"
 
 namespace spk {
 namespace {
@@ -69,6 +70,50 @@ __global__ void k_state_natural(const T *__restrict__ spin, const int32_t *__res
   const int64_t p = blocked_index(g, i, j, k);
   if (spin) out[t] = (int32_t)spin[p];
   if (seed) out[n + t] = seed[p];
+}
+
+template <typename T>
+__global__ void k_slice_pack(const T *__restrict__ spin, Geom g, SliceGeom s, uint32_t *__restrict__ planes) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < (int64_t)g.K * s.nw) slice_pack_word<T>(spin, g, s, (int)(q / s.nw), (uint32_t)(q % s.nw), planes);
+}
+
+template <typename T>
+__global__ void k_slice_unpack(const uint32_t *__restrict__ planes, Geom g, SliceGeom s, T *__restrict__ spin) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < (int64_t)g.K * s.nw) slice_unpack_word<T>(planes, g, s, (int)(q / s.nw), (uint32_t)(q % s.nw), spin);
+}
+
+__global__ void k_slice_seeds_in(const int32_t *__restrict__ seed, Geom g, SliceGeom s, int32_t *__restrict__ sseed) {
+  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x < g.K * s.seedc / 4) slice_seeds_in(seed, g, s, x, sseed);
+}
+
+__global__ void k_slice_seeds_out(const int32_t *__restrict__ sseed, Geom g, SliceGeom s, int32_t *__restrict__ seed) {
+  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x < g.K * s.seedc / 4) slice_seeds_out(sseed, g, s, x, seed);
+}
+
+// Canonical state into planes and seed shadow, and back (spin or seed null:
+// not that part).
+inline void slice_in(hipStream_t stream, const void *spin, int stype, const int32_t *seed, const Geom &g,
+                     const SliceGeom &s, uint32_t *planes, int32_t *sseed) {
+  const auto grid = [](int64_t n) { return dim3((unsigned)((n + 255) / 256)); };
+  if (spin)
+    with_type(stype, [&]<typename T>() {
+      hipLaunchKernelGGL((k_slice_pack<T>), grid((int64_t)g.K * s.nw), dim3(256), 0, stream,
+                         static_cast<const T *>(spin), g, s, planes);
+    });
+  if (seed) hipLaunchKernelGGL(k_slice_seeds_in, grid(g.K * s.seedc / 4), dim3(256), 0, stream, seed, g, s, sseed);
+}
+inline void slice_out(hipStream_t stream, const uint32_t *planes, const int32_t *sseed, const Geom &g,
+                      const SliceGeom &s, void *spin, int stype, int32_t *seed) {
+  const auto grid = [](int64_t n) { return dim3((unsigned)((n + 255) / 256)); };
+  with_type(stype, [&]<typename T>() {
+    hipLaunchKernelGGL((k_slice_unpack<T>), grid((int64_t)g.K * s.nw), dim3(256), 0, stream, planes, g, s,
+                       static_cast<T *>(spin));
+  });
+  hipLaunchKernelGGL(k_slice_seeds_out, grid(g.K * s.seedc / 4), dim3(256), 0, stream, sseed, g, s, seed);
 }
 
 // Compacts accumulator rows: out[2r], out[2r+1] = the sums of row r's

@@ -159,32 +159,10 @@ __global__ __launch_bounds__(kSliceThreads) void k_sweep_slice(uint32_t *__restr
   __shared__ SliceLds L[kSliceThreads / 64];
   const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t v = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * (kSliceThreads / 64) + wid;
-  Counts cnt{0, 0};
-  if (v < (uint32_t)s.waves)
-    cnt = slice_counts(slice_wave<FULL, PG>(planes, sseed, g, s, r, L[wid], m, v, threadIdx.x & 63));
+  SliceCounts n;
+  if (v < (uint32_t)s.waves) slice_wave<FULL, PG>(planes, sseed, g, s, r, L[wid], m, v, threadIdx.x & 63, n);
+  const Counts cnt = slice_counts(n);
   block_accumulate(cnt.nacc, cnt.de, acc, blockIdx.x & (kAccSlots - 1));
-}
-
-template <typename T>
-__global__ void k_slice_pack(const T *__restrict__ spin, Geom g, SliceGeom s, uint32_t *__restrict__ planes) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < (int64_t)g.K * s.nw) slice_pack_word<T>(spin, g, s, (int)(q / s.nw), (uint32_t)(q % s.nw), planes);
-}
-
-template <typename T>
-__global__ void k_slice_unpack(const uint32_t *__restrict__ planes, Geom g, SliceGeom s, T *__restrict__ spin) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < (int64_t)g.K * s.nw) slice_unpack_word<T>(planes, g, s, (int)(q / s.nw), (uint32_t)(q % s.nw), spin);
-}
-
-__global__ void k_slice_seeds_in(const int32_t *__restrict__ seed, Geom g, SliceGeom s, int32_t *__restrict__ sseed) {
-  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x < g.K * s.seedc / 4) slice_seeds_in(seed, g, s, x, sseed);
-}
-
-__global__ void k_slice_seeds_out(const int32_t *__restrict__ sseed, Geom g, SliceGeom s, int32_t *__restrict__ seed) {
-  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x < g.K * s.seedc / 4) slice_seeds_out(sseed, g, s, x, seed);
 }
 
 // Several colour passes in one launch (spk_tile.h): workgroup t loads box t
@@ -712,12 +690,7 @@ int slice_enter(spk_hip_lattice *h) {
     return set_error(SPK_HIP_ENOMEM, "bit planes not available");
   }
   if ((rc = ensure_shadow(h, h->sseed, h->sseed_cap, h->g.K * h->sg.seedc))) return rc;
-  with_type(h->stype, [&]<typename T>() {
-    hipLaunchKernelGGL((k_slice_pack<T>), dim3(grid_for(words, 256)), dim3(256), 0, h->stream,
-                       static_cast<const T *>(h->spin), h->g, h->sg, h->bits);
-  });
-  hipLaunchKernelGGL(k_slice_seeds_in, dim3(grid_for(h->g.K * h->sg.seedc / 4, 256)), dim3(256), 0, h->stream, h->seed,
-                     h->g, h->sg, h->sseed);
+  slice_in(h->stream, h->spin, h->stype, h->seed, h->g, h->sg, h->bits, h->sseed);
   rc = check_hip(hipGetLastError(), "bit-plane pack");
   if (!rc) h->slice_active = true;
   return rc;
@@ -725,13 +698,7 @@ int slice_enter(spk_hip_lattice *h) {
 
 int slice_leave(spk_hip_lattice *h) {
   h->slice_active = false;
-  const int64_t words = (int64_t)h->g.K * h->sg.nw;
-  with_type(h->stype, [&]<typename T>() {
-    hipLaunchKernelGGL((k_slice_unpack<T>), dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->bits, h->g, h->sg,
-                       static_cast<T *>(h->spin));
-  });
-  hipLaunchKernelGGL(k_slice_seeds_out, dim3(grid_for(h->g.K * h->sg.seedc / 4, 256)), dim3(256), 0, h->stream,
-                     h->sseed, h->g, h->sg, h->seed);
+  slice_out(h->stream, h->bits, h->sseed, h->g, h->sg, h->spin, h->stype, h->seed);
   return check_hip(hipGetLastError(), "bit-plane unpack");
 }
 

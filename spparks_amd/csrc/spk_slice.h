@@ -87,7 +87,7 @@ __host__ __device__ inline bool slice_fits(const Geom &g, int q) {
 
 // f.template operator()<PG>() for a lattice's plane groups
 template <typename F>
-void with_plane_groups(int pg, F &&f) {
+__host__ __device__ __forceinline__ void with_plane_groups(int pg, F &&f) {
   static_assert(kSliceMaxPlanes == 20, "1..5 groups");
   switch (pg) {
     case 1: f.template operator()<1>(); break;
@@ -196,6 +196,32 @@ __host__ __device__ __forceinline__ void slice_seeds_out(const int32_t *__restri
 #pragma unroll
   for (int k = 0; k < 4; k++)
     if (k < n) seed[home + k] = (int32_t)o.w[k];
+}
+
+// Spin of the site at (i, j, k), and the place of its seed in the shadow.
+struct SliceSite {
+  int c, i;          // colour, and site within its word
+  uint32_t row, w;   // its word
+};
+__host__ __device__ __forceinline__ SliceSite slice_site(const Geom &g, const SliceGeom &s, int i, int j, int k) {
+  const int a = i >> 1, w = a / s.W;
+  return SliceSite{(i & 1) | (j & 1) << 1 | (k & 1) << 2, a - w * s.W, (uint32_t)((j >> 1) + g.hy * (k >> 1)),
+                   (uint32_t)w};
+}
+__host__ __device__ __forceinline__ int32_t slice_spin_at(const uint32_t *__restrict__ planes, const SliceGeom &s,
+                                                          const SliceSite &x) {
+  const Words<4> *p = reinterpret_cast<const Words<4> *>(planes) + (int64_t)x.c * s.PG * s.nw + x.row * s.pw + x.w;
+  uint32_t v = 0;
+  for (int t = 0; t < s.PG; t++) {
+    const Words<4> y = p[(int64_t)t * s.nw];
+#pragma unroll
+    for (int b = 0; b < 4; b++) v |= ((y.w[b] >> x.i) & 1u) << (4 * t + b);
+  }
+  return (int32_t)v + 1;
+}
+__host__ __device__ __forceinline__ int64_t slice_seed_slot(const SliceGeom &s, const SliceSite &x) {
+  const uint32_t v = x.row / (uint32_t)s.rw, l = 16u * (uint32_t)(x.i >> 3) + (x.row - v * (uint32_t)s.rw) * s.pw + x.w;
+  return (int64_t)x.c * s.seedc + (((int64_t)v * 2 + ((x.i >> 2) & 1)) * 64 + l) * 4 + (x.i & 3);
 }
 
 // -------------------------------------------------------------- primitives
@@ -581,11 +607,12 @@ struct SliceLds {
   int32_t thr[64];
 };
 
-// Colours 2m and 2m+1 of wavefront v's rows.  Returns the lane's changes.  PG: s.PG.
+// Colours 2m and 2m+1 of wavefront v's rows; the lane's changes are added to
+// cnt.  PG: s.PG.
 template <bool FULL, int PG>
-__device__ __forceinline__ SliceCounts slice_wave(uint32_t *__restrict__ planes, int32_t *__restrict__ sseed,
-                                                  const Geom &g, const SliceGeom &s, const Rule &r, SliceLds &L, int m,
-                                                  uint32_t v, uint32_t l) {
+__device__ __forceinline__ void slice_wave(uint32_t *__restrict__ planes, int32_t *__restrict__ sseed, const Geom &g,
+                                           const SliceGeom &s, const Rule &r, SliceLds &L, int m, uint32_t v,
+                                           uint32_t l, SliceCounts &cnt) {
   const uint32_t q2 = 2u * (uint32_t)r.nspins, limit = r.zero_t ? 255u : 104u;
   const int32_t threshold = slice_threshold(r, min((int)l, kSliceThr - 1));
   const SliceLane t = slice_lane(g, s, m, v, l);
@@ -673,7 +700,6 @@ __device__ __forceinline__ SliceCounts slice_wave(uint32_t *__restrict__ planes,
 #pragma unroll
   for (int i = 0; i < PG; i++)
     slice_own_first<FULL>(t, own[0][i], own[1][i], lane_word(own[1][i], t.prev), L.w[2][slot][i].w[t.q], c0);
-  SliceCounts cnt;
   auto decide = [&](int c, SliceColour &col) {
     slice_join(col);
     uint32_t d[5], sum[6];
@@ -706,7 +732,6 @@ __device__ __forceinline__ SliceCounts slice_wave(uint32_t *__restrict__ planes,
 #pragma unroll
     for (int i = 0; i < PG; i++) store_own(1, i, bop3<kSel>(ch, L.w[3][slot][i].w[t.q], own[1][i]));
   }
-  return cnt;
 }
 #endif
 

@@ -154,6 +154,11 @@ static int run(int app, const int *n, int q, double kt, int nsw, const char *in,
   for (long long t = 0; t < N; t++) {
     const long long p = blocked_index(g, t % n[0], (t / n[0]) % n[1], t / ((long long)n[0] * n[1]));
     sn[t] = sp[p], kn[t] = sd[p];
+    const SliceSite x = slice_site(g, s, t % n[0], (t / n[0]) % n[1], t / ((long long)n[0] * n[1]));
+    if (slice_spin_at(planes.data(), s, x) != sn[t] || sseed.at(slice_seed_slot(s, x)) != kn[t]) {
+      fprintf(stderr, "site %lld read in place differs\n", t);
+      return 8;
+    }
   }
   f = fopen(out, "wb");
   if (!f) return 6;
