@@ -476,11 +476,9 @@ int replica_checksum_async(spk_hip_batch *b, int id) {
   }
   unsigned long long *out = b->d_slot + 4 * (size_t)id + 2;
   hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, b->stream, out, (int64_t)1);
-  const int64_t n = (int64_t)R.g.M * R.g.K;
   with_type(R.stype, [&]<typename T>() {
-    hipLaunchKernelGGL((k_checksum<T>), dim3(grid_for(n, 256)), dim3(256), 0, b->stream,
-                       reinterpret_cast<const T *>(b->pool + R.spin_off),
-                       reinterpret_cast<const int32_t *>(b->pool + R.seed_off), R.g, out);
+    launch_checksum<T>(b->stream, b->pool + R.spin_off, reinterpret_cast<const int32_t *>(b->pool + R.seed_off), R.g,
+                       out);
   });
   int rc = check_hip(hipGetLastError(), "checksum launch");
   if (!rc)

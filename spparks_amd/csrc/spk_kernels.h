@@ -3,6 +3,8 @@
 // state.  Each translation unit gets its own copies (anonymous namespace).
 #pragma once
 
+#include <algorithm>
+
 #include "spk_device.h"
 #include "spk_host.h"
 #include "spk_slice.h"
@@ -32,6 +34,13 @@ __global__ __launch_bounds__(256) void k_energy(const T *__restrict__ spin, Geom
 }
 
 __device__ __forceinline__ void natural_ijk(const Geom &g, int64_t t, int &i, int &j, int &k) {
+  if ((uint64_t)t >> 32 == 0) {   // divisions of half the width, a third of the instructions
+    const uint32_t r = (uint32_t)t / (uint32_t)g.nx;
+    i = (int)((uint32_t)t - r * (uint32_t)g.nx);
+    k = (int)(r / (uint32_t)g.ny);
+    j = (int)(r - (uint32_t)k * (uint32_t)g.ny);
+    return;
+  }
   i = (int)(t % g.nx);
   const int64_t r = t / g.nx;
   j = (int)(r % g.ny);
@@ -203,20 +212,36 @@ __host__ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
+// One atomic a workgroup, and at most kChecksumGrid of them: they all meet at
+// one address, and one a wavefront (107 000 of them) made 6.9M sites take 956 us,
+// 31 us this way (and 64^3 15).
+constexpr unsigned kChecksumGrid = 1024;
+
 template <typename T>
-__global__ void k_checksum(const T *__restrict__ spin, const int32_t *__restrict__ seed, Geom g,
-                           unsigned long long *__restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_checksum(const T *__restrict__ spin, const int32_t *__restrict__ seed, Geom g,
+                                                  unsigned long long *__restrict__ out) {
+  __shared__ uint64_t part[4];
+  const int64_t n = (int64_t)g.M * g.K;
   uint64_t h = 0;
-  if (t < (int64_t)g.M * g.K) {
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
     int i, j, k;
     natural_ijk(g, t, i, j, k);
     const int64_t p = blocked_index(g, i, j, k);
-    h = mix64((uint64_t)t * 0xD1B54A32D192ED03ull + (uint64_t)(uint32_t)(int32_t)spin[p] * 0xABC98388FB8FAC03ull +
-              (uint64_t)(uint32_t)seed[p]);
+    h += mix64((uint64_t)t * 0xD1B54A32D192ED03ull + (uint64_t)(uint32_t)(int32_t)spin[p] * 0xABC98388FB8FAC03ull +
+               (uint64_t)(uint32_t)seed[p]);
   }
   h = wave_sum64(h);
-  if ((threadIdx.x & 63) == 0) atomicAdd(out, (unsigned long long)h);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = h;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(out, (unsigned long long)(part[0] + part[1] + part[2] + part[3]));
+}
+
+template <typename T>
+void launch_checksum(hipStream_t stream, const void *spin, const int32_t *seed, const Geom &g,
+                     unsigned long long *out) {
+  const int64_t wg = ((int64_t)g.M * g.K + 255) / 256;
+  hipLaunchKernelGGL((k_checksum<T>), dim3((unsigned)std::min<int64_t>(wg, kChecksumGrid)), dim3(256), 0, stream,
+                     static_cast<const T *>(spin), seed, g, out);
 }
 
 }  // namespace

@@ -1423,8 +1423,7 @@ int spk_hip_checksum(spk_hip_lattice *h, uint64_t *sum) {
   if ((rc = bits_leave(h)) || (rc = ensure_acc(h, 1))) return rc;
   if ((rc = check_hip(hipMemsetAsync(h->acc, 0, sizeof(unsigned long long), h->stream), "memset"))) return rc;
   with_type(h->stype, [&]<typename T>() {
-    hipLaunchKernelGGL((k_checksum<T>), dim3(grid_for(h->N, 256)), dim3(256), 0, h->stream,
-                       static_cast<const T *>(h->spin), h->seed, h->g, h->acc);
+    launch_checksum<T>(h->stream, h->spin, h->seed, h->g, h->acc);
   });
   if ((rc = check_hip(hipGetLastError(), "checksum launch"))) return rc;
   if ((rc = check_hip(hipMemcpyAsync(h->pinned, h->acc, sizeof(*h->pinned), hipMemcpyDeviceToHost, h->stream),
