@@ -24,6 +24,30 @@ double now_s(std::chrono::steady_clock::time_point t0) {
   return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
+// The pool a queue of solves can fill: pool_bytes, or the extents of all of
+// its requests if they are fewer bytes.  (Every request takes one extent once,
+// so such a pool never refuses one that a larger pool takes.)  The device's
+// memory is cleared as it is given back, at 45 GB/s here: a pool of 16 GiB for
+// 0.35 GiB of solves, taken and given back by each call, made calls of 0.10 s wait
+// 0.38 s for it once the cleared memory of the card was used up.  A pool_bytes
+// that the device does not have is refused as before.
+int queue_pool(const spk_hip_request *req, int n, int64_t pool_bytes, int64_t *out) {
+  int64_t sum = 0;
+  for (int i = 0; i < n && sum < pool_bytes; i++) {
+    int64_t b = 0;
+    if (spk_hip_replica_bytes(&req[i].replica.lattice, &b) == SPK_HIP_OK) sum += b;   // the others are refused alone
+  }
+  *out = pool_bytes;
+  if (pool_bytes <= 0 || sum >= pool_bytes) return SPK_HIP_OK;
+  size_t free_bytes = 0, total = 0;
+  const int rc = check_hip(hipMemGetInfo(&free_bytes, &total), "hipMemGetInfo");
+  if (rc) return rc;
+  if ((uint64_t)pool_bytes > free_bytes)
+    return set_error(SPK_HIP_ENOMEM, "device pool of %lld bytes not available", (long long)pool_bytes);
+  *out = std::max<int64_t>(sum, 256);
+  return SPK_HIP_OK;
+}
+
 struct BatchGuard {
   spk_hip_batch *b = nullptr;
   ~BatchGuard() { spk_hip_batch_destroy(b); }
@@ -39,8 +63,8 @@ extern "C" int spk_hip_serve(const spk_hip_request *req, int n, int64_t pool_byt
     if (req[i].arrive < req[i - 1].arrive) return set_error(SPK_HIP_EINVAL, "requests not sorted by arrival");
   spk_hip_serve_stats st{};
   BatchGuard g;
-  int rc = spk_hip_batch_create(pool_bytes, max_live, &g.b);
-  if (rc) return rc;
+  int rc = queue_pool(req, n, pool_bytes, &pool_bytes);
+  if (rc || (rc = spk_hip_batch_create(pool_bytes, max_live, &g.b))) return rc;
   if ((rc = spk_hip_batch_set_launch(g.b, block, grid))) return rc;
   bool tuned = block != 0;   // a zero shape is tuned on the first block, which waits
 

@@ -85,3 +85,17 @@ def test_sliced_replica_takes_uploads_and_an_extent_again(orc):
         s, k = B.download(rid)
         assert np.array_equal(s, spin) and np.array_equal(k, seeds)
         assert B.status(rid)[3] == orc.energy(d, spin)
+
+
+def test_queue_takes_no_more_than_its_solves_and_refuses_what_the_device_lacks():
+    import spparks_amd as S
+    from spparks_amd import batch as bmod
+    reqs = [{"app": a, "lattice": l, "shape": s, "nspins": q, "kT": k, "seed": sd, "sweeps": n, "arrive": 0.0}
+            for a, l, s, q, k, sd, n in MIX[:4]]
+    small, _ = bmod.serve(reqs, pool_bytes=sum(bmod.replica_bytes(c[0], c[1], *c[2], c[3]) for c in MIX[:4]), max_live=4)
+    large, st = bmod.serve(reqs, pool_bytes=1 << 30, max_live=4)
+    assert st["max_live"] == 4
+    for a, b in zip(small, large):
+        assert a["status"] == b["status"] == 0 and a["checksum"] == b["checksum"] and a["energy"] == b["energy"]
+    with pytest.raises(S.HipError, match="not available"):
+        bmod.serve(reqs, pool_bytes=1 << 44, max_live=4)
