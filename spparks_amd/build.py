@@ -89,7 +89,7 @@ def build_emulator():
     AddressSanitizer for the CPU tests.  Test infrastructure."""
     emul = os.path.join(ROOT, "tests", "emul")
     outs = []
-    for name in ("spk_emul", "spk_emul_tile", "spk_emul_slice", "spk_emul_pair"):
+    for name in ("spk_emul", "spk_emul_tile", "spk_emul_slice", "spk_emul_pair", "spk_emul_neigh"):
         src = os.path.join(emul, name + ".hip")
         if not os.path.exists(src):
             continue

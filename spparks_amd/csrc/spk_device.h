@@ -926,16 +926,36 @@ struct RawWords {
   Lanes<T> pk[NPACK];
 };
 
+// What a pack reads.
+template <int LAT, typename T, typename I>
+struct PackLoad {
+  I self;             // the pack's offset within its colour's sub-grid
+  int k;              // real lanes (hx - a0)
+  Lanes<T> old;
+  Words<4> sd;
+  RawWords<T, StencilWords<LAT>::NSEG, StencilWords<LAT>::NPACK> raw;
+
+  // segment m's pack shifted one site towards side `off`
+  __host__ __device__ __forceinline__ Lanes<T> beside(int m, int off, bool ragged) const {
+    Lanes<T> S = shifted<T>(raw.seg[m], raw.extra[m], off);
+    if (ragged) {
+      const RowEnd<T> rowend(off ? k : 5);   // only the +x side wraps inside a pack
+      rowend.apply(S, raw.extra[m]);
+    }
+    return S;
+  }
+};
+
 // XDIR: the side (0, 1) every segment shifts towards, when the caller knows
 // it for the whole launch (sq/8n and sc/26n: the colour's x parity); -1
 // takes each segment's own.
-template <int LAT, typename T, bool TWO, typename I, int XDIR = -1>
-__host__ __device__ __forceinline__ PackWork<T, TWO, I> pack_count(const T *__restrict__ spin,
-                                                                   const int32_t *__restrict__ seed,
-                                                                   const Geom &g, const Rule &r, int c, int a0,
-                                                                   int b, int e) {
+template <int LAT, typename T, typename I, int XDIR = -1>
+__host__ __device__ __forceinline__ PackLoad<LAT, T, I> pack_load(const T *__restrict__ spin,
+                                                                  const int32_t *__restrict__ seed, const Geom &g,
+                                                                  int c, int a0, int b, int e) {
   using SW = StencilWords<LAT>;
-  PackWork<T, TWO, I> w;
+  PackLoad<LAT, T, I> w;
+  auto &raw = w.raw;
   const I Mp = (I)g.Mp;
   // row offsets px*y + pxy*z; px*y as a 24-bit multiply (see RowOffset)
   const RowOffset<I> px((I)g.px);
@@ -948,7 +968,6 @@ __host__ __device__ __forceinline__ PackWork<T, TWO, I> pack_count(const T *__re
 
   // ---- load phase: the offsets of every word the pack needs first, then
   // every load, before any word is used: one memory round trip per pack
-  RawWords<T, SW::NSEG, SW::NPACK> raw;
   const T *sbase[SW::NSEG], *pbase[SW::NPACK];
   I srow[SW::NSEG], prow[SW::NPACK];
   int ns = 0, np = 0;
@@ -1001,7 +1020,7 @@ __host__ __device__ __forceinline__ PackWork<T, TWO, I> pack_count(const T *__re
       }
   }
   w.old = load_lanes<T, I>(colour(c), w.self);
-  const Words<4> sd = *reinterpret_cast<const Words<4> *>(elem<I>(elem<I>(seed, (I)c * Mp), w.self));
+  w.sd = *reinterpret_cast<const Words<4> *>(elem<I>(elem<I>(seed, (I)c * Mp), w.self));
 #pragma unroll
   for (int m = 0; m < SW::NSEG; m++) {
     raw.seg[m] = load_lanes<T, I>(sbase[m], srow[m] + (I)a0);
@@ -1011,24 +1030,34 @@ __host__ __device__ __forceinline__ PackWork<T, TWO, I> pack_count(const T *__re
 #pragma unroll
   for (int m = 0; m < SW::NPACK; m++) raw.pk[m] = load_lanes<T, I>(pbase[m], prow[m] + (I)a0);
   fence_schedule();   // no counting work may be scheduled between the loads
+  return w;
+}
+
+template <int LAT, typename T, bool TWO, typename I, int XDIR = -1>
+__host__ __device__ __forceinline__ PackWork<T, TWO, I> pack_count(const T *__restrict__ spin,
+                                                                   const int32_t *__restrict__ seed,
+                                                                   const Geom &g, const Rule &r, int c, int a0,
+                                                                   int b, int e) {
+  using SW = StencilWords<LAT>;
+  const PackLoad<LAT, T, I> ld = pack_load<LAT, T, I, XDIR>(spin, seed, g, c, a0, b, e);
+  const auto &raw = ld.raw;
+  PackWork<T, TWO, I> w;
+  w.self = ld.self;
+  w.k = ld.k;
+  w.old = ld.old;
 
   // ---- count phase: first draws and proposals, then every word compared
   // with the old and the proposed lanes
 #pragma unroll
   for (int v = 0; v < 4; v++) {
-    w.s[v] = pm_step((int32_t)sd.w[v]);
+    w.s[v] = pm_step((int32_t)ld.sd.w[v]);
     w.pr[v] = propose_as<TWO>(r, w.s[v]);
   }
   const Lanes<T> prop = Lanes<T>::pack(w.pr);
   const bool ragged = (g.hx & 3) != 0;   // same for the whole launch
   // segment m: its pack and the pack shifted one site towards side `off`
   auto segment = [&](int m, int off) {
-    Lanes<T> S = shifted<T>(raw.seg[m], raw.extra[m], off);
-    if (ragged) {
-      const RowEnd<T> rowend(off ? w.k : 5);   // only the +x side wraps inside a pack
-      rowend.apply(S, raw.extra[m]);
-    }
-    w.tally.add2(raw.seg[m], S, w.old, prop);
+    w.tally.add2(raw.seg[m], ld.beside(m, off, ragged), w.old, prop);
   };
 #pragma unroll
   for (int m = 0; m < SW::NSEG; m++) segment(m, XDIR >= 0 ? XDIR : raw.off[m]);

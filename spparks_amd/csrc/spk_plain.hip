@@ -19,6 +19,7 @@
 #include "spk_host.h"
 #include "spk_kernels.h"
 #include "spk_pair.h"
+#include "spk_neigh.h"
 #include "spk_slice.h"
 #include "spk_tile.h"
 
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(1024) void k_sweep_tile(const T *__restrict__ spin_
 // One colour pass of a proposal variant (potts/neigh, potts/neighonly,
 // ising/single): one slot per thread (4 consecutive slots per pack, so a
 // wavefront's own-site accesses stay unit-stride), neighbours read in the
-// reference's order.
+// reference's order.  The lattices that k_sweep_neigh does not take.
 template <int LAT, typename T, int APP>
 __global__ __launch_bounds__(1024) void k_sweep_variant(T *__restrict__ spin, int32_t *__restrict__ seed, Geom g,
                                                         Rule r, int color, unsigned long long *__restrict__ acc) {
@@ -264,6 +265,25 @@ __global__ __launch_bounds__(1024) void k_sweep_variant(T *__restrict__ spin, in
   const int64_t t = (int64_t)tile * blockDim.x + threadIdx.x;
   Counts cnt{0, 0};
   if (t < (int64_t)g.Mp) cnt = variant_site<LAT, T, APP>(spin, seed, g, r, s_thr, color, (uint32_t)t);
+  block_accumulate_pack(cnt.nacc, cnt.de, acc, blockIdx.x & (kAccSlots - 1));
+}
+
+// The same for potts/neigh and potts/neighonly in halfwords (spk_neigh.h),
+// four sites a thread.  VALU bound: 2010 instructions a wavefront of 256 sites
+// at sc/26n against 854 for 64, 8 wavefronts a SIMD at 256^3.  us a sweep there,
+// Q = 10^4 and 100: k_sweep_variant 390, 390, this kernel 247, 245; sq/8n at
+// 2048^2 37.6, 28.0.
+template <int LAT, typename T, int APP, typename I, int XD>
+__global__ __launch_bounds__(1024) void k_sweep_neigh(T *__restrict__ spin, int32_t *__restrict__ seed, Geom g, Rule r,
+                                                      TileMap m, int color, unsigned long long *__restrict__ acc) {
+  __shared__ int s_thr[32];
+  if (threadIdx.x < 28) s_thr[threadIdx.x] = r.thr[threadIdx.x];
+  __syncthreads();
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  int a0, b, e;
+  Counts cnt{0, 0};
+  if (tile < m.nxc * m.nyg * m.nzg && tile_site(g, m, (uint32_t)tile, threadIdx.x, a0, b, e))
+    cnt = neigh_pack<LAT, T, APP, I, XD>(spin, seed, g, r, s_thr, color, a0, b, e);
   block_accumulate_pack(cnt.nacc, cnt.de, acc, blockIdx.x & (kAccSlots - 1));
 }
 
@@ -368,7 +388,49 @@ void allow_lds(K kern, size_t lds) {
 
 unsigned grid_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
+// Lattices that k_sweep_neigh takes: row segments of one x side, and values of
+// at most 15 bits.  On sq/8n, whose 28 pairs are soon compared, a quarter of the
+// wavefronts pays from more than 2^18 sites a colour on; us a sweep, one
+// site a thread and this way: 512^2 13.4, 15.1; 1024^2 16.4, 15.4 (18.1 in workgroups of
+// 512); 1280^2 22.6, 18.9; 1600^2 25.9, 22.4; 2048^2 35.2, 26.3.  On sc/26n at
+// every size: 32^3 59.7, 54.9; 64^3 56.1, 55.0; 96^3 59.5, 57.3; 128^3 73.3, 56.6.
+bool neigh_packed(const spk_hip_lattice *h) {
+  return (h->d.app == SPK_HIP_POTTS_NEIGH || h->d.app == SPK_HIP_POTTS_NEIGHONLY) &&
+         (h->g.lat == SPK_HIP_SC_26N || (h->g.lat == SPK_HIP_SQ_8N && h->g.Mp > (1 << 18))) && h->stype != kI32 &&
+         h->rule.nspins <= kNeighMaxQ;
+}
+
+// (workgroups of 256 unless the caller chose: 22.4 us a sweep of sq/8n at 1600^2
+// against 25.0 with the other kernels' 512)
+int launch_neigh(spk_hip_lattice *h, int color, unsigned long long *acc) {
+  const int bs = h->block_set ? h->block : 256;
+  const TileMap m = make_tile_map(h->g, bs);
+  unsigned grid = (unsigned)m.nxc * m.nyg * m.nzg;
+  grid = (grid + kNumXcd - 1) / kNumXcd * kNumXcd;   // xcd_tile needs a multiple of 8
+  const bool off32 = offsets_fit_32(h->g);
+  with_lattice(h->g.lat, [&]<int LAT>() {
+    with_type(h->stype, [&]<typename T>() {
+      if constexpr ((LAT == SPK_HIP_SQ_8N || LAT == SPK_HIP_SC_26N) && sizeof(T) <= 2) {
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(grid), dim3(bs), 0, h->stream, static_cast<T *>(h->spin), h->seed, h->g,
+                             h->rule, m, color, acc);
+        };
+        auto with_x = [&]<int APP, typename I>() {
+          color & 1 ? go(k_sweep_neigh<LAT, T, APP, I, 1>) : go(k_sweep_neigh<LAT, T, APP, I, 0>);
+        };
+        auto with_app = [&]<int APP>() {
+          off32 ? with_x.template operator()<APP, uint32_t>() : with_x.template operator()<APP, int64_t>();
+        };
+        if (h->d.app == SPK_HIP_POTTS_NEIGH) with_app.template operator()<SPK_HIP_POTTS_NEIGH>();
+        else with_app.template operator()<SPK_HIP_POTTS_NEIGHONLY>();
+      }
+    });
+  });
+  return check_hip(hipGetLastError(), "sweep kernel launch");
+}
+
 int launch_variant(spk_hip_lattice *h, int color, unsigned long long *acc) {
+  if (neigh_packed(h)) return launch_neigh(h, color, acc);
   const int bs = h->block;
   unsigned grid = grid_for(h->g.Mp, bs);
   grid = (grid + kNumXcd - 1) / kNumXcd * kNumXcd;   // xcd_tile needs a multiple of 8
@@ -520,6 +582,11 @@ double plain_sweep_us(const spk_hip_lattice *h) {
     // to 78 at 256^3)
     const SliceGeom sg = slice_geom(h->g, h->rule.nspins);
     return h->g.K / 2 * (4.6 + 0.55 * sg.PG + sg.waves / 4096.0 * (3.4 + 1.75 * sg.PG));
+  }
+  if (neigh_packed(h)) {   // 6.9-7.1 us a pass of sc/26n up to 128^3, 10.9 at 160^3, 31 at 256^3
+    const int nn = maxneigh_of(h->g.lat);
+    const double us = (260 + 30 * nn + 1.5 * nn * (nn - 1)) * kUsPerValu, waves = (double)h->g.Mp / 4 / 64;
+    return h->g.K * std::max(3.0 + 1.2 * us, 2.6 + 1.06 * waves / (kCus * kSimds) * us);
   }
   if (variant_app(h->d.app)) {
     const double us = tile_site_valu(h) * kUsPerValu, waves = (double)h->g.Mp / 64;
