@@ -71,6 +71,18 @@ def bytes_per_update(lattice, sbytes):
     return NCOLORS[lattice] * sbytes + 8 + sbytes
 
 
+def plane_groups(q):
+    """Groups of four bit planes that hold spins 1..q."""
+    return -(-max(1, (q - 1).bit_length()) // 4)
+
+
+def sliced_bytes_per_update(q):
+    """The same of the bit-sliced sc/26n pass: a launch reads and writes the
+    seeds of two of the eight colours, reads the planes of the whole lattice (in
+    groups of four: half a byte a site each) and writes two colours'."""
+    return 8 + 0.5 * plane_groups(q) * (1 + 2 / 8) / (2 / 8)
+
+
 def load_traffic(workload):
     """rocprofv3-measured HBM traffic of the workload's dominant kernel:
     (bytes per launch or None, the measurement's details or None)."""
@@ -214,7 +226,10 @@ def run_ensemble(args):
 
     value = updates / wall_b / 1e9
     plain = updates / wall_p / 1e9 if wall_p > 0 else None
-    bytes_alg = sum(n * nsw * bytes_per_update(r["lattice"], spin_bytes(r["app"], r["nspins"]))
+    # (the ensemble's sc/26n replicas all fill their words enough to sweep on
+    # bit planes; words that are not full are not counted)
+    bytes_alg = sum(n * nsw * (sliced_bytes_per_update(r["nspins"]) if r["lattice"] == "sc/26n" else
+                               bytes_per_update(r["lattice"], spin_bytes(r["app"], r["nspins"])))
                     for n, r in zip(sites, reps))
     achieved = bytes_alg / (dev_ms / 1e3) / 1e9
     return {
@@ -236,7 +251,7 @@ def run_ensemble(args):
                    "compared": "final spins+seeds hash, Naccept, energy: batched vs plain"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": load_traffic("ensemble-512")[0],
-                     "kernel": "k_batch_step (all variants of the block)",
+                     "kernel": "k_batch_slice (sc/26n on bit planes) and k_batch_step (sq/4n)",
                      "device_ms": round(dev_ms, 3), "step_launches": nl},
         "cpu_baseline": None,
     }
@@ -375,18 +390,20 @@ def run(args):
     variant = app in VARIANTS and not planes and not boxes
     launches = None   # (two-sweep launches, per-colour launches) of a call on paired planes
     if variant:
-        # one site per thread, neighbours gathered in the reference's order;
-        # the same bytes as the per-colour design
-        kernel = "k_sweep_variant<%s, %s, %s>" % (lattice, tname, app)
+        # neighbours in the reference's order, four sites a thread where the
+        # library's rule packs them and one elsewhere; the same bytes as the
+        # per-colour design
+        packed = (app != "ising/single" and sb <= 2 and q < 32768
+                  and (lattice == "sc/26n" or (lattice == "sq/8n" and n > 4 << 18)))
+        kernel = "k_sweep_%s<%s, %s, %s>" % ("neigh" if packed else "variant", lattice, tname, app)
         bytes_per_launch = B * n // K
         B_kernel = B
     elif sliced:
         # a launch reads and writes the seeds of two colours, reads the planes
         # of the whole lattice (held in groups of four) and writes two colours'
-        groups = -(-max(1, (q - 1).bit_length()) // 4)
-        kernel = "k_sweep_slice<%d plane groups> (bit planes, two colours per launch)" % groups
-        bytes_per_launch = int(n * (2 * 8 / K + 0.5 * groups * (1 + 2 / K)))
-        B_kernel = bytes_per_launch / (n * 2 / K)
+        kernel = "k_sweep_slice<%d plane groups> (bit planes, two colours per launch)" % plane_groups(q)
+        B_kernel = sliced_bytes_per_update(q)
+        bytes_per_launch = int(B_kernel * n * 2 / K)
     elif boxes:
         # the state crosses HBM once each way per launch (halos come on top);
         # the kernel is bound by the time of its passes in LDS

@@ -222,10 +222,13 @@ int spk_hip_last_timing(spk_hip_lattice *h, double *ms, int64_t *nlaunch);
 /* ======================================================================
    Batched replicas: many independent lattices (each its own script: app,
    lattice, size, Q, kT, seed, sweep count) resident in one device pool and
-   advanced together.  Each colour step of a block is one persistent kernel
-   over a tile work-list spanning every replica that is due a colour pass
-   at that step; a replica's K*n passes of an n-sweep block are spread evenly
-   over the block's steps, always in colour order 1..K.  Every replica's
+   advanced together.  Each step of a block is one kernel per kind of replica
+   over a tile work-list spanning every replica of the kind that is due a pass
+   at that step; a replica's K*n passes of an n-sweep block (K/2*n of two colours
+   where it sweeps on bit planes: sc/26n rows that fill at least half of 32-bit
+   words) are spread evenly over the kind's steps, always in colour order 1..K.
+   Planes are held beside the pool, in memory taken while a quarter of the
+   device's stays free; a replica without them sweeps its spins.  Every replica's
    trajectory is identical to running it alone (the strict sweep is
    decomposition independent), which the tests check.  Blocks after the
    first are replayed as HIP graphs.  No counterpart in the reference, which
@@ -273,7 +276,8 @@ int spk_hip_batch_status(spk_hip_batch *b, int id, int *done, int *left, int64_t
 /* Cumulative Naccept and energy after each of the first n sweeps. */
 int spk_hip_batch_trace(spk_hip_batch *b, int id, int n, int64_t *naccept, double *energy);
 
-/* Launch shape of the step kernel: block = threads per tile (64..1024,
+/* Launch shape of the step kernels of replicas that are not on bit planes (those
+   have a wavefront for every tile): block = threads per workgroup (64..1024,
    multiple of 64), grid = persistent workgroups.  0, 0 = autotune: the next
    run times candidate shapes on its own steps (results do not depend on the
    shape) and keeps the fastest. */

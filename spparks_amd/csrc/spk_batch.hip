@@ -1,7 +1,8 @@
 // spk_batch.hip -- libspk_hip.so, batched replicas: a device pool holding many
-// independent lattices, one persistent kernel per colour step over a tile
-// work-list spanning all replicas due a pass at that step, HIP-graph replay of
-// blocks, and an autotuner for the launch shape.  ABI in include/spk_hip.h.
+// independent lattices, one kernel per step and kind of replica over a tile
+// work-list spanning all replicas due a pass at that step (a colour, or two of
+// them on bit planes), HIP-graph replay of blocks, and an autotuner for the
+// launch shape.  ABI in include/spk_hip.h.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -386,11 +387,12 @@ struct spk_hip_batch {
   int inflight_rows = 0;
   unsigned long long *h_rows = nullptr;   // pinned: folded rows of the block in flight
   int cap_h_rows = 0;
-  // per replica slot: an energy accumulator row, the folded initial energy
-  // and the checksum, copied to pinned memory in stream order
+  // per replica slot: an energy accumulator row, the checksum, and in pinned
+  // memory the initial energy (written there by the fold) and the checksum
+  // (copied), both in stream order
   unsigned long long *d_erow = nullptr;   // [slots][kAccRow]
-  unsigned long long *d_slot = nullptr;   // [slots][4]: energy, (unused), checksum, (unused)
-  unsigned long long *h_slot = nullptr;   // pinned copy of d_slot
+  unsigned long long *d_slot = nullptr;   // [slots][4]: word 2 the checksum
+  unsigned long long *h_slot = nullptr;   // pinned, [slots][4]: energy, its fold's second word, checksum
 };
 
 namespace {

@@ -174,10 +174,10 @@ __global__ __launch_bounds__(kSliceThreads) void k_sweep_slice(uint32_t *__restr
 // compare, decide, barrier: 0.8-1 us for 32 passes of 128^2 sq/8n, VALU busy
 // 38%); large ones, the VALU (54% busy on 1500 x 1002 sq/8n, with 14% of the
 // events in the halo).  us a sweep, before and now:
-//   sq/4n Ising 256^2 10.2, 2.9; 1000^2 10.8, 4.8; 1500^2 11.5, 7.7
+//   sq/4n Ising 256^2 10.2, 2.9 (1000^2 10.8, 4.8, but 4.1 in k_sweep_bits_pair)
 //   sq/8n Potts 128^2 Q=100 9.2, 4.4 (one workgroup before)
 //   sq/8n Potts 1500 x 1002 Q=100 15.1, 9.5
-//   sc/26n Potts 32^3 Q=1000 33.6, 12.8; 64^3 Q=10^5 37.6, 15.5; 100^3 35.4, 26.3
+//   sc/26n Potts 32^3 Q=1000 33.6, 12.8; 64^3 Q=10^5 37.6, 15.5
 // One site a thread (VEC 1) against packs of 4: 16.2 against 24.1 on 64^3
 // sc/26n, 4.4 against 5.6 on 128^2 sq/8n, but 11.2 against 9.5 on 1500 x 1002,
 // where the VALU counts.
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(1024) void k_sweep_variant(T *__restrict__ spin, in
 }
 
 // The same for potts/neigh and potts/neighonly in halfwords (spk_neigh.h),
-// four sites a thread.  VALU bound: 2010 instructions a wavefront of 256 sites
+// four sites a thread.  VALU bound: 1970 instructions a wavefront of 256 sites
 // at sc/26n against 854 for 64, 8 wavefronts a SIMD at 256^3.  us a sweep there,
 // Q = 10^4 and 100: k_sweep_variant 390, 390, this kernel 247, 245; sq/8n at
 // 2048^2 37.6, 28.0.
@@ -568,7 +568,7 @@ double pair_sweep_us(const spk_hip_lattice *h) {
 // over the lattice one colour at a time (bit planes where they apply) or in
 // one workgroup.  Short passes are latency: 3 us and a thread's own chain
 // (measured 3.5 us on sc/6n at 40^3, 4.2 on sc/26n at 32^3 to 100^3, 5.1-6.2
-// on bit planes at 256^2 to 2000^2, 7.0 for potts/neigh on sc/26n at 32^3).
+// on bit planes at 256^2 to 2000^2).
 double plain_sweep_us(const spk_hip_lattice *h) {
   if (resident_bytes(h)) {
     const double waves = std::ceil((double)h->g.Mp / 4 / 64);
