@@ -604,30 +604,42 @@ double tile_item_us(const spk_hip_lattice *h, int vec) {
 // Microseconds a sweep is expected to take in boxes of w sites, S sweeps a
 // launch, vec sites a thread: the launch with its loads and stores, then each
 // pass bound by the wavefronts a SIMD has of it or by one wavefront's own time.
-double tile_sweep_us(const spk_hip_lattice *h, const int (&w)[3], int S, int vec, TileShape *shape) {
-  TilePlan tp;
-  const int size = (int)spin_bytes(h->stype);
-  if (S * h->g.K > kTileMaxPass || !tile_plan_make(h->g, w, 0, S * h->g.K, vec, size, &tp)) return 1e30;
-  const size_t lds = tile_lds(tp);
+// us a sweep no better than `best` come back as 1e30.
+double tile_sweep_us(const spk_hip_lattice *h, const int (&w)[3], int S, int vec, const TileRegion &r, double best,
+                     TileShape *shape) {
+  const int size = (int)spin_bytes(h->stype), K = h->g.K;
+  Geom gl;
+  geom_init(gl, h->g.lat, r.ext[0], r.ext[1], r.ext[2]);
+  const int64_t slots = (int64_t)K * gl.Mp;
+  const size_t lds = (size_t)((slots * size + 15) / 16 * 16 + slots * 4);   // tile_lds of the plan
   if (lds > h->max_lds) return 1e30;
-  uint32_t most = 0;
-  for (int k = 0; k < tp.npass; k++) most = std::max(most, tp.pass[k].items);
-  const uint32_t packs = (uint32_t)tp.gl.K * (uint32_t)(tp.gl.Mp / 4);   // loaded and stored by every thread
+  uint32_t items[kTileMaxPass], most = 0;
+  for (int k = 0, c = 0; k < S * K; k++, c = c + 1 == K ? 0 : c + 1) {
+    const TileSpan t = tile_span(h->g.lat, r, k, c);
+    items[k] = tile_packs(t, vec) * (uint32_t)(t.b[1] - t.b[0]) * (uint32_t)(t.e[1] - t.e[0]);
+    most = std::max(most, items[k]);
+  }
+  const uint32_t packs = (uint32_t)(slots / 4);   // loaded and stored by every thread
   const int block = (int)std::min<uint32_t>(1024, (std::max(most, packs) + 63) / 64 * 64);
-  const int64_t tiles = (int64_t)tp.cx * tp.cy * tp.cz;
+  int64_t tiles = 1;
+  const int n[3] = {h->g.nx, h->g.ny, h->g.nz};
+  double own = 1;
+  for (int d = 0; d < 3; d++) tiles *= r.whole[d] ? 1 : (n[d] + w[d] - 1) / w[d], own *= r.whole[d] ? n[d] : w[d];
   const int per_cu = (int)((tiles + kCus - 1) / kCus);
   const int fit = std::max(1, std::min((int)((160 << 10) / (lds + 1024)), 16 * 64 / block));   // boxes a CU holds at once
   const int together = std::min(per_cu, fit), rounds = (per_cu + together - 1) / together;
   const double item_us = tile_item_us(h, vec);
-  double us = 0;
-  for (int k = 0; k < tp.npass; k++) {
-    const double waves = std::ceil(tp.pass[k].items / 64.0), turns = std::ceil(tp.pass[k].items / (double)block);
+  const double moved = (double)lds + own * (4 + size);   // bytes a box moves
+  double us = together * moved / 20e3;   // a CU's share of the memory rate, about 20 GB/s a us
+  const uint32_t threads = (uint32_t)block;
+  for (int k = 0; k < S * K; k++) {
+    const double waves = (items[k] + 63) / 64, turns = (items[k] + threads - 1) / threads;
     us += 0.3 + std::max(turns * (0.15 + 1.3 * item_us), 1.2 * together * waves / kSimds * item_us);
   }
-  const double moved = (double)lds + (double)tp.wx * tp.wy * tp.wz * (4 + size);   // bytes a box moves
-  us += together * moved / 20e3;   // a CU's share of the memory rate, about 20 GB/s a us
-  if (shape) *shape = TileShape{{w[0], w[1], w[2]}, S, vec, block};
-  return (5.0 + rounds * us) / S;
+  us = (5.0 + rounds * us) / S;
+  if (us >= best) return 1e30;
+  *shape = TileShape{{w[0], w[1], w[2]}, S, vec, block};
+  return us;
 }
 
 // Whether boxes of w sites fit LDS for launches that start at any colour
@@ -663,28 +675,38 @@ void tile_choose(spk_hip_lattice *h) {
     return v;
   };
   const std::vector<int> vx = sizes(h->g.nx, 8), vy = sizes(h->g.ny, 2), vz = sizes(h->g.nz, 2);
-  for (int S : {1, 2, 3, 4, 6, 8}) {
-    if (S * h->g.K > kTileMaxPass) break;
-    for (int wx : vx)
-      for (int wy : vy)
-        for (int wz : vz) {
-          const int64_t own = (int64_t)wx * wy * wz;
-          const int64_t tiles = (h->N + own - 1) / own;
-          if (tiles > 1024 || tiles < 2 || own * (4 + (int)spin_bytes(h->stype)) > (int64_t)h->max_lds) continue;
-          const int w[3] = {wx, wy, wz};
-          for (int vec : {1, kVec}) {
-            if (vec > 1 && variant_app(h->d.app)) continue;
-            // no less than this whatever the halo: most shapes end here
-            const double item_us = tile_item_us(h, vec), items = (double)own / h->g.K / vec;
-            const int per_cu = (int)((tiles + kCus - 1) / kCus);
-            const double least = std::max(0.15 + 1.3 * item_us, 1.2 * per_cu * items / 64 / kSimds * item_us);
-            if ((5.0 + S * h->g.K * (0.3 + least)) / S >= best) continue;
+  const int64_t most = std::min<int64_t>(h->N - 1, (int64_t)h->max_lds / (4 + (int)spin_bytes(h->stype)));
+  const int64_t fewest = (h->N + 1023) / 1024;   // sites of a box: at most 1024 boxes, at least two
+  const double item_us[2] = {tile_item_us(h, 1), tile_item_us(h, kVec)}, move_us = 2.0 * (4 + spin_bytes(h->stype)) / 20e3;
+  const int vecs = variant_app(h->d.app) ? 1 : 2;
+  TileRegion region;
+  for (int wx : vx)
+    for (int wy : vy) {
+      if ((int64_t)wx * wy * vz[0] < fewest) break;   // extents fall
+      for (int wz : vz) {
+        const int64_t own = (int64_t)wx * wy * wz;
+        if (own < fewest) break;
+        if (own > most) continue;
+        const int per_cu = (int)(((h->N + own - 1) / own + kCus - 1) / kCus);
+        const int w[3] = {wx, wy, wz};
+        double pass_us[2];   // no less than this a pass whatever the halo: most shapes end here
+        for (int v = 0; v < vecs; v++)
+          pass_us[v] = 0.3 + std::max(0.15 + 1.3 * item_us[v],
+                                      1.2 * per_cu * ((double)own / h->g.K / (v ? kVec : 1)) / 64 / kSimds * item_us[v]);
+        for (int S : {1, 2, 3, 4, 6, 8}) {
+          if (S * h->g.K > kTileMaxPass) break;
+          bool known = false;
+          for (int v = 0; v < vecs; v++) {
+            if ((5.0 + per_cu * own * move_us) / S + h->g.K * pass_us[v] >= best) continue;
+            if (!known && !(known = tile_region(h->g, w, 0, S * h->g.K, region))) break;
+            const int vec = v ? kVec : 1;
             TileShape t;
-            const double us = tile_sweep_us(h, w, S, vec, &t);
+            const double us = tile_sweep_us(h, w, S, vec, region, best, &t);
             if (us < best && tile_fits(h, w, S, vec)) best = us, h->tile = t;
           }
         }
-  }
+      }
+    }
 }
 
 // Which kernels a sweeps call of a lattice beyond one workgroup's reach takes.

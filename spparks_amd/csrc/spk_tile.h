@@ -61,27 +61,29 @@ __host__ __device__ inline int tile_parity(int lat, int c, int d) {
   return -1;
 }
 
-// Fills the plan for `npass` passes from colour c0 on, for owned boxes of
-// w[] lattice sites (w[d] >= the edge: the whole dimension; otherwise even, a
-// multiple of 8 in x).  False when a box would not fit the plan's tables.
-// vec: sites per thread; spin_size: bytes per stored spin.
-inline bool tile_plan_make(const Geom &g, const int (&w)[3], int c0, int npass, int vec, int spin_size, TilePlan *tp) {
+// What passes c0 .. c0+npass-1 update of a box of w sites: pass k the sites
+// [lo[k], hi[k]) of the box moved by org, and the box with its halo, ext sites
+// from org.  False where a plan cannot hold it.
+struct TileRegion {
+  bool whole[3];
+  int org[3], ext[3];
+  int lo[kTileMaxPass][3], hi[kTileMaxPass][3];
+};
+inline bool tile_region(const Geom &g, const int (&w)[3], int c0, int npass, TileRegion &r) {
   if (npass < 1 || npass > kTileMaxPass) return false;
   const int n[3] = {g.nx, g.ny, g.nz};
-  bool whole[3];
-  int lo[3], hi[3];   // N_k, half open
+  int lo[3], hi[3];
   for (int d = 0; d < 3; d++) {
-    whole[d] = w[d] >= n[d];
+    r.whole[d] = w[d] >= n[d];
     lo[d] = 0;
-    hi[d] = whole[d] ? n[d] : w[d];
+    hi[d] = r.whole[d] ? n[d] : w[d];
   }
-  int plo[kTileMaxPass][3], phi[kTileMaxPass][3];
-  for (int k = npass - 1; k >= 0; k--) {
-    const int c = (c0 + k) % g.K;
+  int c = (c0 + npass - 1) % g.K;
+  for (int k = npass - 1; k >= 0; k--, c = c ? c - 1 : g.K - 1) {
     for (int d = 0; d < 3; d++) {
-      plo[k][d] = lo[d];
-      phi[k][d] = hi[d];
-      if (whole[d]) continue;
+      r.lo[k][d] = lo[d];
+      r.hi[k][d] = hi[d];
+      if (r.whole[d]) continue;
       const int p = tile_parity(g.lat, c, d);
       if (p < 0 || (lo[d] & 1) == p) lo[d]--;
       if (p < 0 || ((hi[d] - 1) & 1) == p) hi[d]++;
@@ -89,18 +91,58 @@ inline bool tile_plan_make(const Geom &g, const int (&w)[3], int c0, int npass, 
   }
   // the box with its halo: x from a multiple of 8 (packs of 4 sub-grid
   // sites), y and z from an even row, so parities carry over
-  int org[3], ext[3];
   for (int d = 0; d < 3; d++) {
     const int unit = d == 0 ? 8 : 2;
-    if (whole[d]) {
-      org[d] = 0;
-      ext[d] = n[d];
+    if (r.whole[d]) {
+      r.org[d] = 0;
+      r.ext[d] = n[d];
     } else {
-      org[d] = -((-lo[d] + unit - 1) / unit * unit);
-      ext[d] = (hi[d] - org[d] + unit - 1) / unit * unit;
+      r.org[d] = -((-lo[d] + unit - 1) / unit * unit);
+      r.ext[d] = (hi[d] - r.org[d] + unit - 1) / unit * unit;
     }
   }
-  if (ext[0] > 65535 || ext[1] > 65535 || ext[2] > 65535 || (int64_t)ext[0] * ext[1] * ext[2] > (1 << 20)) return false;
+  return r.ext[0] <= 65535 && r.ext[1] <= 65535 && r.ext[2] <= 65535 &&
+         (int64_t)r.ext[0] * r.ext[1] * r.ext[2] <= (1 << 20);
+}
+
+// The sub-grid of the halo box that pass k (colour c) updates: a along x in
+// sites, b and e its rows and planes.
+struct TileSpan {
+  int a[2], b[2], e[2];
+};
+inline TileSpan tile_span(int lat, const TileRegion &r, int k, int c) {
+  const bool ysub = lat == SPK_HIP_SQ_8N || lat == SPK_HIP_SC_26N, zsub = lat == SPK_HIP_SC_26N;
+  auto sub = [&](int d, bool halved, int (&o)[2]) {
+    const int l = r.lo[k][d] - r.org[d], h = r.hi[k][d] - r.org[d];
+    if (!halved) {
+      o[0] = l, o[1] = h;
+      return;
+    }
+    const int p = tile_parity(lat, c, d);
+    if (p < 0) o[0] = l / 2, o[1] = (h + 1) / 2;        // x of a checkerboard: both parities
+    else o[0] = (l - p + 1) / 2, o[1] = (h - p + 1) / 2;   // sites 2r + p in [l, h)
+  };
+  TileSpan t;
+  sub(0, true, t.a);
+  sub(1, ysub, t.b);
+  sub(2, zsub, t.e);
+  return t;
+}
+// packs of vec sites along x from t.a
+inline uint32_t tile_packs(const TileSpan &t, int vec) {
+  return vec == 4 ? (uint32_t)((t.a[1] + 3) / 4 - t.a[0] / 4) : (uint32_t)(t.a[1] - t.a[0]);
+}
+
+// Fills the plan for `npass` passes from colour c0 on, for owned boxes of
+// w[] lattice sites (w[d] >= the edge: the whole dimension; otherwise even, a
+// multiple of 8 in x).  False when a box would not fit the plan's tables.
+// vec: sites per thread; spin_size: bytes per stored spin.
+inline bool tile_plan_make(const Geom &g, const int (&w)[3], int c0, int npass, int vec, int spin_size, TilePlan *tp) {
+  TileRegion r;
+  if (!tile_region(g, w, c0, npass, r)) return false;
+  const int n[3] = {g.nx, g.ny, g.nz};
+  const int (&org)[3] = r.org, (&ext)[3] = r.ext;
+  const bool (&whole)[3] = r.whole;
   geom_init(tp->gl, g.lat, ext[0], ext[1], ext[2]);
   tp->ox = -org[0], tp->oy = -org[1], tp->oz = -org[2];
   tp->wx = whole[0] ? n[0] : w[0], tp->wy = whole[1] ? n[1] : w[1], tp->wz = whole[2] ? n[2] : w[2];
@@ -109,28 +151,13 @@ inline bool tile_plan_make(const Geom &g, const int (&w)[3], int c0, int npass, 
   tp->npass = npass;
   tp->vec = vec;
   tp->spin_bytes = ((uint32_t)tp->gl.K * (uint32_t)tp->gl.Mp * (uint32_t)spin_size + 15u) / 16u * 16u;
-  const bool ysub = g.lat == SPK_HIP_SQ_8N || g.lat == SPK_HIP_SC_26N, zsub = g.lat == SPK_HIP_SC_26N;
   for (int k = 0; k < npass; k++) {
-    const int c = (c0 + k) % g.K;
-    int a[2], b[2], e[2];
-    auto sub = [&](int d, bool halved, int (&r)[2]) {
-      const int l = plo[k][d] - org[d], h = phi[k][d] - org[d];
-      if (!halved) {
-        r[0] = l, r[1] = h;
-        return;
-      }
-      const int p = tile_parity(g.lat, c, d);
-      if (p < 0) r[0] = l / 2, r[1] = (h + 1) / 2;        // x of a checkerboard: both parities
-      else r[0] = (l - p + 1) / 2, r[1] = (h - p + 1) / 2;   // sites 2r + p in [l, h)
-    };
-    sub(0, true, a);
-    sub(1, ysub, b);
-    sub(2, zsub, e);
+    const TileSpan sp = tile_span(g.lat, r, k, (c0 + k) % g.K);
     TilePass &t = tp->pass[k];
-    t.p0 = (uint16_t)(a[0] / vec);
-    t.np = (uint16_t)((a[1] + vec - 1) / vec - a[0] / vec);
-    t.b0 = (uint16_t)b[0], t.nb = (uint16_t)(b[1] - b[0]);
-    t.e0 = (uint16_t)e[0], t.ne = (uint16_t)(e[1] - e[0]);
+    t.p0 = (uint16_t)(sp.a[0] / vec);
+    t.np = (uint16_t)tile_packs(sp, vec);
+    t.b0 = (uint16_t)sp.b[0], t.nb = (uint16_t)(sp.b[1] - sp.b[0]);
+    t.e0 = (uint16_t)sp.e[0], t.ne = (uint16_t)(sp.e[1] - sp.e[0]);
     t.items = (uint32_t)t.np * t.nb * t.ne;
     t.fp = fastdiv_make(t.np);
     t.fb = fastdiv_make(t.nb);
