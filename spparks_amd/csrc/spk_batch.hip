@@ -1099,9 +1099,12 @@ int spk_hip_batch_run(spk_hip_batch *b, int max_sweeps, int use_graph) {
       return w;
     };
     const int C = (int)cand.size();
-    // each candidate gets whole sweeps of an 8-colour replica when the
-    // block has room, else single steps in turn
-    const int per = L / C >= 8 ? L / C / 8 * 8 : 1;
+    // each candidate gets whole sweeps (of the replica with most steps) when
+    // the block has room, else single steps in turn
+    int sweeps = 1;
+    for (const auto &R : b->reps) sweeps = std::max(sweeps, R.live ? R.block_sweeps : 0);
+    const int unit = std::max(1, L / sweeps);
+    const int per = L / C >= unit ? L / C / unit * unit : 1;
     std::vector<double> t_ms(C, 0.0), work(C, 0.0);
     double tot = 0.0;
     int j = 0;
