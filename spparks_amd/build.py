@@ -101,6 +101,28 @@ def build_emulator():
     return outs
 
 
+def build_host_library():
+    """tests/emul/libspk_host.so: the library's own sources as host code on a
+    stand-in for the HIP runtime, for the CPU tests of its host side.  Test
+    infrastructure."""
+    emul = os.path.join(ROOT, "tests", "emul")
+    src = os.path.join(emul, "spk_host.hip")
+    if not os.path.exists(src):
+        return None
+    out = os.path.join(emul, "libspk_host.so")
+    srcs = [os.path.join(CSRC, s) for s in HIP_SOURCES] + [src]
+    objs = [os.path.join(emul, os.path.basename(s)[:-4] + ".host.o") for s in srcs]
+    with ThreadPoolExecutor(4) as pool:
+        list(pool.map(lambda s, o: run([hipcc(), "-x", "hip", "--offload-host-only", "-fuse-cuid=none", "-O1",
+                                        "-std=c++20", "-ffp-contract=off", "-fPIC", "-I" + INCLUDE, "-I" + CSRC,
+                                        "-c", s, "-o", o]), srcs, objs))
+    # (without a cuid the sources share the names of their registration data)
+    run([cxx(), "-shared", "-Wl,-Bsymbolic", "-Wl,-z,defs", "-Wl,-z,muldefs", "-o", out, *objs, "-lpthread"])
+    for o in objs:
+        os.remove(o)
+    return out
+
+
 def build_abi_consumer():
     """tests/abi/consumer: a plain C99 caller of libspk_hip.so and
     libspparks_hip.so through their headers.  Test infrastructure."""

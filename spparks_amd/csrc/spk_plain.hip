@@ -877,6 +877,17 @@ int ensure_pinned(spk_hip_lattice *h, int rows) {
   return SPK_HIP_OK;
 }
 
+// Pinned memory for the whole state of a small lattice; without it downloads
+// go through the staging array.
+bool ensure_pinned_state(spk_hip_lattice *h) {
+  if (!h->pinned_state && hipHostMalloc(&h->pinned_state, 2 * (size_t)h->N * sizeof(int32_t), hipHostMallocDefault) !=
+                              hipSuccess) {
+    h->pinned_state = nullptr;
+    (void)hipGetLastError();   // not an error of the call
+  }
+  return h->pinned_state != nullptr;
+}
+
 // Two sweeps in one launch (k_sweep_bits_pair), from the planes and seeds
 // at `from` (0: bits/sseed, 1: bits2/sseed2) to the others.
 int launch_pair(spk_hip_lattice *h, int from, unsigned long long *acc) {
@@ -1320,9 +1331,7 @@ int spk_hip_download(spk_hip_lattice *h, int32_t *spin, int32_t *seed) {
   // ends it.  As two kernels, two copies and two waits, and so: 64^2 30.8 and
   // 13.9 us, 128^2 45.5 and 17.4, 40^3 52.5 and 32.0; from 50^3 on the copy out
   // of that memory takes what is saved.
-  if (h->N <= kHostStateSites &&
-      (h->pinned_state ||
-       hipHostMalloc(&h->pinned_state, 2 * bytes, hipHostMallocDefault) == hipSuccess)) {
+  if (h->N <= kHostStateSites && ensure_pinned_state(h)) {
     with_type(h->stype, [&]<typename T>() {
       hipLaunchKernelGGL((k_state_natural<T>), dim3(grid_for(h->N, 256)), dim3(256), 0, h->stream,
                          spin ? static_cast<const T *>(h->spin) : nullptr, seed ? h->seed : nullptr, h->pinned_state,

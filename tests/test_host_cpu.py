@@ -1,0 +1,75 @@
+"""The library's host side on the CPU: its own sources, built as host code
+against a stand-in for the HIP runtime (tests/emul/spk_host.hip) in which
+kernels do nothing and every launch and allocation is counted.  What a call
+launches, allocates and gives back, and what it does when an allocation
+fails."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIB = os.path.join(HERE, "emul", "libspk_host.so")
+
+
+class Runtime:
+    """The stand-in's own calls."""
+
+    def __init__(self, L):
+        self.L = L
+        for name in ("device_bytes", "device_calls", "pinned_calls", "execs", "captures"):
+            f = getattr(L, "spk_host_" + name)
+            f.restype = C.c_long
+            setattr(self, name, f)
+        L.spk_host_log.restype = C.c_char_p
+        for name in ("limit", "free_memory"):
+            getattr(L, "spk_host_" + name).argtypes = [C.c_size_t]
+
+    def limit(self, more):
+        """Device allocations fail beyond `more` bytes from now."""
+        self.L.spk_host_limit(self.device_bytes() + more if more is not None else 0)
+
+    def fail_pinned(self, n):
+        self.L.spk_host_fail_pinned(n)
+
+    def fail_info(self, n):
+        self.L.spk_host_fail_info(n)
+
+    def free_memory(self, n):
+        self.L.spk_host_free_memory(n)
+
+    def log(self):
+        """(kernel, workgroups, threads) of the launches since the last call."""
+        return [(a, int(b), int(c)) for a, b, c in
+                (line.rsplit(" ", 2) for line in self.L.spk_host_log().decode().splitlines())]
+
+    def sweeps(self):
+        """Names of the sweep kernels launched since the last call."""
+        return [n.split("<")[0] for n, _, _ in self.log() if n.startswith(("k_sweep", "k_batch"))]
+
+
+@pytest.fixture
+def host(monkeypatch):
+    from spparks_amd import batch, hip
+    L = hip.load_library(LIB)
+    monkeypatch.setattr(hip, "_lib", L)
+    monkeypatch.setattr(batch, "_bound", False)
+    r = Runtime(L)
+    L.spk_host_reset()
+    yield r
+    L.spk_host_reset()
+
+
+def lattice(app="potts", style="sq/8n", shape=(64, 64, 1), q=100, kt=0.5):
+    import spparks_amd as S
+    return S.Lattice(app, style, *shape, nspins=q, temperature=kt)
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 1), (256, 256, 1)])
+def test_download_without_pinned_memory_takes_the_staging_path(host, shape):
+    with lattice(shape=shape) as L:
+        host.fail_pinned(1)
+        spin, seed = L.download()
+        assert spin.size == seed.size == L.n
+        L.download()
