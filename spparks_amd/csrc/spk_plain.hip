@@ -323,6 +323,7 @@ struct spk_hip_lattice {
   int bitplanes = 1;
   bool bits_active = false;
   bool pairs = false;                  // planes in the spt-8 layout, sweeps two per launch
+  bool pairs_ok = true;                // false once the second planes did not fit the device's memory
   // the same for bit-sliced lattices (spk_slice.h), which use bits and sseed
   // for their planes and seeds
   bool slice_active = false;
@@ -751,14 +752,20 @@ int ensure_planes(uint32_t *&p, const spk_hip_lattice *h) {
 }
 
 int bits_enter(spk_hip_lattice *h) {
-  h->pairs = h->bitplanes == 1 && pair_fits(h->g) && pair_sweep_us(h) < colour_bits_us(h);
+  h->pairs = h->pairs_ok && h->bitplanes == 1 && pair_fits(h->g) && pair_sweep_us(h) < colour_bits_us(h);
   h->bg = bit_geom(h->g, h->pairs ? 8 : h->bitplanes == 1 ? kBitSites : h->bitplanes);
   int rc;
   if ((rc = ensure_planes(h->bits, h)) || (rc = ensure_shadow(h, h->sseed, h->sseed_cap, 2 * h->bg.seedc)))
     return rc;
   if (h->pairs &&
-      ((rc = ensure_planes(h->bits2, h)) || (rc = ensure_shadow(h, h->sseed2, h->sseed2_cap, 2 * h->bg.seedc))))
-    return rc;
+      ((rc = ensure_planes(h->bits2, h)) || (rc = ensure_shadow(h, h->sseed2, h->sseed2_cap, 2 * h->bg.seedc)))) {
+    if (rc != SPK_HIP_ENOMEM) return rc;
+    (void)hipGetLastError();   // no room for the second planes: one colour a launch, which needs none
+    (void)hipFree(h->bits2);
+    h->bits2 = nullptr;
+    h->pairs_ok = false;
+    return bits_enter(h);
+  }
   const int64_t words = 2 * (int64_t)h->g.hy * h->bg.pw;
   hipLaunchKernelGGL(k_bits_pack, dim3(grid_for(words, 256)), dim3(256), 0, h->stream,
                      static_cast<const uint8_t *>(h->spin), h->g, h->bg, h->bits);

@@ -73,3 +73,29 @@ def test_download_without_pinned_memory_takes_the_staging_path(host, shape):
         spin, seed = L.download()
         assert spin.size == seed.size == L.n
         L.download()
+
+
+def state_bytes(L):
+    """Bytes of a two-state sq/4n lattice's planes and of their seeds."""
+    nx, ny, _ = L.shape
+    pw = (nx // 2 + 31) // 32
+    return 2 * ny * pw * 4, 2 * ny * pw * 32 * 4
+
+
+@pytest.mark.parametrize("second", [0.0, 0.5, 1.2])
+def test_two_state_lattice_without_second_planes_sweeps_one_colour_a_launch(host, second):
+    """Room for the planes and their seeds, and for none, some, or the planes
+    and part of the seeds of the second ones."""
+    with lattice("ising", "sq/4n", (1000, 1000, 1), 2, 2.269) as L:
+        planes, seeds = state_bytes(L)
+        host.limit(int(planes * (1 + second) + seeds))
+        host.log()
+        L.prepare(5)
+        L.sweeps(5)
+        assert host.sweeps() == ["k_sweep_bits"] * 10 and L.last_timing()[1] == 10
+        host.limit(None)
+        L.sweeps(4)
+        assert host.sweeps() == ["k_sweep_bits"] * 8
+    with lattice("ising", "sq/4n", (1000, 1000, 1), 2, 2.269) as L:
+        L.sweeps(4)
+        assert host.sweeps() == ["k_sweep_bits_pair"] * 2
