@@ -785,7 +785,11 @@ int slice_enter(spk_hip_lattice *h) {
     h->bits = nullptr;
     return set_error(SPK_HIP_ENOMEM, "bit planes not available");
   }
-  if ((rc = ensure_shadow(h, h->sseed, h->sseed_cap, h->g.K * h->sg.seedc))) return rc;
+  if ((rc = ensure_shadow(h, h->sseed, h->sseed_cap, h->g.K * h->sg.seedc))) {
+    (void)hipFree(h->bits);   // of no use without the seeds
+    h->bits = nullptr;
+    return rc;
+  }
   slice_in(h->stream, h->spin, h->stype, h->seed, h->g, h->sg, h->bits, h->sseed);
   rc = check_hip(hipGetLastError(), "bit-plane pack");
   if (!rc) h->slice_active = true;

@@ -99,3 +99,13 @@ def test_two_state_lattice_without_second_planes_sweeps_one_colour_a_launch(host
     with lattice("ising", "sq/4n", (1000, 1000, 1), 2, 2.269) as L:
         L.sweeps(4)
         assert host.sweeps() == ["k_sweep_bits_pair"] * 2
+
+
+def test_sliced_lattice_without_its_seeds_keeps_no_planes(host):
+    with lattice("potts", "sc/26n", (128, 128, 128), 10000) as L:
+        before = host.device_bytes()
+        host.limit(128**3 * 5)   # planes of 2 bytes a site fit, 4 of seeds beside them do not
+        host.log()
+        L.sweeps(2)
+        assert host.sweeps() == ["k_sweep_color"] * 16
+        assert host.device_bytes() == before
