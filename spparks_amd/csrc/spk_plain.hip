@@ -548,10 +548,29 @@ double tile_site_valu(const spk_hip_lattice *h) {
 constexpr double kUsPerValu = 4.0 / 2400.0;   // a wavefront's instruction on its SIMD: 4 cycles at 2.4 GHz
 constexpr int kSimds = 4, kCus = 256;
 
+// Whether a pass on bit planes (two colours) is faster than two of the packed
+// kernel.  Rows of an awkward width leave bits of their plane words empty, as work
+// and as seed memory (hx 8: three quarters of them).  Both sides' times fitted
+// to 487 lattices from 16 x 100^2 to 256^3 and 40 x 1000^2, Q of 5 to 10^6,
+// mostly within 5%: two of them are on the slower side, by 1 and 4%.  us a sweep,
+// packed and on planes:
+//   16 x 400^2 Q=5 38.3, 33.2; Q=3000 42.3, 45.8; 16 x 700^2 Q=5 55.5, 64.3
+//   16 x 1000^2 Q=100 82.1, 134; Q=10^4 97, 190; 32 x 512^2 Q=100 55.7, 49.7; Q=60000 62.8, 66.6
+//   40 x 400^2 Q=5 52.0, 34.6; Q=10^6 76.6, 57.9; 256^3 Q=5 80.2, 42.9; Q=10^6 142, 74.9
+bool slice_pays(const spk_hip_lattice *h) {
+  const SliceGeom sg = slice_geom(h->g, h->rule.nspins);
+  const double waves = sg.waves / 1024.0, planes = 4.1 + 0.33 * sg.PG + waves * (1.28 + 0.469 * sg.PG);
+  const double pw = (double)h->g.Mp / 4 / 64 / 1024;   // the packed kernel's wavefronts
+  const double packed = h->stype == kU8    ? std::max(4.0, 3.7 + 0.855 * pw)
+                        : h->stype == kU16 ? std::max(4.3, 4.05 + 1.038 * pw)
+                                           : std::max(4.8, 3.8 + 1.83 * pw);
+  return planes < 0.98 * 2 * packed;
+}
+
 // Lattices that sweep on bit planes of the spins (spk_slice.h).
 bool slice_eligible(const spk_hip_lattice *h) {
   return h->slice_ok && !variant_app(h->d.app) && !h->block_set && slice_fits(h->g, h->rule.nspins) &&
-         h->rule.half == (1 << 30);
+         h->rule.half == (1 << 30) && slice_pays(h);
 }
 
 // Microseconds a sweep is expected to take on bit planes, one colour a launch

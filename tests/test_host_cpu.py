@@ -109,3 +109,22 @@ def test_sliced_lattice_without_its_seeds_keeps_no_planes(host):
         L.sweeps(2)
         assert host.sweeps() == ["k_sweep_color"] * 16
         assert host.device_bytes() == before
+
+
+@pytest.mark.parametrize("shape,q,sliced", [
+    ((16, 700, 700), 100, False),      # words a quarter full
+    ((16, 1000, 1000), 10000, False),
+    ((32, 512, 512), 60000, False),    # half full
+    ((32, 700, 700), 3000, False),
+    ((32, 512, 512), 5, True),
+    ((32, 700, 700), 1000000, True),
+    ((48, 500, 500), 60000, True),     # three quarters
+    ((224, 224, 200), 10000, True),
+])
+def test_narrow_rows_sweep_on_planes_only_where_that_is_faster(host, shape, q, sliced):
+    """A row of up to 16 sites a colour leaves half of its plane words or more
+    empty: large lattices of them sweep packed (one launch a colour)."""
+    with lattice("potts", "sc/26n", shape, q) as L:
+        host.log()
+        L.sweeps(1)
+        assert host.sweeps() == (["k_sweep_slice"] * 4 if sliced else ["k_sweep_color"] * 8)
