@@ -927,10 +927,8 @@ int launch_pair(spk_hip_lattice *h, int from, unsigned long long *acc) {
 }
 
 // Sweep-kernel launches that launch_sweeps makes for n sweeps.
-int tile_launches(const spk_hip_lattice *h, int n);
-int64_t sweep_launches(const spk_hip_lattice *h, int n, Route route) {
-  if (route == kRouteTile) return tile_launches(h, n);
-  if (route == kRouteSlice) return (int64_t)h->g.K / 2 * n;
+int64_t sweep_launches(const spk_hip_lattice *h, int n) {
+  if (h->slice_active) return (int64_t)h->g.K / 2 * n;
   if (h->bits_active && h->pairs) return 2 * (n / 4) + (int64_t)h->g.K * (n % 4);
   return (int64_t)h->g.K * n;
 }
@@ -978,7 +976,12 @@ int launch_tile(spk_hip_lattice *h, int from, int q0, int q1, unsigned long long
 
 // n sweeps through the tile kernel, split evenly over its launches: whole
 // sweeps each, or (one sweep, or one sweep a launch and an odd number of
-// them) at colours inside a sweep
+// them) at colours inside a sweep.  Launched one by one, never captured: the
+// device takes longer over a launch than the host, and a graph for each number of
+// sweeps and each temperature cost 70 us where one workgroup had needed none.  us
+// a call of 2, 10 and 200 sweeps: 100^2 Ising replayed 49, 50, 492, launched 32, 43,
+// 425; 128^2 sq/8n 45, 66, 857 and 35, 59, 786; 64^3 sc/26n 59, 176, 3018 and
+// 51, 175, 2980.  After a change of temperature 2 sweeps took 126, 125 and 134.
 int launch_tiles(spk_hip_lattice *h, int n, unsigned long long *acc, int64_t *nlaunch) {
   const int m = tile_launches(h, n);
   auto cut = [&](int j) {
@@ -1097,7 +1100,7 @@ int piece_graph(spk_hip_lattice *h, int n, Route rt, hipGraphExec_t *out) {
   hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->acc, words);
   int64_t nl = 0;
   rc = check_hip(hipGetLastError(), "zero launch");
-  if (!rc) rc = rt == kRouteTile ? launch_tiles(h, n, h->acc, &nl) : launch_sweeps(h, n, h->acc, &nl);
+  if (!rc) rc = launch_sweeps(h, n, h->acc, &nl);
   const hipError_t e = hipStreamEndCapture(h->stream, &graph);
   if (!rc) rc = check_hip(e, "end capture");
   if (rc) {
@@ -1461,7 +1464,25 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
   // (on the bit planes the state stays there)
   Route rt;
   if ((rc = enter_route(h, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
-  if (h->chunk > 0) {
+  // rows [0, n) cleared
+  auto clear = [&](int n) {
+    const int64_t words = (int64_t)n * kAccRow;
+    hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->acc, words);
+    return check_hip(hipGetLastError(), "zero launch");
+  };
+  if (rt == kRouteTile) {
+    // boxes: from the host (launch_tiles), in pieces of kInitialAccRows sweeps
+    if ((rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows))) ||
+        (rc = check_hip(hipEventRecord(h->ev0, h->stream), "event")))
+      return rc;
+    for (int done = 0; done < nsweeps;) {
+      const int n = std::min(nsweeps - done, kInitialAccRows);
+      if ((rc = clear(n)) || (rc = launch_tiles(h, n, h->acc, &nlaunch)) ||
+          (rc = launch_fold(h, h->acc, n, h->pinned + (size_t)done * 2)))
+        return rc;
+      done += n;
+    }
+  } else if (h->chunk > 0) {
     // graph replays (graph_pieces); each piece's rows are folded into the
     // pinned rows [done, done + n) before the next piece clears them
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
@@ -1477,16 +1498,11 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
         return rc;
       done += pieces[k];
     }
-    for (int n : pieces) nlaunch += sweep_launches(h, n, rt);
+    for (int n : pieces) nlaunch += sweep_launches(h, n);
   } else {
     // every launch from the host: rows [0, nsweeps)
-    if ((rc = ensure_acc(h, nsweeps))) return rc;
-    const int64_t words = (int64_t)nsweeps * kAccRow;
-    if ((rc = check_hip(hipEventRecord(h->ev0, h->stream), "event"))) return rc;
-    hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->acc, words);
-    if ((rc = check_hip(hipGetLastError(), "zero launch")) ||
-        (rc = rt == kRouteTile ? launch_tiles(h, nsweeps, h->acc, &nlaunch)
-                               : launch_sweeps(h, nsweeps, h->acc, &nlaunch)) ||
+    if ((rc = ensure_acc(h, nsweeps)) || (rc = check_hip(hipEventRecord(h->ev0, h->stream), "event")) ||
+        (rc = clear(nsweeps)) || (rc = launch_sweeps(h, nsweeps, h->acc, &nlaunch)) ||
         (rc = launch_fold(h, h->acc, nsweeps, h->pinned)))
       return rc;
   }
@@ -1523,7 +1539,9 @@ int spk_hip_prepare(spk_hip_lattice *h, int nsweeps) {
   int rc;
   Route rt;
   if ((rc = enter_route(h, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
-  if (h->chunk > 0) {
+  if (rt == kRouteTile) {
+    if ((rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows)))) return rc;
+  } else if (h->chunk > 0) {
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
     if ((rc = ensure_acc(h, pieces[0]))) return rc;
     for (int n : pieces) {

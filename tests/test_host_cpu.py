@@ -128,3 +128,32 @@ def test_narrow_rows_sweep_on_planes_only_where_that_is_faster(host, shape, q, s
         host.log()
         L.sweeps(1)
         assert host.sweeps() == (["k_sweep_slice"] * 4 if sliced else ["k_sweep_color"] * 8)
+
+
+@pytest.mark.parametrize("case", [("potts", "sq/8n", (128, 128, 1), 100), ("ising", "sq/4n", (100, 100, 1), 2)],
+                         ids=lambda c: "x".join(map(str, c[2])))
+def test_boxes_capture_no_graph(host, case):
+    """Lattices of one workgroup's size have no graph to capture for each number of
+    sweeps and each temperature, as in one workgroup."""
+    with lattice(*case) as L:
+        captures = host.captures()
+        for n in range(2, 40, 7):
+            L.set_temperature(0.1 * n)
+            L.prepare(n)
+            host.log()
+            L.sweeps(n)
+            assert set(host.sweeps()) == {"k_sweep_tile"}
+        assert host.captures() == captures
+
+
+def test_boxes_take_long_calls_in_pieces(host):
+    with lattice("potts", "sq/8n", (600, 500, 1)) as L:
+        L.prepare(2)
+        L.energy()
+        before = host.device_bytes()
+        host.log()
+        L.sweeps(2500)
+        log = [n.split("<")[0] for n, _, _ in host.log()]
+        assert log.count("k_zero_u64") == log.count("k_fold_rows") == 3
+        assert host.device_bytes() == before
+        assert log.count("k_sweep_tile") == L.last_timing()[1] < 2500 and log.count("k_sweep_tile") % 2 == 0
