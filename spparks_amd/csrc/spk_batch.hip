@@ -158,6 +158,7 @@ __global__ __launch_bounds__(1024) void k_batch_step(char *__restrict__ pool, co
 // quarter empty on the average, and the last wavefronts of a step.  Replicas
 // with most planes first in the list: 0.099 and 97, taken back.
 constexpr int kSliceBlock = 256;
+constexpr int kSliceResident = 1024;   // workgroups the chip holds at once: four a compute unit
 
 __global__ __launch_bounds__(kSliceBlock, 4) void k_batch_slice(const BatchRep *__restrict__ reps,
                                                              const StepDesc *__restrict__ steps,
@@ -166,8 +167,13 @@ __global__ __launch_bounds__(kSliceBlock, 4) void k_batch_slice(const BatchRep *
   __shared__ SliceLds lds[kSliceBlock / 64];
   const StepDesc sd = steps[j];
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int t = xcd_tile(blockIdx.x, gridDim.x) * (kSliceBlock / 64) + wid;
-  if (t >= sd.total) return;   // no wavefront waits for another
+  // an eighth of the step's own workgroups to each XCD, whatever the grid (one
+  // recorded for more of them has surplus ones: spread over the grid the tiles would leave
+  // the last XCD idle)
+  const int per = (sd.total + kNumXcd * kSliceBlock / 64 - 1) / (kNumXcd * kSliceBlock / 64);
+  const int xcd = (int)blockIdx.x % kNumXcd, wg = (int)blockIdx.x / kNumXcd;
+  const int t = (xcd * per + wg) * (kSliceBlock / 64) + wid;
+  if (wg >= per || t >= sd.total) return;   // no wavefront waits for another
   const int *pp = pre + sd.pre_first;
   int lo = 0, hi = sd.count - 1;   // the replica holding tile t: last i with pp[i] <= t
   while (lo < hi) {
@@ -377,8 +383,15 @@ struct spk_hip_batch {
   hipEvent_t fork_ev = nullptr, join_ev[kNumVariants] = {};
   // launch shape
   int block = 0, grid = 0;          // 0 = autotune on the next run
-  // by (block, grid, then v and L of each variant), then by k_batch_slice's grid
-  std::map<std::vector<int>, std::map<int, hipGraphExec_t>> graphs;
+  // recorded blocks, at most kMaxGraphs of them
+  struct Recorded {
+    std::vector<int> key;   // block, grid, then v and L of each variant
+    int slice_grid;         // workgroups of k_batch_slice
+    hipGraphExec_t exec;
+    int64_t used;           // when last
+  };
+  std::vector<Recorded> graphs;
+  int64_t graph_uses = 0;
   std::vector<hipEvent_t> events;
   double last_ms = 0.0;
   int64_t last_updates = 0, last_nlaunch = 0;
@@ -493,14 +506,18 @@ int replica_checksum_async(spk_hip_batch *b, int id) {
 // Builds the block's replica table and, per variant present, the step
 // schedule.  Replica r with P_r passes is due at step j when
 // floor((j+1)P_r/L) > floor(j P_r/L), L being its variant's steps; its pass
-// index is then floor(j P_r/L), so its passes run once each, in order.  L_out
-// is the largest of the variants' L, which launch_steps counts in.
+// index is then floor(j P_r/L), so its passes run once each, in order.  A
+// variant has the steps of as many sweeps as the block's longest replica, its
+// own or another's: the kinds then differ in nothing from block to block that
+// a recorded graph would have to follow.  L_out is the largest of the variants'
+// L, which launch_steps counts in.
 int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, int64_t *updates_out) {
   b->h_reps.clear();
   std::vector<int> vrep;   // variant of each table entry
   int L = 0, rows = 0;
   int64_t updates = 0;
-  int steps[kNumVariants] = {};
+  int passes[kNumVariants] = {};   // a sweep's, of the kinds present
+  int sweeps = 0;
   for (int id = 0; id < (int)b->reps.size(); id++) {
     Replica &R = b->reps[id];
     R.block_sweeps = 0;
@@ -515,7 +532,8 @@ int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, 
     br.rule = R.rule;
     br.stype = R.stype;
     const bool sliced = R.variant == kSliceVariant;
-    br.P = (sliced ? R.g.K / 2 : R.g.K) * R.block_sweeps;
+    passes[R.variant] = sliced ? R.g.K / 2 : R.g.K;
+    br.P = passes[R.variant] * R.block_sweeps;
     br.acc_row = R.acc_row;
     br.tiles = sliced ? R.s.waves : (int)((R.g.Mp / kVec + kTile - 1) / kTile);
     br.spin_off = R.spin_off;
@@ -526,8 +544,7 @@ int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, 
     R.stale = sliced;
     b->h_reps.push_back(br);
     vrep.push_back(R.variant);
-    steps[R.variant] = std::max(steps[R.variant], br.P);
-    L = std::max(L, br.P);
+    sweeps = std::max(sweeps, R.block_sweeps);
     updates += (int64_t)R.g.M * R.g.K * R.block_sweeps;
   }
   b->variants.clear();
@@ -535,8 +552,9 @@ int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, 
   b->h_act.clear();
   b->h_pre.clear();
   for (int v = 0; v < kNumVariants; v++) {
-    if (!steps[v]) continue;
-    spk_hip_batch::Variant var{v, steps[v], (int)b->h_steps.size(), 0};
+    if (!passes[v]) continue;
+    spk_hip_batch::Variant var{v, passes[v] * sweeps, (int)b->h_steps.size(), 0};
+    L = std::max(L, var.L);
     for (int j = 0; j < var.L; j++) {
       StepDesc sd{(int)b->h_act.size(), 0, (int)b->h_pre.size(), 0};
       b->h_pre.push_back(0);
@@ -565,9 +583,24 @@ int build_schedule(spk_hip_batch *b, int max_sweeps, int *L_out, int *rows_out, 
 }
 
 void drop_graphs(spk_hip_batch *b) {
-  for (auto &kv : b->graphs)
-    for (auto &gv : kv.second) (void)hipGraphExecDestroy(gv.second);
+  for (auto &r : b->graphs) (void)hipGraphExecDestroy(r.exec);
   b->graphs.clear();
+}
+
+// Graphs a batch holds; the one not used for longest makes way.
+constexpr size_t kMaxGraphs = 64;
+
+// The grid a step of `need` workgroups of k_batch_slice is recorded with when
+// their number has changed: as many as the chip holds at once, or the next of four
+// sizes in an octave, so that a queue whose tiles change with every solve does not
+// have every block recorded.  The surplus workgroups leave at once.  300 mixed solves,
+// 16 live, 5 sweeps a block: 134 blocks took 121 ms with most of them recorded (49 ms
+// of steps), 86 with 11 graphs.
+int recorded_grid(int need) {
+  if (need == 0) return 0;
+  int unit = kSliceResident / 4;
+  while (unit * 8 <= need) unit *= 2;
+  return std::max(kSliceResident, (need + unit - 1) / unit * unit);
 }
 
 int upload_schedule(spk_hip_batch *b, int rows, bool clear_acc) {
@@ -984,12 +1017,27 @@ int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph) {
       key.push_back(var.L);
       if (var.v == kSliceVariant) need = var.grid;
     }
-    // a graph recorded for more workgroups serves, up to half as many again
-    // (the surplus ones leave at once): a queue of solves changes its tiles
-    // with every one that comes or goes
-    auto &shapes = b->graphs[key];
-    auto it = shapes.lower_bound(need);
-    if (it == shapes.end() || it->first > need + need / 2) {
+    // a graph recorded for more workgroups serves, up to half as many again:
+    // a queue of solves changes its tiles with every one that comes or goes
+    spk_hip_batch::Recorded *rec = nullptr;
+    // to record with: an ensemble that keeps its replicas has no use for more
+    int slice_grid = need ? std::max(need, kSliceResident) : 0;
+    for (auto &r : b->graphs) {
+      if (r.key != key) continue;
+      slice_grid = recorded_grid(need);
+      if (r.slice_grid >= need && r.slice_grid <= std::max(kSliceResident, need + need / 2) &&
+          (!rec || r.slice_grid < rec->slice_grid))
+        rec = &r;
+    }
+    if (!rec) {
+      if (b->graphs.size() >= kMaxGraphs) {
+        auto old = std::min_element(b->graphs.begin(), b->graphs.end(),
+                                    [](const auto &x, const auto &y) { return x.used < y.used; });
+        (void)hipGraphExecDestroy(old->exec);
+        b->graphs.erase(old);
+      }
+      for (auto &var : b->variants)
+        if (var.v == kSliceVariant) var.grid = slice_grid;
       hipGraph_t graph = nullptr;
       if ((rc = check_hip(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "begin capture")))
         return rc;
@@ -1004,10 +1052,12 @@ int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph) {
       rc = check_hip(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "graph instantiate");
       (void)hipGraphDestroy(graph);
       if (rc) return rc;
-      it = shapes.emplace(need, exec).first;
+      b->graphs.push_back({key, slice_grid, exec, 0});
+      rec = &b->graphs.back();
     }
+    rec->used = ++b->graph_uses;
     if ((rc = check_hip(hipEventRecord(b->events[0], b->stream), "event")) ||
-        (rc = check_hip(hipGraphLaunch(it->second, b->stream), "graph launch")) ||
+        (rc = check_hip(hipGraphLaunch(rec->exec, b->stream), "graph launch")) ||
         (rc = check_hip(hipEventRecord(b->events[1], b->stream), "event")))
       return rc;
   } else {

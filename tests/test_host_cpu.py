@@ -157,3 +157,46 @@ def test_boxes_take_long_calls_in_pieces(host):
         assert log.count("k_zero_u64") == log.count("k_fold_rows") == 3
         assert host.device_bytes() == before
         assert log.count("k_sweep_tile") == L.last_timing()[1] < 2500 and log.count("k_sweep_tile") % 2 == 0
+
+
+def mixed_queue(n, seed=6):
+    rng = np.random.default_rng(seed)
+    reqs = []
+    for i in range(n):
+        e = 2 * int(rng.integers(8, 33))
+        style, shape, q = [("sc/26n", (e, e, e), 3000), ("sq/8n", (4 * e, 4 * e, 1), 100),
+                           ("sc/26n", (2 * e, e, e), 100)][int(rng.integers(0, 3))]
+        reqs.append({"app": "potts", "lattice": style, "shape": shape, "nspins": q, "kT": 0.5, "seed": i + 1,
+                     "sweeps": int(rng.integers(3, 60)), "arrive": 0.0})
+    return reqs
+
+
+def test_queue_of_mixed_solves_records_few_graphs(host):
+    """A queue whose replicas come and go changes its tile counts, and the sweeps
+    each kind has left, with nearly every block: the blocks share graphs."""
+    from spparks_amd import batch
+    start = host.captures()
+    res, st = batch.serve(mixed_queue(300), pool_bytes=4 << 30, max_live=16, block_sweeps=5, block=256, grid=2048)
+    assert all(r["status"] == 0 for r in res) and st["blocks"] > 100
+    # sweeps of a block are 5 until the queue runs out; of the kinds present (4:
+    # planes and packed rows of u8 and u16) the two with most replicas always are, and the
+    # grid has four sizes an octave
+    assert host.captures() - start <= 40
+    assert host.execs() == 0
+
+
+def test_batch_holds_a_bounded_number_of_graphs(host):
+    from spparks_amd import batch
+    with batch.Batch(16 << 20, 2) as B:
+        B.set_launch(256, 1024)
+        B.add(batch.replica_desc("potts", "sq/8n", 64, 64, nspins=100, temperature=0.5, nsweeps=10**6))
+        for n in (100, *range(1, 101)):      # (the longest first: its tables serve the others)
+            B.run(n)
+        assert host.execs() == 64
+        start = host.captures()
+        for n in range(37, 101):
+            B.run(n)
+        assert host.captures() == start      # the 64 used last are held
+        B.run(36)
+        assert host.captures() == start + 1 and host.execs() == 64
+    assert host.execs() == 0
