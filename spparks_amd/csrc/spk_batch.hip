@@ -306,8 +306,12 @@ class SideMemory {
       if (c->alloc.alloc(n, &off)) return c->base + off;
     const int64_t size = std::max<int64_t>(n, (int64_t)64 << 20);
     size_t free_bytes = 0, total = 0;
-    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || (int64_t)free_bytes - size < (int64_t)(total / 4)) return nullptr;
     char *p = nullptr;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+      (void)hipGetLastError();   // not an error of the call
+      return nullptr;
+    }
+    if ((int64_t)free_bytes - size < (int64_t)(total / 4)) return nullptr;
     if (hipMalloc(&p, (size_t)size) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;

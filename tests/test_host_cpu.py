@@ -200,3 +200,17 @@ def test_batch_holds_a_bounded_number_of_graphs(host):
         B.run(36)
         assert host.captures() == start + 1 and host.execs() == 64
     assert host.execs() == 0
+
+
+def test_batch_takes_replicas_where_free_memory_is_not_known(host):
+    from spparks_amd import batch
+    with batch.Batch(64 << 20, 2) as B:
+        B.set_launch(256, 1024)
+        host.fail_info(1)
+        assert B.add(batch.replica_desc("potts", "sc/26n", 64, 64, 64, nspins=100, temperature=0.5, nsweeps=3)) == 0
+        host.log()
+        B.run(3)
+        assert "k_batch_slice" not in host.sweeps()
+    host.fail_info(2)   # the queue's pool, and the planes of its first solve
+    res, _ = batch.serve(mixed_queue(4), pool_bytes=1 << 30, max_live=4, block=256, grid=1024)
+    assert all(r["status"] == 0 for r in res)
