@@ -228,8 +228,10 @@ int spk_hip_last_timing(spk_hip_lattice *h, double *ms, int64_t *nlaunch);
    at that step; a replica's K*n passes of an n-sweep block (K/2*n of two colours
    where it sweeps on bit planes: sc/26n rows that fill at least half of 32-bit
    words) are spread evenly over the kind's steps, always in colour order 1..K.
-   Planes are held beside the pool, in memory taken while a quarter of the
-   device's stays free; a replica without them sweeps its spins.  Every replica's
+   Planes are held beside the pool, at most twice the bytes that their replicas
+   hold in it (in chunks of 64 MiB or one replica's), in memory taken while a quarter of
+   the device's stays free and given back, but for one chunk, as replicas go; a
+   replica without them sweeps its spins.  Every replica's
    trajectory is identical to running it alone (the strict sweep is
    decomposition independent), which the tests check.  Blocks after the
    first are replayed as HIP graphs.  No counterpart in the reference, which
@@ -250,7 +252,8 @@ typedef struct spk_hip_replica_desc {
 int spk_hip_batch_create(int64_t pool_bytes, int max_replicas, spk_hip_batch **out);
 void spk_hip_batch_destroy(spk_hip_batch *b);
 
-/* Bytes a replica of this description occupies in a pool (admission). */
+/* Bytes a replica of this description occupies in a pool (admission); planes
+   beside the pool are not counted. */
 int spk_hip_replica_bytes(const spk_hip_desc *d, int64_t *bytes);
 
 /* Admit a replica: allocate it in the pool and build its initial state on

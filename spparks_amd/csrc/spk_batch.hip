@@ -293,8 +293,9 @@ struct Shape {
 
 // Device memory for the planes of sliced replicas, beside the pool (whose
 // extents and admission are as for any replica): chunks taken as replicas need
-// them and given back with the batch.  A chunk is taken only while a quarter of
-// the device's memory stays free; a replica without one runs on its packed spins.
+// them.  A chunk is taken only while a quarter of the device's memory stays free; a
+// replica without one runs on its packed spins.  An empty chunk is given back,
+// but for one, which a queue's next solve takes again.
 class SideMemory {
  public:
   ~SideMemory() {
@@ -320,9 +321,23 @@ class SideMemory {
     chunks_.back()->alloc.alloc(n, &off);
     return p + off;
   }
+  // (nothing on the device may use [p, p + n) any more)
   void give(char *p, int64_t n) {
-    for (auto &c : chunks_)
-      if (p >= c->base && p < c->base + c->size) c->alloc.release(p - c->base, n);
+    bool spare = false;   // another chunk is empty
+    auto at = chunks_.end();
+    for (auto it = chunks_.begin(); it != chunks_.end(); ++it) {
+      Chunk &c = **it;
+      if (p >= c.base && p < c.base + c.size) {
+        c.alloc.release(p - c.base, n);
+        at = it;
+      } else {
+        spare |= c.alloc.used() == 0;
+      }
+    }
+    if (spare && at != chunks_.end() && (*at)->alloc.used() == 0) {
+      (void)hipFree((*at)->base);
+      chunks_.erase(at);
+    }
   }
 
  private:
@@ -847,6 +862,7 @@ int spk::batch_add_async(spk_hip_batch *b, const spk_hip_replica_desc *r, int *i
   if ((rc = check_hip(hipGetLastError(), "replica set-up launch")) ||
       (rc = replica_energy_async(b, slot, R))) {
     b->alloc->release(R.off, R.bytes);
+    (void)hipStreamSynchronize(b->stream);   // what was launched of it
     if (R.planes) b->side.give(reinterpret_cast<char *>(R.planes), R.side_bytes);
     return rc;
   }

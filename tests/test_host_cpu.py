@@ -214,3 +214,27 @@ def test_batch_takes_replicas_where_free_memory_is_not_known(host):
     host.fail_info(2)   # the queue's pool, and the planes of its first solve
     res, _ = batch.serve(mixed_queue(4), pool_bytes=1 << 30, max_live=4, block=256, grid=1024)
     assert all(r["status"] == 0 for r in res)
+
+
+def test_batch_gives_back_the_memory_of_planes(host):
+    """All but one of its chunks of 64 MiB (the first replica that comes again
+    finds its planes there), and that one with the batch."""
+    from spparks_amd import batch
+    base = host.device_bytes()
+    desc = batch.replica_desc("potts", "sc/26n", 128, 128, 128, nspins=1000, temperature=0.5, nsweeps=1)
+    with batch.Batch(256 << 20, 20) as B:
+        B.set_launch(256, 1024)
+        empty = host.device_bytes()
+        ids = [B.add(desc) for _ in range(16)]      # 12 MiB of planes and seeds each: 5 a chunk
+        B.run(1)
+        held = host.device_bytes()
+        assert held - empty >= 4 * (64 << 20)
+        for rid in ids[::2] + ids[1::2]:
+            B.remove(rid)
+        assert held - host.device_bytes() == 3 * (64 << 20)
+        calls = host.device_calls()
+        host.log()
+        B.add(desc)
+        B.run(1)
+        assert "k_batch_slice" in host.sweeps() and host.device_calls() == calls
+    assert host.device_bytes() == base
