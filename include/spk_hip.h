@@ -283,8 +283,8 @@ int spk_hip_batch_trace(spk_hip_batch *b, int id, int n, int64_t *naccept, doubl
 /* Launch shape of the step kernels of replicas that are not on bit planes (those
    have a wavefront for every tile): block = threads per workgroup (64..1024,
    multiple of 64), grid = persistent workgroups.  0, 0 = autotune: the next
-   run times candidate shapes on its own steps (results do not depend on the
-   shape) and keeps the fastest. */
+   run with such replicas times candidate shapes on its own steps (results do not
+   depend on the shape) and keeps the fastest. */
 int spk_hip_batch_set_launch(spk_hip_batch *b, int block, int grid);
 
 /* Last run: device milliseconds between events around its steps, site

@@ -401,7 +401,8 @@ struct spk_hip_batch {
   hipStream_t vstream[kNumVariants] = {};
   hipEvent_t fork_ev = nullptr, join_ev[kNumVariants] = {};
   // launch shape
-  int block = 0, grid = 0;          // 0 = autotune on the next run
+  int block = 0, grid = 0;
+  bool tune = true;                 // choose them on the next run that has packed spins to sweep
   // recorded blocks, at most kMaxGraphs of them
   struct Recorded {
     std::vector<int> key;   // block, grid, then v and L of each variant
@@ -963,12 +964,14 @@ int spk_hip_batch_set_launch(spk_hip_batch *b, int block, int grid) {
   if (!b) return set_error(SPK_HIP_EINVAL, "null batch");
   if (block == 0 && grid == 0) {
     b->block = b->grid = 0;
+    b->tune = true;
     return SPK_HIP_OK;
   }
   if (block < 64 || block > 1024 || block % 64 || grid < 1)
     return set_error(SPK_HIP_EINVAL, "block must be a multiple of 64 in [64,1024] and grid >= 1");
   b->block = block;
   b->grid = (grid + kNumXcd - 1) / kNumXcd * kNumXcd;
+  b->tune = false;
   return SPK_HIP_OK;
 }
 
@@ -1010,13 +1013,23 @@ static void apply_rows(spk_hip_batch *b) {
   }
 }
 
+// Whether the next block is to choose the launch shape: one that has replicas
+// on packed spins (k_batch_slice has its own grid, so a block of nothing else has
+// nothing to try).
+bool batch_tunes(const spk_hip_batch *b) {
+  if (!b->tune) return false;
+  for (auto &R : b->reps)
+    if (R.live && R.variant != kSliceVariant && R.done < R.desc.nsweeps) return true;
+  return false;
+}
+
 // Queues one block (every replica with sweeps left advances by up to
 // max_sweeps) with the launch shape already set, and returns without
 // waiting.  Work queued on the batch stream afterwards (admissions,
 // checksums) runs after the block.
 int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph) {
   if (b->inflight) return set_error(SPK_HIP_ESTATE, "a block is already in flight");
-  if (b->block == 0) return set_error(SPK_HIP_ESTATE, "no launch shape set");
+  if (b->block == 0 && batch_tunes(b)) return set_error(SPK_HIP_ESTATE, "no launch shape set");
   int rc;
   int L = 0, rows = 0;
   int64_t updates = 0;
@@ -1025,6 +1038,10 @@ int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph) {
   b->last_nlaunch = block_launches(b);
   b->last_ms = 0.0;
   if (L == 0) return SPK_HIP_OK;
+  if (b->block == 0) {   // all on planes, which the shape does not concern
+    b->block = kSliceBlock;
+    b->grid = std::max(kNumXcd, b->ncu * 4 / kNumXcd * kNumXcd);
+  }
   if ((rc = ensure_events(b, 2 * (size_t)L + 2)) || (rc = ensure_streams(b)) ||
       (rc = upload_schedule(b, rows, true)))
     return rc;
@@ -1128,7 +1145,7 @@ int spk_hip_batch_run(spk_hip_batch *b, int max_sweeps, int use_graph) {
   if (max_sweeps <= 0) return set_error(SPK_HIP_EINVAL, "max_sweeps must be positive");
   int rc;
   if ((rc = batch_complete(b))) return rc;
-  if (b->block != 0) {
+  if (!batch_tunes(b)) {
     if ((rc = batch_launch(b, max_sweeps, use_graph != 0))) return rc;
     return batch_complete(b);
   }
@@ -1145,82 +1162,79 @@ int spk_hip_batch_run(spk_hip_batch *b, int max_sweeps, int use_graph) {
   if ((rc = ensure_events(b, 2 * (size_t)L + 2)) || (rc = ensure_streams(b)) ||
       (rc = upload_schedule(b, rows, true)))
     return rc;
-  if (b->block == 0) {
-    // autotune: candidate shapes (workgroup size x wavefronts per CU) run
-    // the block's own steps, as a replay runs them (no wait between steps);
-    // results do not depend on the shape.  The tile list is the same for
-    // every shape (a tile is one wavefront's work).
-    // (k_batch_slice has its own grid: a block of nothing else has nothing to try)
-    std::vector<Shape> cand;
-    const bool only_sliced = b->variants.size() == 1 && b->variants[0].v == kSliceVariant;
-    for (int bs : only_sliced ? std::vector<int>{256} : std::vector<int>{64, 128, 256})
-      for (int wpc : only_sliced ? std::vector<int>{16} : std::vector<int>{8, 16, 32}) {
-        const int grid = std::max(kNumXcd, b->ncu * wpc * 64 / bs / kNumXcd * kNumXcd);
-        cand.push_back(Shape{bs, grid});
-      }
-    auto step_work = [&](int j) {   // sites updated in step j
-      double w = 0.0;
-      for (const auto &var : b->variants) {
-        const int at = (int)(((int64_t)j * var.L) / L);
-        if (at == (int)(((int64_t)(j + 1) * var.L) / L)) continue;
-        const StepDesc &sd = b->h_steps[var.first + at];
-        for (int a = 0; a < sd.count; a++) w += (double)b->h_reps[b->h_act[sd.first + a]].g.M;
-      }
-      return w;
-    };
-    const int C = (int)cand.size();
-    // each candidate gets whole sweeps (of the replica with most steps) when
-    // the block has room, else single steps in turn
-    int sweeps = 1;
-    for (const auto &R : b->reps) sweeps = std::max(sweeps, R.live ? R.block_sweeps : 0);
-    const int unit = std::max(1, L / sweeps);
-    const int per = L / C >= unit ? L / C / unit * unit : 1;
-    std::vector<double> t_ms(C, 0.0), work(C, 0.0);
-    double tot = 0.0;
-    int j = 0;
-    auto timed = [&](int j0, int j1, const Shape &sh, double *ms_out) -> int {
-      int rc;
-      if ((rc = check_hip(hipEventRecord(b->events[0], b->stream), "event")) ||
-          (rc = launch_steps(b, j0, j1, L, sh.block, sh.grid)) ||
-          (rc = check_hip(hipEventRecord(b->events[1], b->stream), "event")) ||
-          (rc = check_hip(hipStreamSynchronize(b->stream), "tune sync")))
-        return rc;
-      float ms = 0.f;
-      if ((rc = check_hip(hipEventElapsedTime(&ms, b->events[0], b->events[1]), "event time"))) return rc;
-      *ms_out = ms;
-      return SPK_HIP_OK;
-    };
-    auto trial = [&](int c) -> int {   // candidate c takes the next `per` steps
-      const int j1 = std::min(L, j + per);
-      double ms = 0.0;
-      const int rc = timed(j, j1, cand[c], &ms);
-      if (rc) return rc;
-      for (int q = j; q < j1; q++) work[c] += step_work(q);
-      t_ms[c] += ms;
-      tot += ms;
-      j = j1;
-      return SPK_HIP_OK;
-    };
-    if (per > 1) {
-      for (int c = 0; c < C; c++)
+  // autotune: candidate shapes (workgroup size x wavefronts per CU) run
+  // the block's own steps, as a replay runs them (no wait between steps);
+  // results do not depend on the shape.  The tile list is the same for
+  // every shape (a tile is one wavefront's work).
+  std::vector<Shape> cand;
+  for (int bs : {64, 128, 256})
+    for (int wpc : {8, 16, 32}) {
+      const int grid = std::max(kNumXcd, b->ncu * wpc * 64 / bs / kNumXcd * kNumXcd);
+      cand.push_back(Shape{bs, grid});
+    }
+  auto step_work = [&](int j) {   // sites updated in step j
+    double w = 0.0;
+    for (const auto &var : b->variants) {
+      const int at = (int)(((int64_t)j * var.L) / L);
+      if (at == (int)(((int64_t)(j + 1) * var.L) / L)) continue;
+      const StepDesc &sd = b->h_steps[var.first + at];
+      for (int a = 0; a < sd.count; a++) w += (double)b->h_reps[b->h_act[sd.first + a]].g.M;
+    }
+    return w;
+  };
+  const int C = (int)cand.size();
+  // each candidate gets whole sweeps (of the replica with most steps) when
+  // the block has room, else single steps in turn
+  int sweeps = 1;
+  for (const auto &R : b->reps) sweeps = std::max(sweeps, R.live ? R.block_sweeps : 0);
+  const int unit = std::max(1, L / sweeps);
+  const int per = L / C >= unit ? L / C / unit * unit : 1;
+  std::vector<double> t_ms(C, 0.0), work(C, 0.0);
+  double tot = 0.0;
+  int j = 0;
+  auto timed = [&](int j0, int j1, const Shape &sh, double *ms_out) -> int {
+    int rc;
+    if ((rc = check_hip(hipEventRecord(b->events[0], b->stream), "event")) ||
+        (rc = launch_steps(b, j0, j1, L, sh.block, sh.grid)) ||
+        (rc = check_hip(hipEventRecord(b->events[1], b->stream), "event")) ||
+        (rc = check_hip(hipStreamSynchronize(b->stream), "tune sync")))
+      return rc;
+    float ms = 0.f;
+    if ((rc = check_hip(hipEventElapsedTime(&ms, b->events[0], b->events[1]), "event time"))) return rc;
+    *ms_out = ms;
+    return SPK_HIP_OK;
+  };
+  auto trial = [&](int c) -> int {   // candidate c takes the next `per` steps
+    const int j1 = std::min(L, j + per);
+    double ms = 0.0;
+    const int rc = timed(j, j1, cand[c], &ms);
+    if (rc) return rc;
+    for (int q = j; q < j1; q++) work[c] += step_work(q);
+    t_ms[c] += ms;
+    tot += ms;
+    j = j1;
+    return SPK_HIP_OK;
+  };
+  if (per > 1) {
+    for (int c = 0; c < C; c++)
+      if ((rc = trial(c))) return rc;
+  } else {
+    while (j < L)
+      for (int c = 0; c < C && j < L; c++)
         if ((rc = trial(c))) return rc;
-    } else {
-      while (j < L)
-        for (int c = 0; c < C && j < L; c++)
-          if ((rc = trial(c))) return rc;
-    }
-    int best = 0;
-    for (int c = 1; c < C; c++)
-      if (work[c] / std::max(t_ms[c], 1e-9) > work[best] / std::max(t_ms[best], 1e-9)) best = c;
-    b->block = cand[best].block;
-    b->grid = cand[best].grid;
-    if (j < L) {   // the steps after the trial chunks run with the winner
-      double ms = 0.0;
-      if ((rc = timed(j, L, cand[best], &ms))) return rc;
-      tot += ms;
-    }
-    b->last_ms = tot;
   }
+  int best = 0;
+  for (int c = 1; c < C; c++)
+    if (work[c] / std::max(t_ms[c], 1e-9) > work[best] / std::max(t_ms[best], 1e-9)) best = c;
+  b->block = cand[best].block;
+  b->grid = cand[best].grid;
+  b->tune = false;
+  if (j < L) {   // the steps after the trial chunks run with the winner
+    double ms = 0.0;
+    if ((rc = timed(j, L, cand[best], &ms))) return rc;
+    tot += ms;
+  }
+  b->last_ms = tot;
   if ((rc = queue_rows(b, rows)) || (rc = check_hip(hipStreamSynchronize(b->stream), "readback sync")))
     return rc;
   apply_rows(b);

@@ -12,6 +12,8 @@ namespace spk {
 // Admits a replica; its set-up and initial energy are queued on the batch
 // stream (after a block in flight) and nothing waits.
 int batch_add_async(spk_hip_batch *b, const spk_hip_replica_desc *r, int *id);
+// Whether the next block is to choose the launch shape (spk_hip_batch_run does).
+bool batch_tunes(const spk_hip_batch *b);
 // Queues one block with the launch shape already set; returns at once.
 int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph);
 // Waits for everything queued on the batch stream; applies the per-sweep

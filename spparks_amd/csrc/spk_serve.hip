@@ -68,7 +68,6 @@ extern "C" int spk_hip_serve(const spk_hip_request *req, int n, int64_t pool_byt
   int rc = queue_pool(req, n, pool_bytes, &pool_bytes);
   if (rc || (rc = spk_hip_batch_create(pool_bytes, max_live, &g.b))) return rc;
   if ((rc = spk_hip_batch_set_launch(g.b, block, grid))) return rc;
-  bool tuned = block != 0;   // a zero shape is tuned on the first block, which waits
 
   std::vector<int> owner(max_live, -1);   // replica id -> request index
   std::deque<int> waiting;                // arrived, not yet admitted (FIFO)
@@ -125,10 +124,10 @@ extern "C" int spk_hip_serve(const spk_hip_request *req, int n, int64_t pool_byt
     finishing.clear();
     for (int id = 0; id < max_live; id++)
       if (owner[id] >= 0 && batch_left(g.b, id) <= block_sweeps) finishing.push_back(id);
-    if (!tuned) {
-      // the first block tunes the launch shape on its own steps and waits
+    if (batch_tunes(g.b)) {
+      // a zero shape is tuned on the steps of the first block that it concerns,
+      // which waits
       if ((rc = spk_hip_batch_run(g.b, block_sweeps, 1))) return rc;
-      tuned = true;
     } else if ((rc = batch_launch(g.b, block_sweeps, true))) {
       return rc;
     }

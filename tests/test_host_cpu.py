@@ -238,3 +238,36 @@ def test_batch_gives_back_the_memory_of_planes(host):
         B.run(1)
         assert "k_batch_slice" in host.sweeps() and host.device_calls() == calls
     assert host.device_bytes() == base
+
+
+def shapes_tried(host):
+    """Launch shapes of the batched kernel of packed spins since the last log."""
+    return len({(g, b) for n, g, b in host.log() if n.startswith("k_batch_step")})
+
+
+def test_launch_shape_is_tuned_on_packed_spins(host):
+    """A block of replicas on planes only has no shape to choose: the next one with
+    packed spins does, in a batch and in a queue."""
+    from spparks_amd import batch
+    planes = batch.replica_desc("potts", "sc/26n", 64, 64, 64, nspins=100, temperature=0.5, nsweeps=60)
+    packed = batch.replica_desc("potts", "sq/8n", 64, 64, nspins=100, temperature=0.5, nsweeps=60)
+    with batch.Batch(64 << 20, 4) as B:
+        B.run(5)
+        assert B.last_timing()["block"] == 0
+        B.add(planes)
+        host.log()
+        B.run(5)
+        assert shapes_tried(host) == 0 and B.last_timing()["block"] > 0
+        B.add(packed)
+        B.run(20)
+        assert shapes_tried(host) == 9
+        B.run(20)
+        assert shapes_tried(host) == 1
+        B.set_launch(0, 0)
+        B.run(20)
+        assert shapes_tried(host) == 9
+    reqs = [{"app": "potts", "lattice": l, "shape": s, "nspins": 100, "kT": 0.5, "seed": 1, "sweeps": 100, "arrive": t}
+            for l, s, t in (("sc/26n", (64, 64, 64), 0.0), ("sq/8n", (64, 64, 1), 0.0))]
+    res, _ = batch.serve(reqs, pool_bytes=batch.replica_bytes("potts", "sc/26n", 64, 64, 64, 100), max_live=4,
+                         block_sweeps=20)      # one after the other
+    assert all(r["status"] == 0 for r in res) and shapes_tried(host) == 9
