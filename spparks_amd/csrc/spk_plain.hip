@@ -729,7 +729,8 @@ void tile_choose(spk_hip_lattice *h) {
     }
 }
 
-// Which kernels a sweeps call of a lattice beyond one workgroup's reach takes.
+// Which kernels a sweeps call of a lattice beyond one workgroup's reach takes
+// (enter_route: a single sweep may take another).
 Route route(spk_hip_lattice *h) {
   if (!h->tile_known) tile_choose(h);
   if (h->tile.sweeps > 0) return kRouteTile;
@@ -873,10 +874,18 @@ bool ensure_tile_buffers(spk_hip_lattice *h) {
   return h->spin2 != nullptr;
 }
 
-// Brings the state to the layout the next sweeps run on: the bit planes, or
+// Lattices of boxes that make a call of one sweep one colour a launch (from
+// the host, as boxes are): boxes would take two launches whatever their size,
+// each with its halo.  us a call, boxes and colours: sc/6n 16 x 14 x 92 30, 27; sq/4n
+// 692 x 580 33, 28, 5126 x 220 41, 31, 234 x 9944 46, 31; sq/8n 1156 x 380 34, 47, 1066 x
+// 1402 40, 47, 390 x 6628 56, 49, 1174 x 4090 61, 49.
+bool tile_single(const spk_hip_lattice *h) { return h->g.K == 2 || (h->g.K == 4 && h->N > 7 << 18); }
+
+// Brings the state to the layout the next n sweeps run on: the bit planes, or
 // the bytes.
-int enter_route(spk_hip_lattice *h, Route *out) {
+int enter_route(spk_hip_lattice *h, int n, Route *out) {
   Route rt = route(h);
+  if (rt == kRouteTile && n == 1 && tile_single(h)) rt = kRouteColour;
   if (rt == kRouteTile && !ensure_tile_buffers(h)) rt = route(h);
   *out = rt;
   if (rt == kRouteBits) return h->bits_active ? SPK_HIP_OK : bits_enter(h);
@@ -890,6 +899,9 @@ int enter_route(spk_hip_lattice *h, Route *out) {
   }
   return bits_leave(h);
 }
+
+// Whether sweeps off the boxes are replayed from graphs (tile_single's are not).
+bool replayed(const spk_hip_lattice *h) { return h->chunk > 0 && h->tile.sweeps == 0; }
 
 int ensure_pinned(spk_hip_lattice *h, int rows) {
   if (rows <= h->pinned_rows) return SPK_HIP_OK;
@@ -1463,7 +1475,7 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
   }
   // (on the bit planes the state stays there)
   Route rt;
-  if ((rc = enter_route(h, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
+  if ((rc = enter_route(h, nsweeps, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
   // rows [0, n) cleared
   auto clear = [&](int n) {
     const int64_t words = (int64_t)n * kAccRow;
@@ -1482,7 +1494,7 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
         return rc;
       done += n;
     }
-  } else if (h->chunk > 0) {
+  } else if (replayed(h)) {
     // graph replays (graph_pieces); each piece's rows are folded into the
     // pinned rows [done, done + n) before the next piece clears them
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
@@ -1538,10 +1550,10 @@ int spk_hip_prepare(spk_hip_lattice *h, int nsweeps) {
   if (nsweeps == 0 || resident_call(h, nsweeps)) return SPK_HIP_OK;
   int rc;
   Route rt;
-  if ((rc = enter_route(h, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
+  if ((rc = enter_route(h, nsweeps, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
   if (rt == kRouteTile) {
     if ((rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows)))) return rc;
-  } else if (h->chunk > 0) {
+  } else if (replayed(h)) {
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
     if ((rc = ensure_acc(h, pieces[0]))) return rc;
     for (int n : pieces) {

@@ -271,3 +271,27 @@ def test_launch_shape_is_tuned_on_packed_spins(host):
     res, _ = batch.serve(reqs, pool_bytes=batch.replica_bytes("potts", "sc/26n", 64, 64, 64, 100), max_live=4,
                          block_sweeps=20)      # one after the other
     assert all(r["status"] == 0 for r in res) and shapes_tried(host) == 9
+
+
+@pytest.mark.parametrize("case,single", [
+    (("ising", "sq/4n", (692, 580, 1), 2), True),
+    (("ising", "sq/4n", (362, 5944, 1), 2), True),
+    (("potts", "sc/6n", (16, 128, 196), 255), True),
+    (("potts", "sq/8n", (600, 500, 1), 100), False),
+    (("potts", "sq/8n", (1174, 4090, 1), 100), True),
+    (("potts", "sc/26n", (64, 64, 64), 1000), False),
+], ids=lambda v: v[1] + "-" + "x".join(map(str, v[2])) if isinstance(v, tuple) else None)
+def test_single_sweep_of_boxes_goes_one_colour_a_launch_where_that_is_faster(host, case, single):
+    with lattice(*case) as L:
+        k = {"sq/4n": 2, "sc/6n": 2, "sq/8n": 4, "sc/26n": 8}[case[1]]
+        L.energy()
+        captures = host.captures()
+        for n in (1, 2, 3, 1):
+            L.prepare(n)
+            host.log()
+            L.sweeps(n)
+            if n == 1 and single:
+                assert host.sweeps() == ["k_sweep_color"] * (k * n) and L.last_timing()[1] == k * n
+            else:
+                assert set(host.sweeps()) == {"k_sweep_tile"}
+        assert host.captures() == captures
