@@ -580,9 +580,18 @@ double pair_sweep_us(const spk_hip_lattice *h) {
   const int band = pair_band(h->g), rounds = ((h->g.hy + band - 1) / band + kCus - 1) / kCus;
   // band rows of the four passes, wavefronts a row, their time a row
   const double rows = 4 * band + 12, waves = pair_stage((h->g.hx + 31) / 32) / 64;
-  const double us = h->d.app == SPK_HIP_ISING_SINGLE ? 0.085 : 0.105;
+  double us = h->d.app == SPK_HIP_ISING_SINGLE ? 0.085 : 0.105;
+  // bands that wait for a compute unit, of rows that fill one wavefront a group:
+  // 1.0 to 1.28 of that time
+  if (rounds > 1 && waves == 1) us *= 1.28;
   return (5.0 + rounds * rows * waves * us) / 2;
 }
+
+// Two sweeps a launch on bit planes where that is faster (of 160 lattices two are on
+// the slower side, by 3 and 6%).  us a sweep, one colour a launch and two sweeps a launch:
+// ising/single 44 x 4748 8.6, 9.7; 834 x 8680 13.6, 14.7; 558 x 9782 12.6, 14.9;
+// 1580 x 5552 17.8, 15.7; Ising 1404 x 7722 23.5, 20.8
+bool pair_pays(const spk_hip_lattice *h) { return pair_fits(h->g) && pair_sweep_us(h) < colour_bits_us(h); }
 
 // Microseconds a sweep is expected to take through the kernels that pass
 // over the lattice one colour at a time (bit planes where they apply) or in
@@ -595,7 +604,7 @@ double plain_sweep_us(const spk_hip_lattice *h) {
     return h->g.K * (0.25 + std::max(1.0, waves / kSimds) * 4 * site_valu(h) * kUsPerValu * 1.2);
   }
   if (bits_eligible(h))
-    return h->bitplanes == 1 && pair_fits(h->g) ? std::min(pair_sweep_us(h), colour_bits_us(h)) : colour_bits_us(h);
+    return h->bitplanes == 1 && pair_pays(h) ? pair_sweep_us(h) : colour_bits_us(h);
   if (slice_eligible(h)) {
     // a wavefront's own time, and what a launch adds as its wavefronts fill
     // the SIMDs (22 to 31 us a sweep for 1 to 5 plane groups up to 128^3, 41
@@ -772,7 +781,7 @@ int ensure_planes(uint32_t *&p, const spk_hip_lattice *h) {
 }
 
 int bits_enter(spk_hip_lattice *h) {
-  h->pairs = h->pairs_ok && h->bitplanes == 1 && pair_fits(h->g) && pair_sweep_us(h) < colour_bits_us(h);
+  h->pairs = h->pairs_ok && h->bitplanes == 1 && pair_pays(h);
   h->bg = bit_geom(h->g, h->pairs ? 8 : h->bitplanes == 1 ? kBitSites : h->bitplanes);
   int rc;
   if ((rc = ensure_planes(h->bits, h)) || (rc = ensure_shadow(h, h->sseed, h->sseed_cap, 2 * h->bg.seedc)))

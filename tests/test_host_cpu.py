@@ -295,3 +295,19 @@ def test_single_sweep_of_boxes_goes_one_colour_a_launch_where_that_is_faster(hos
             else:
                 assert set(host.sweeps()) == {"k_sweep_tile"}
         assert host.captures() == captures
+
+
+@pytest.mark.parametrize("app,shape,pairs", [
+    ("ising/single", (44, 4748, 1), False),     # bands in rounds on the compute units
+    ("ising/single", (834, 8680, 1), False),
+    ("ising/single", (558, 9782, 1), False),
+    ("ising/single", (1580, 5552, 1), True),
+    ("ising", (1404, 7722, 1), True),
+    ("ising", (4096, 4096, 1), True),
+])
+def test_two_sweeps_a_launch_where_that_is_faster(host, app, shape, pairs):
+    with lattice(app, "sq/4n", shape, 2, 2.269) as L:
+        host.log()
+        L.sweeps(4)
+        names = set(host.sweeps())
+        assert pairs == ("k_sweep_bits_pair" in names), names
