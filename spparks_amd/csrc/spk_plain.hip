@@ -535,13 +535,16 @@ double site_valu(const spk_hip_lattice *h) {
   return h->stype == kU8 ? 45 + 3.3 * nn : h->stype == kU16 ? 66 + 2.5 * nn : 60 + 4.5 * nn;
 }
 
+// potts/neigh and potts/neighonly
+bool first_appearance(const spk_hip_lattice *h) { return variant_app(h->d.app) && h->d.app != SPK_HIP_ISING_SINGLE; }
+
 // The same for the tile kernel's one-site events.
 double tile_site_valu(const spk_hip_lattice *h) {
   const int nn = maxneigh_of(h->g.lat);
   // the first-appearance rules compare every pair of neighbours, each
   // compare's mask through the scalar unit (counted as their time, not only
   // their instructions: 5.2 us a pass of sc/26n with one wavefront a SIMD)
-  if (variant_app(h->d.app) && h->d.app != SPK_HIP_ISING_SINGLE) return 75 + 8.0 * nn + 1.9 * nn * nn;
+  if (first_appearance(h)) return 75 + 8.0 * nn + 1.9 * nn * nn;
   return h->rule.nspins == 2 ? 70 + 2.0 * nn : 75 + 5.0 * nn;
 }
 
@@ -582,8 +585,8 @@ double pair_sweep_us(const spk_hip_lattice *h) {
   const double rows = 4 * band + 12, waves = pair_stage((h->g.hx + 31) / 32) / 64;
   double us = h->d.app == SPK_HIP_ISING_SINGLE ? 0.085 : 0.105;
   // bands that wait for a compute unit, of rows that fill one wavefront a group:
-  // 1.0 to 1.28 of that time
-  if (rounds > 1 && waves == 1) us *= 1.28;
+  // 1.0 to 1.3 of that time
+  if (rounds > 1 && waves == 1) us *= 1.3;
   return (5.0 + rounds * rows * waves * us) / 2;
 }
 
@@ -665,6 +668,9 @@ double tile_sweep_us(const spk_hip_lattice *h, const int (&w)[3], int S, int vec
     const double waves = (items[k] + 63) / 64, turns = (items[k] + threads - 1) / threads;
     us += 0.3 + std::max(turns * (0.15 + 1.3 * item_us), 1.2 * together * waves / kSimds * item_us);
   }
+  // (a site a thread: 1.05 to 1.4 of that in 900 lattices, but for the
+  // first-appearance rules' 0.9 to 1.3; packs 0.8 to 1.2)
+  if (vec == 1 && !first_appearance(h)) us *= 1.15;
   us = (5.0 + rounds * us) / S;
   if (us >= best) return 1e30;
   *shape = TileShape{{w[0], w[1], w[2]}, S, vec, block};
@@ -693,8 +699,12 @@ void tile_choose(spk_hip_lattice *h) {
   if (h->g.lat == SPK_HIP_SQ_4N && h->rule.nspins == 2 && h->stype == kU8 && h->bitplanes != 1) return;
   if (h->N > (int64_t)8 << 20 || !offsets_fit_32(h->g)) return;
   // the gain the model can be trusted with (within a fifth of the measured
-  // time from 64^2 to 2000^2 and 128^3)
-  double best = (resident_bytes(h) ? 0.75 : slice_eligible(h) ? 0.85 : 0.9) * plain_sweep_us(h);
+  // time): of 2000 lattices of 2000 to 8 * 10^6 sites four are slower in boxes, by 4 to 9%
+  double best = (resident_bytes(h)                    ? 0.86
+                 : slice_eligible(h)                  ? 0.93
+                 : h->d.app == SPK_HIP_ISING_SINGLE   ? 0.97
+                                                      : 0.9) *
+                plain_sweep_us(h);
   auto sizes = [](int n, int unit) {   // extents that cut n into near-equal boxes
     std::vector<int> v;
     for (int cuts : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64}) {

@@ -311,3 +311,19 @@ def test_two_sweeps_a_launch_where_that_is_faster(host, app, shape, pairs):
         L.sweeps(4)
         names = set(host.sweeps())
         assert pairs == ("k_sweep_bits_pair" in names), names
+
+
+@pytest.mark.parametrize("case,boxes", [
+    # sites a thread against packs, and boxes against one colour a launch
+    (("ising", "sc/6n", (178, 18, 128), 2), False),
+    (("potts", "sc/6n", (138, 16, 132), 100), False),
+    (("ising/single", "sq/4n", (6776, 346, 1), 2), False),
+    (("ising", "sc/6n", (16, 104, 154), 2), True),
+    (("potts", "sq/8n", (128, 128, 1), 100), True),
+    (("potts", "sc/26n", (64, 64, 64), 100000), True),
+], ids=lambda v: v[1] + "-" + "x".join(map(str, v[2])) if isinstance(v, tuple) else None)
+def test_boxes_where_they_are_faster(host, case, boxes):
+    with lattice(*case) as L:
+        host.log()
+        L.sweeps(24)
+        assert boxes == ("k_sweep_tile" in host.sweeps())
