@@ -919,8 +919,13 @@ int enter_route(spk_hip_lattice *h, int n, Route *out) {
   return bits_leave(h);
 }
 
-// Whether sweeps off the boxes are replayed from graphs (tile_single's are not).
-bool replayed(const spk_hip_lattice *h) { return h->chunk > 0 && h->tile.sweeps == 0; }
+int64_t sweep_launches(const spk_hip_lattice *h, int n);
+// Whether n sweeps off the boxes are replayed from graphs (tile_single's are
+// not).  Two launches are soon made: a call of one sweep took 42 us replayed and 33 so
+// on 150 x 130 x 110 sc/6n, 43 and 34 on 410 x 7614 sq/4n, 58 and 48 on 4096^2 Ising.
+bool replayed(const spk_hip_lattice *h, int n) {
+  return h->chunk > 0 && h->tile.sweeps == 0 && sweep_launches(h, n) > 2;
+}
 
 int ensure_pinned(spk_hip_lattice *h, int rows) {
   if (rows <= h->pinned_rows) return SPK_HIP_OK;
@@ -1513,7 +1518,7 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
         return rc;
       done += n;
     }
-  } else if (replayed(h)) {
+  } else if (replayed(h, nsweeps)) {
     // graph replays (graph_pieces); each piece's rows are folded into the
     // pinned rows [done, done + n) before the next piece clears them
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
@@ -1572,7 +1577,7 @@ int spk_hip_prepare(spk_hip_lattice *h, int nsweeps) {
   if ((rc = enter_route(h, nsweeps, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
   if (rt == kRouteTile) {
     if ((rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows)))) return rc;
-  } else if (replayed(h)) {
+  } else if (replayed(h, nsweeps)) {
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
     if ((rc = ensure_acc(h, pieces[0]))) return rc;
     for (int n : pieces) {

@@ -327,3 +327,16 @@ def test_boxes_where_they_are_faster(host, case, boxes):
         host.log()
         L.sweeps(24)
         assert boxes == ("k_sweep_tile" in host.sweeps())
+
+
+def test_calls_of_two_launches_capture_no_graph(host):
+    with lattice("potts", "sc/6n", (150, 130, 110), 50) as L:
+        captures = host.captures()
+        for _ in range(3):
+            L.prepare(1)
+            host.log()
+            L.sweeps(1)
+            assert host.sweeps() == ["k_sweep_color"] * 2
+        assert host.captures() == captures
+        L.sweeps(2)
+        assert host.captures() == captures + 1
