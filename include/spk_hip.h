@@ -205,8 +205,9 @@ int spk_hip_set_resident(spk_hip_lattice *h, int enable);
    graph is captured on first use and kept until a setting that changes the
    launches (set_launch, set_bitplanes, set_temperature, set_graph) drops
    the cache.  chunk_sweeps = 0 launches every kernel from the host, as calls
-   of no more than two launches and lattices in boxes (set_launch) or one
-   workgroup (set_resident) always do.
+   of no more than two launches and lattices in boxes (set_launch; but for long
+   calls of potts/neigh and potts/neighonly on sc/26n) or one workgroup
+   (set_resident) always do.
    Results are identical either way. */
 int spk_hip_set_graph(spk_hip_lattice *h, int chunk_sweeps);
 

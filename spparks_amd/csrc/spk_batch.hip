@@ -615,7 +615,8 @@ constexpr size_t kMaxGraphs = 64;
 // sizes in an octave, so that a queue whose tiles change with every solve does not
 // have every block recorded.  The surplus workgroups leave at once.  300 mixed solves,
 // 16 live, 5 sweeps a block: 134 blocks took 121 ms with most of them recorded (49 ms
-// of steps), 86 with 11 graphs.
+// of steps), 90 with 18 graphs (and the surplus workgroups
+// of an ensemble of few sliced replicas, recorded so at once, cost it 2%).
 int recorded_grid(int need) {
   if (need == 0) return 0;
   int unit = kSliceResident / 4;
@@ -1057,8 +1058,7 @@ int batch_launch(spk_hip_batch *b, int max_sweeps, bool use_graph) {
     // a graph recorded for more workgroups serves, up to half as many again:
     // a queue of solves changes its tiles with every one that comes or goes
     spk_hip_batch::Recorded *rec = nullptr;
-    // to record with: an ensemble that keeps its replicas has no use for more
-    int slice_grid = need ? std::max(need, kSliceResident) : 0;
+    int slice_grid = need;   // to record with: an ensemble that keeps its replicas has no use for more
     for (auto &r : b->graphs) {
       if (r.key != key) continue;
       slice_grid = recorded_grid(need);

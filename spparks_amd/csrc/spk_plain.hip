@@ -919,12 +919,17 @@ int enter_route(spk_hip_lattice *h, int n, Route *out) {
   return bits_leave(h);
 }
 
-int64_t sweep_launches(const spk_hip_lattice *h, int n);
-// Whether n sweeps off the boxes are replayed from graphs (tile_single's are
-// not).  Two launches are soon made: a call of one sweep took 42 us replayed and 33 so
-// on 150 x 130 x 110 sc/6n, 43 and 34 on 410 x 7614 sq/4n, 58 and 48 on 4096^2 Ising.
-bool replayed(const spk_hip_lattice *h, int n) {
-  return h->chunk > 0 && h->tile.sweeps == 0 && sweep_launches(h, n) > 2;
+int64_t sweep_launches(const spk_hip_lattice *h, int n, Route route);
+// Whether n sweeps are replayed from graphs.  Two launches are soon made: a
+// call of one sweep took 42 us replayed and 33 so on 150 x 130 x 110 sc/6n, 43 and
+// 34 on 410 x 7614 sq/4n, 58 and 48 on 4096^2 Ising.  Boxes (and tile_single's colours)
+// are launched from the host (launch_tiles), but for long calls of the first-appearance
+// rules on sc/26n, whose launches take 45 us and more: 24 sweeps of 92 x 32 x 44 1183 us
+// replayed, 1201 launched.
+bool replayed(const spk_hip_lattice *h, int n, Route route) {
+  if (h->chunk == 0) return false;
+  if (route == kRouteTile) return first_appearance(h) && h->g.K == 8 && sweep_launches(h, n, route) >= 8;
+  return h->tile.sweeps == 0 && sweep_launches(h, n, route) > 2;
 }
 
 int ensure_pinned(spk_hip_lattice *h, int rows) {
@@ -963,7 +968,9 @@ int launch_pair(spk_hip_lattice *h, int from, unsigned long long *acc) {
 }
 
 // Sweep-kernel launches that launch_sweeps makes for n sweeps.
-int64_t sweep_launches(const spk_hip_lattice *h, int n) {
+int tile_launches(const spk_hip_lattice *h, int n);
+int64_t sweep_launches(const spk_hip_lattice *h, int n, Route route) {
+  if (route == kRouteTile) return tile_launches(h, n);
   if (h->slice_active) return (int64_t)h->g.K / 2 * n;
   if (h->bits_active && h->pairs) return 2 * (n / 4) + (int64_t)h->g.K * (n % 4);
   return (int64_t)h->g.K * n;
@@ -1012,7 +1019,7 @@ int launch_tile(spk_hip_lattice *h, int from, int q0, int q1, unsigned long long
 
 // n sweeps through the tile kernel, split evenly over its launches: whole
 // sweeps each, or (one sweep, or one sweep a launch and an odd number of
-// them) at colours inside a sweep.  Launched one by one, never captured: the
+// them) at colours inside a sweep.  Launched one by one rather than captured (replayed): the
 // device takes longer over a launch than the host, and a graph for each number of
 // sweeps and each temperature cost 70 us where one workgroup had needed none.  us
 // a call of 2, 10 and 200 sweeps: 100^2 Ising replayed 49, 50, 492, launched 32, 43,
@@ -1136,7 +1143,7 @@ int piece_graph(spk_hip_lattice *h, int n, Route rt, hipGraphExec_t *out) {
   hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->acc, words);
   int64_t nl = 0;
   rc = check_hip(hipGetLastError(), "zero launch");
-  if (!rc) rc = launch_sweeps(h, n, h->acc, &nl);
+  if (!rc) rc = rt == kRouteTile ? launch_tiles(h, n, h->acc, &nl) : launch_sweeps(h, n, h->acc, &nl);
   const hipError_t e = hipStreamEndCapture(h->stream, &graph);
   if (!rc) rc = check_hip(e, "end capture");
   if (rc) {
@@ -1506,19 +1513,7 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
     hipLaunchKernelGGL(k_zero_u64, dim3(grid_for(words, 256)), dim3(256), 0, h->stream, h->acc, words);
     return check_hip(hipGetLastError(), "zero launch");
   };
-  if (rt == kRouteTile) {
-    // boxes: from the host (launch_tiles), in pieces of kInitialAccRows sweeps
-    if ((rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows))) ||
-        (rc = check_hip(hipEventRecord(h->ev0, h->stream), "event")))
-      return rc;
-    for (int done = 0; done < nsweeps;) {
-      const int n = std::min(nsweeps - done, kInitialAccRows);
-      if ((rc = clear(n)) || (rc = launch_tiles(h, n, h->acc, &nlaunch)) ||
-          (rc = launch_fold(h, h->acc, n, h->pinned + (size_t)done * 2)))
-        return rc;
-      done += n;
-    }
-  } else if (replayed(h, nsweeps)) {
+  if (replayed(h, nsweeps, rt)) {
     // graph replays (graph_pieces); each piece's rows are folded into the
     // pinned rows [done, done + n) before the next piece clears them
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
@@ -1534,7 +1529,19 @@ int spk_hip_sweeps(spk_hip_lattice *h, int nsweeps, int64_t *naccept_total, int6
         return rc;
       done += pieces[k];
     }
-    for (int n : pieces) nlaunch += sweep_launches(h, n);
+    for (int n : pieces) nlaunch += sweep_launches(h, n, rt);
+  } else if (rt == kRouteTile) {
+    // boxes: from the host (launch_tiles), in pieces of kInitialAccRows sweeps
+    if ((rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows))) ||
+        (rc = check_hip(hipEventRecord(h->ev0, h->stream), "event")))
+      return rc;
+    for (int done = 0; done < nsweeps;) {
+      const int n = std::min(nsweeps - done, kInitialAccRows);
+      if ((rc = clear(n)) || (rc = launch_tiles(h, n, h->acc, &nlaunch)) ||
+          (rc = launch_fold(h, h->acc, n, h->pinned + (size_t)done * 2)))
+        return rc;
+      done += n;
+    }
   } else {
     // every launch from the host: rows [0, nsweeps)
     if ((rc = ensure_acc(h, nsweeps)) || (rc = check_hip(hipEventRecord(h->ev0, h->stream), "event")) ||
@@ -1575,16 +1582,14 @@ int spk_hip_prepare(spk_hip_lattice *h, int nsweeps) {
   int rc;
   Route rt;
   if ((rc = enter_route(h, nsweeps, &rt)) || (rc = ensure_pinned(h, nsweeps))) return rc;
-  if (rt == kRouteTile) {
-    if ((rc = ensure_acc(h, std::min(nsweeps, kInitialAccRows)))) return rc;
-  } else if (replayed(h, nsweeps)) {
+  if (replayed(h, nsweeps, rt)) {
     const std::vector<int> pieces = graph_pieces(h->chunk, nsweeps);
     if ((rc = ensure_acc(h, pieces[0]))) return rc;
     for (int n : pieces) {
       hipGraphExec_t exec;
       if ((rc = piece_graph(h, n, rt, &exec))) return rc;
     }
-  } else if ((rc = ensure_acc(h, nsweeps))) {
+  } else if ((rc = ensure_acc(h, rt == kRouteTile ? std::min(nsweeps, kInitialAccRows) : nsweeps))) {
     return rc;
   }
   return check_hip(hipStreamSynchronize(h->stream), "prepare sync");

@@ -340,3 +340,31 @@ def test_calls_of_two_launches_capture_no_graph(host):
         assert host.captures() == captures
         L.sweeps(2)
         assert host.captures() == captures + 1
+
+
+def test_long_calls_of_first_appearance_boxes_are_replayed(host):
+    with lattice("potts/neighonly", "sc/26n", (92, 32, 44), 656669) as L:
+        captures = host.captures()
+        L.sweeps(3)
+        L.set_temperature(0.4)
+        L.sweeps(3)
+        assert host.captures() == captures and "k_sweep_tile" in host.sweeps()
+        L.prepare(24)
+        assert host.captures() == captures + 1
+        host.log()
+        L.sweeps(24)
+        assert host.captures() == captures + 1
+        assert host.sweeps() == ["k_sweep_tile"] * L.last_timing()[1]
+
+
+def test_few_replicas_on_planes_take_no_more_workgroups_than_they_need(host):
+    """An ensemble of constant shape; the grid grows in steps only once it has
+    changed."""
+    from spparks_amd import batch
+    with batch.Batch(64 << 20, 4) as B:
+        B.set_launch(256, 1024)
+        B.add(batch.replica_desc("potts", "sc/26n", 64, 64, 64, nspins=100, temperature=0.5, nsweeps=60))
+        host.log()
+        B.run(10)
+        grids = {g for n, g, _ in host.log() if n.startswith("k_batch_slice")}
+        assert len(grids) == 1 and 16 <= grids.pop() <= 24      # 1024 rows, 16 a wavefront, 4 wavefronts
