@@ -379,7 +379,9 @@ def run(args):
     resident = (not args.no_resident and app not in VARIANTS and n * (sb + 4) <= 160 * 1024
                 and nlaunch == 1)
     two_state = lattice == "sq/4n" and (app in ("ising", "ising/single") or q == 2)
-    paired = two_state and 2050 <= shape[0] <= 4096 and shape[1] >= 64   # two sweeps a launch on planes
+    # two sweeps a launch on planes (boxes of two-state lattices run six or more)
+    paired = (two_state and shape[0] <= 4096 and shape[1] >= 64
+              and nlaunch == 2 * (steps // 4) + 2 * (steps % 4))
     # lattices whose colour passes are short: boxes of the lattice in LDS,
     # several passes a launch (the library's rule)
     boxes = not resident and not paired and nlaunch < K * steps
@@ -425,7 +427,7 @@ def run(args):
         # per-colour launches (8 + 3/8 bytes per update each)
         pairs = (K * steps - nlaunch) // 3
         colour = nlaunch - pairs
-        kernel = "k_sweep_bits_pair (two sweeps per launch, bands of 16 rows)"
+        kernel = "k_sweep_bits_pair (two sweeps per launch, bands of rows)"
         bytes_per_launch = int((8 + 2 / 8) * n)
         B_kernel = bytes_per_launch / (2 * n)
         # a per-colour launch counted as its share of a pair launch's bytes

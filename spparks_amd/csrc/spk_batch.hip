@@ -153,7 +153,7 @@ __global__ __launch_bounds__(1024) void k_batch_step(char *__restrict__ pool, co
 // the same on a whole wavefront.
 // Batches of 100 sweeps, ms a sweep of the device, packed spins and planes:
 // 32 replicas of edge 34..126 (13.6M sites) beside 32 two-state ones 0.151,
-// 0.098; 24 solves of edge 32..190 (18.2e9 updates in all) 128, 94 ms.  What
+// 0.098; 24 solves of edge 32..190 (18.2e9 updates in all) 128, 89 ms.  What
 // bounds it is k_sweep_slice's (VALU and a wavefront's own chain), on words a
 // quarter empty on the average, and the last wavefronts of a step.  Replicas
 // with most planes first in the list: 0.099 and 97, taken back.

@@ -174,10 +174,10 @@ __global__ __launch_bounds__(kSliceThreads) void k_sweep_slice(uint32_t *__restr
 // compare, decide, barrier: 0.8-1 us for 32 passes of 128^2 sq/8n, VALU busy
 // 38%); large ones, the VALU (54% busy on 1500 x 1002 sq/8n, with 14% of the
 // events in the halo).  us a sweep, before and now:
-//   sq/4n Ising 256^2 10.2, 2.9 (1000^2 10.8, 4.8, but 4.1 in k_sweep_bits_pair)
-//   sq/8n Potts 128^2 Q=100 9.2, 4.4 (one workgroup before)
-//   sq/8n Potts 1500 x 1002 Q=100 15.1, 9.5
-//   sc/26n Potts 32^3 Q=1000 33.6, 12.8; 64^3 Q=10^5 37.6, 15.5
+//   sq/4n Ising 256^2 10.2, 2.3 (1000^2 10.8, 4.8, but 4.1 in k_sweep_bits_pair)
+//   sq/8n Potts 128^2 Q=100 9.2, 3.8 (one workgroup before)
+//   sq/8n Potts 1500 x 1002 Q=100 15.1, 8.8
+//   sc/26n Potts 32^3 Q=1000 33.6, 12.1; 64^3 Q=10^5 37.6, 15.1
 // One site a thread (VEC 1) against packs of 4: 16.2 against 24.1 on 64^3
 // sc/26n, 4.4 against 5.6 on 128^2 sq/8n, but 11.2 against 9.5 on 1500 x 1002,
 // where the VALU counts.
