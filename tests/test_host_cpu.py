@@ -368,3 +368,16 @@ def test_few_replicas_on_planes_take_no_more_workgroups_than_they_need(host):
         B.run(10)
         grids = {g for n, g, _ in host.log() if n.startswith("k_batch_slice")}
         assert len(grids) == 1 and 16 <= grids.pop() <= 24      # 1024 rows, 16 a wavefront, 4 wavefronts
+
+
+def test_kind_of_few_sweeps_takes_few_steps(host):
+    """Beside a replica of another kind with many."""
+    from spparks_amd import batch
+    with batch.Batch(64 << 20, 4) as B:
+        B.set_launch(256, 1024)
+        B.add(batch.replica_desc("potts", "sc/26n", 64, 64, 64, nspins=100, temperature=0.5, nsweeps=10))
+        B.add(batch.replica_desc("ising", "sq/4n", 64, 64, nsweeps=100, temperature=2.0))
+        host.log()
+        B.run(100)
+        names = host.sweeps()
+        assert names.count("k_batch_step") == 2 * 100 and names.count("k_batch_slice") <= 4 * 20
