@@ -51,7 +51,9 @@ class Runtime:
 
 @pytest.fixture
 def host(monkeypatch):
-    from spparks_amd import batch, hip
+    from spparks_amd import batch, build, hip
+    if not os.path.exists(LIB):
+        build.build_host_library()
     L = hip.load_library(LIB)
     monkeypatch.setattr(hip, "_lib", L)
     monkeypatch.setattr(batch, "_bound", False)
