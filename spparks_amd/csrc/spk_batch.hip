@@ -620,8 +620,8 @@ constexpr size_t kMaxGraphs = 64;
 // sizes in an octave, so that a queue whose tiles change with every solve does not
 // have every block recorded.  The surplus workgroups leave at once.  300 mixed solves,
 // 16 live, 5 sweeps a block: 134 blocks took 121 ms with most of them recorded (49 ms
-// of steps), 100 with 24 graphs (and the surplus workgroups
-// of an ensemble of few sliced replicas, recorded so at once, cost it 2%).
+// of steps), 100 with 24 graphs.  (Not at once: an ensemble of few sliced replicas
+// would pay 2% for surplus workgroups.)
 int recorded_grid(int need) {
   if (need == 0) return 0;
   int unit = kSliceResident / 4;

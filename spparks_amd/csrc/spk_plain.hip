@@ -1019,9 +1019,10 @@ int launch_tile(spk_hip_lattice *h, int from, int q0, int q1, unsigned long long
 
 // n sweeps through the tile kernel, split evenly over its launches: whole
 // sweeps each, or (one sweep, or one sweep a launch and an odd number of
-// them) at colours inside a sweep.  Launched one by one rather than captured (replayed): the
-// device takes longer over a launch than the host, and a graph for each number of
-// sweeps and each temperature cost 70 us where one workgroup had needed none.  us
+// them) at colours inside a sweep.  Launched one by one rather than captured
+// (replayed): the device takes longer over a launch than the host, and a graph for
+// each number of sweeps and each temperature cost 70 us where one workgroup had
+// needed none.  us
 // a call of 2, 10 and 200 sweeps: 100^2 Ising replayed 49, 50, 492, launched 32, 43,
 // 425; 128^2 sq/8n 45, 66, 857 and 35, 59, 786; 64^3 sc/26n 59, 176, 3018 and
 // 51, 175, 2980.  After a change of temperature 2 sweeps took 126, 125 and 134.
